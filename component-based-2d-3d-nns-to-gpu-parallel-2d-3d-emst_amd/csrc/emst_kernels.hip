@@ -2261,9 +2261,10 @@ __global__ __launch_bounds__(kBlock) void k_comp_keep(int64_t n, const uint32_t*
 __global__ __launch_bounds__(kBlock) void k_comp_prep(int64_t n, const float4* __restrict__ pts,
                                                      const int32_t* __restrict__ label,
                                                      int32_t* __restrict__ corr,
-                                                     const uint64_t* __restrict__ corr_key,
+                                                     uint64_t* __restrict__ corr_key,
                                                      const uint64_t* __restrict__ comp1,
-                                                     uint64_t* __restrict__ open_mask, const Counters* C)
+                                                     const Node* __restrict__ nodes, const Cloud* __restrict__ cl,
+                                                     int ncl, uint64_t* __restrict__ open_mask, const Counters* C)
 {
     if (C->done) return;
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2277,6 +2278,15 @@ __global__ __launch_bounds__(kBlock) void k_comp_prep(int64_t n, const float4* _
             need = lbb <= key_bound(comp1[lp]);
             if (need && p > 0 && label[p - 1] == lp && same_xyz(pts[p - 1], pts[p])) need = false;
             if (!need) corr[p] = -1;    // the absorbed target's d2 stays as the bound
+            // a cloud that is one component holds nothing outside it (in a
+            // batch, clouds finish rounds apart: each one's points searched
+            // once more through every pass, 1.45 of 2.19 ms per run of 256
+            // clouds of 10^2-10^4 points went to the searches, now 0.97)
+            if (need && __float_as_int(nodes[2 * cl[find_cloud(cl, ncl, p)].lbase + 1].pad[1]) == lp) {
+                need = false;
+                corr[p] = -2;
+                corr_key[p] = kEmptyKey;
+            }
         }
     }
     const uint64_t m = __ballot(need);
@@ -2488,6 +2498,19 @@ constexpr int kSmallPacket = 8;
 constexpr int kKnnGatherWork = 1024;
 constexpr int kKnnGatherLeaves = 256;
 
+// minimum over the wave, the same in every lane
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v)
+{
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false));     // quad_perm [1,0,3,2]
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false));     // quad_perm [2,3,0,1]
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, false));    // row_half_mirror
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, false));    // row_mirror
+    // one value per row of 16
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    return min(min(a, b), min(c, d));
+}
+
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
 {
     const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, m);
@@ -2584,9 +2607,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
     // one packet per block; a grid smaller than the packets (the resumed
     // dispatch, whose queries are few but unknown to the host) loops
     const int qpp = nq <= kSmallDispatch ? kSmallPacket : 64;
-    for (int64_t pk = blockIdx.x;; pk += gridDim.x) {
-        if (pk * qpp >= nq) {
-            if (open_out != nullptr && threadIdx.x == 0 && pk == (int64_t)blockIdx.x) open_out[pk] = 0ull;
+    // The resumed dispatch (no open_out) gives every block a run of
+    // consecutive packets, so that the packets in flight are spread over all
+    // components: the first ones find their components' edges, which bound the
+    // packets after them (7.2*10^6 points in 512 clouds of eight Gaussians:
+    // 17.9 -> 15.9 ms per run).  The first dispatch keeps one packet per block
+    // in list order: runs there left the chip with a tail (10^7 clustered
+    // points 13.4 -> 14.5 ms), and parts spread out by a stride lost their
+    // neighbours' cache lines (13.8 ms).
+    const int64_t npk = (nq + qpp - 1) / qpp;
+    const int64_t run = open_out == nullptr ? (npk + gridDim.x - 1) / gridDim.x : 1;
+    const int64_t pk0 = (int64_t)blockIdx.x * run, pk1 = open_out == nullptr ? min(npk, pk0 + run) : npk;
+    for (int64_t pk = pk0;; pk += open_out == nullptr ? 1 : (int64_t)gridDim.x) {
+        if (pk >= pk1) {
+            if (open_out != nullptr && threadIdx.x == 0 && pk == pk0) open_out[pk] = 0ull;
             break;
         }
         const int lane = __lane_id();
@@ -2765,7 +2799,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                 bool done_by_gather = false;
                 uint32_t B = open ? (uint32_t)bnd : 0u;
                 for (int off = 32; off > 0; off >>= 1) B = max(B, (uint32_t)__shfl_xor((int)B, off));
-                if (B < 0x7f800000u) {
+                {
                     float qlo[3] = {open ? px : INFINITY, open ? py : INFINITY, open ? pz : INFINITY};
                     float qhi[3] = {open ? px : -INFINITY, open ? py : -INFINITY, open ? pz : -INFINITY};
                     int32_t imin = open ? inner : 0x7fffffff;
@@ -2779,7 +2813,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                     }
                     const int fo = (int)__builtin_ctzll(__ballot(open));
                     const int32_t lab0 = __builtin_amdgcn_readfirstlane(__shfl(mylab, fo));
-                    const int32_t skip_lab = __ballot(open && mylab != lab0) == 0ull ? lab0 : (int32_t)0x80000000;
+                    const bool one_lab = __ballot(open && mylab != lab0) == 0ull;
+                    const int32_t skip_lab = one_lab ? lab0 : (int32_t)0x80000000;
                     int head = 0, tail = gather_start(L, work), ngl = 0;
                     bool over = false;
                     __builtin_amdgcn_wave_barrier();
@@ -2789,7 +2824,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                         head += take;
                         st_nodes += (uint32_t)take;
                         bool pass_ = false, leaf = false;
-                        uint32_t bd = 0;
+                        uint32_t bd = 0, ub = 0xffffffffu;
                         if (lane < take) {
                             const Node x = tree[nd];
                             const int32_t xl = __float_as_int(x.pad[1]);
@@ -2804,7 +2839,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                             leaf = nd >= L;
                             pass_ = xl != kNlabEmpty && xl != skip_lab && bd <= B &&
                                     (int32_t)__float_as_uint(far) > imin && !(leaf && nd == pre);
+                            // it holds a point outside every query's component
+                            // (it holds two components, or the queries lie in
+                            // one, which is another): none needs more than
+                            // its far corner, which then bounds the gathering.
+                            // Without it a pass whose radius first reaches a far
+                            // cluster gathered most of that cluster, outgrew its
+                            // lists and walked (512 clouds of eight Gaussians:
+                            // 153000 -> 34000 walks per run)
+                            if (pass_ && (xl == kNlabMixed || one_lab)) ub = __float_as_uint(far);
                         }
+                        B = min(B, wave_min_u32(ub));
+                        pass_ = pass_ && bd <= B;
                         const uint64_t ml = __ballot(pass_ && leaf);
                         const int nlf = __popcll(ml);
                         int add;
@@ -2832,7 +2878,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                         for (int c0 = 0; c0 < ngl; c0 += 64) {
                             const int cn = min(64, ngl - c0);
                             const uint64_t e = wave_sort_u64(lane < cn ? gathered[c0 + lane] : kEmptyKey);
-                            for (int i = 0; i < cn; ++i) try_leaf(__builtin_amdgcn_readlane((int)(uint32_t)e, i));
+                            for (int i = 0; i < cn; ++i) {
+                                // (gathered before B shrank to less than its distance)
+                                if ((uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(e >> 32), i) > B) break;
+                                try_leaf(__builtin_amdgcn_readlane((int)(uint32_t)e, i));
+                            }
                         }
                     }
                 }
@@ -2843,7 +2893,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                 // this pass on (no leaf has been visited in it yet, so their
                 // bests are empty), while the round's list has room
                 bool handed = false;        // this lane's query went to the per-query pass
-                if (!done_by_gather && defer != nullptr && B < 0x7f800000u) {
+                if (!done_by_gather && defer != nullptr) {
                     const uint64_t entry = ((uint64_t)(uint32_t)pass << 32) | (uint32_t)p;
                     if (D == 3) {
                         handed = wave_append_capped_u64(open, entry, defer, &C->deferred, kDeferCap);
@@ -3122,8 +3172,8 @@ __global__ __launch_bounds__(64 * kDeferWaves) void k_comp_search_deferred(
                 }
             };
             bool done_by_gather = false;
-            if ((uint32_t)bnd < 0x7f800000u) {
-                const uint32_t B = (uint32_t)bnd;
+            {
+                uint32_t B = (uint32_t)bnd;
                 int head = 0, tail = gather_start(L, work), ngl = 0;
                 bool over = false;
                 while (head < tail) {
@@ -3132,7 +3182,7 @@ __global__ __launch_bounds__(64 * kDeferWaves) void k_comp_search_deferred(
                     head += take;
                     st_nodes += (uint32_t)take;
                     bool pass_ = false, leaf = false;
-                    uint32_t bd = 0;
+                    uint32_t bd = 0, ub = 0xffffffffu;
                     if (lane < take) {
                         const Node x = tree[nd];
                         const int32_t xl = __float_as_int(x.pad[1]);
@@ -3140,7 +3190,10 @@ __global__ __launch_bounds__(64 * kDeferWaves) void k_comp_search_deferred(
                         bd = __float_as_uint(box_d2(x, far));
                         leaf = nd >= L;
                         pass_ = xl != kNlabEmpty && xl != mylab && bd <= B && (int32_t)__float_as_uint(far) > inner;
+                        if (pass_) ub = __float_as_uint(far);       // it holds a point outside
                     }
+                    B = min(B, wave_min_u32(ub));
+                    pass_ = pass_ && bd <= B;
                     const uint64_t ml = __ballot(pass_ && leaf);
                     const int nlf = __popcll(ml);
                     int add;
@@ -4095,8 +4148,8 @@ void launch_comp_round(int dim, int64_t n, const float4* pts, const uint32_t* id
     hipLaunchKernelGGL(dim == 3 ? k_comp_keep<kKnn3> : k_comp_keep<kKnn2>, dim3(g), dim3(kBlock), 0, s, n, ids,
                        label, corr, corr_key, comp1, nb,
                        (const Counters*)C);
-    hipLaunchKernelGGL(k_comp_prep, dim3(g), dim3(kBlock), 0, s, n, pts, label, corr, (const uint64_t*)corr_key,
-                       (const uint64_t*)comp1, sc.open_mask, (const Counters*)C);
+    hipLaunchKernelGGL(k_comp_prep, dim3(g), dim3(kBlock), 0, s, n, pts, label, corr, corr_key,
+                       (const uint64_t*)comp1, (const Node*)nodes, cl, ncl, sc.open_mask, (const Counters*)C);
     open_compact(sc.open_mask, P, sc.off, sc.tmp, nullptr, sc.list, s);
     const uint32_t* nq = sc.off + P;
     const float* seed_r = nullptr;
