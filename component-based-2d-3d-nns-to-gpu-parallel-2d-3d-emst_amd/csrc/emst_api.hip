@@ -1,7 +1,7 @@
 // emst_api.hip -- host side of the C ABI (include/emst.h).
 //
 // A context holds one point set on one device and one HIP stream.  The build
-// (bbox, rescale, Morton sort, hierarchy, round-1 cone search) runs inside
+// (bbox, rescale, sort along a curve, hierarchy, round-1 cone search) runs inside
 // the first emst_run/emst_step, so that a timed run starts from resident
 // input points, like the reference's cuda_duree span plus its cell build.
 #include <algorithm>
@@ -84,7 +84,7 @@ struct emst_ctx {
     int ncl = 0;
     std::vector<Cloud> hcl;
     int64_t nleaves = 0, Lmax = 0;
-    int mbits = 16;                   // Morton bits per axis
+    int mbits = 16;                   // sort key bits per axis
     int64_t target_edges = 0;         // sum over clouds of (points - 1)
     const float* xyz = nullptr;       // input points on the device (AoS)
     bool have_points = false;
@@ -332,7 +332,7 @@ int layout_clouds(emst_ctx* c, int bucket)
         target += std::max<int64_t>(cl.n - 1, 0);
     }
     c->target_edges = target;
-    // Morton bits per axis: the cloud index takes the top key bits of a batch.
+    // Key bits per axis: the cloud index takes the top key bits of a batch.
     // Keys of 48 bits (16 per axis in 3D, 24 in 2D, fewer in a batch) sort in
     // 6 radix passes instead of 8; the leaves stay the same cells wherever a
     // cell holds at most a leaf's points, down to 2^-16 of the box (a longer
@@ -353,6 +353,22 @@ int layout_clouds(emst_ctx* c, int bucket)
 }
 
 LeafTable leaf_table(const emst_ctx* c) { return LeafTable{c->lstart.p, c->leaf_of.p}; }
+
+// Points are sorted along a Hilbert curve, or along a Morton curve where the
+// order shows in results: the component search's sample log describes every
+// point's own leaf cell, and those are Morton cells (emst_get_radius_samples).
+bool hilbert_order(const emst_ctx* c) { return !(c->opt.round_search == 1 && c->opt.log_samples == 1); }
+
+int sort_key_bits(const emst_ctx* c)
+{
+    int bits = c->mbits * c->dim;
+    if (c->ncl > 1) {
+        int cb = 0;
+        while ((1ll << cb) < c->ncl) ++cb;
+        bits += cb;
+    }
+    return bits;
+}
 
 // The leaves of the sorted points (LeafTable), then each cloud's hierarchy:
 // its leaf count sets its slot count L (a power of two) and its node offset.
@@ -494,7 +510,7 @@ DupState dup_state(emst_ctx* c)
     return d;
 }
 
-// bbox, rescale, Morton sort, hierarchy, round-1 cone search
+// bbox, rescale, sort, hierarchy, round-1 cone search
 NbrList nbr_list(emst_ctx* c)
 {
     if (!c->knn_built) return NbrList{nullptr, nullptr, nullptr};
@@ -519,14 +535,8 @@ int build(emst_ctx* c)
                             c->ncl == 1 ? std::string("input holds a NaN or Inf coordinate")
                                         : "cloud " + std::to_string(k) + " holds a NaN or Inf coordinate");
     }
-    launch_rescale_morton(c->xyz, c->dcl.p, c->ncl, n, c->dim, c->mbits, c->P, c->resc.p, c->keys0.p, s);
-    int key_bits = c->mbits * c->dim;
-    if (c->ncl > 1) {
-        int cb = 0;
-        while ((1ll << cb) < c->ncl) ++cb;
-        key_bits += cb;
-    }
-    radix_sort(c->keys0.p, c->vals0.p, c->keys1.p, c->vals1.p, n, key_bits, true, c->hist.p, c->scan_tmp.p, s);
+    launch_rescale_keys(c->xyz, c->dcl.p, c->ncl, n, c->dim, c->mbits, c->P, c->resc.p, c->keys0.p, hilbert_order(c), s);
+    radix_sort(c->keys0.p, c->vals0.p, c->keys1.p, c->vals1.p, n, sort_key_bits(c), true, c->hist.p, c->scan_tmp.p, s);
     launch_gather_sorted(c->resc.p, c->vals0.p, n, c->dim, c->pts.p, c->inv.p, c->ids.p, s);
     int rcl = make_leaves(c);
     if (rcl) return rcl;
@@ -961,14 +971,8 @@ void issue_one_launch_build(emst_ctx* c)
     hipStream_t s = c->stream;
     launch_bbox(c->xyz, c->dcl.p, c->ncl, n, c->dim, c->P, s);
     launch_params(c->P, c->dcl.p, c->ncl, c->dim, c->mbits, s);
-    launch_rescale_morton(c->xyz, c->dcl.p, c->ncl, n, c->dim, c->mbits, c->P, c->resc.p, c->keys0.p, s);
-    int key_bits = c->mbits * c->dim;
-    if (c->ncl > 1) {
-        int cb = 0;
-        while ((1ll << cb) < c->ncl) ++cb;
-        key_bits += cb;
-    }
-    radix_sort(c->keys0.p, c->vals0.p, c->keys1.p, c->vals1.p, n, key_bits, true, c->hist.p, c->scan_tmp.p, s);
+    launch_rescale_keys(c->xyz, c->dcl.p, c->ncl, n, c->dim, c->mbits, c->P, c->resc.p, c->keys0.p, hilbert_order(c), s);
+    radix_sort(c->keys0.p, c->vals0.p, c->keys1.p, c->vals1.p, n, sort_key_bits(c), true, c->hist.p, c->scan_tmp.p, s);
     launch_gather_sorted(c->resc.p, c->vals0.p, n, c->dim, c->pts.p, c->inv.p, c->ids.p, s);
     launch_leaves(c->keys0.p, n, c->dcl.p, c->ncl, c->bucket, c->vals1.p, reinterpret_cast<uint32_t*>(c->keys1.p),
                   c->scan_tmp.p, c->lstart.p, c->leaf_of.p, c->cloud_lf.p, c->P, c->C, true, s);
@@ -1077,6 +1081,66 @@ int run_one_launch(emst_ctx* c)
         c->times[2] += elapsed(c->ev[2], c->ev[3]);
     }
     c->times[3] = c->times[0] + c->times[1] + c->times[2];
+    return EMST_OK;
+}
+
+// Training pairs of the cone search: the features of every point on the
+// Morton order and its leaf cells (the curve the samples are defined on; the
+// search itself runs on the Hilbert order), in that order, and the targets
+// from the cone candidates.  One cloud.
+int morton_samples(emst_ctx* c, float* feat, float* target)
+{
+    const int64_t n = c->n;
+    hipStream_t s = c->stream;
+    DevBuf<uint64_t> keys0, keys1;
+    DevBuf<uint32_t> vals0, vals1, ids;
+    DevBuf<float4> pts;
+    DevBuf<int32_t> inv, lstart, leaf_of, cloud_lf, rep, runs, list, gslot;
+    DevBuf<Cloud> dcl;
+    DevBuf<Node> nodes;
+    DevBuf<Counters> cnt;
+    int rc;
+    if ((rc = ensure(c, keys0, n)) || (rc = ensure(c, keys1, n)) || (rc = ensure(c, vals0, n)) ||
+        (rc = ensure(c, vals1, n)) || (rc = ensure(c, ids, n)) || (rc = ensure(c, pts, n)) ||
+        (rc = ensure(c, inv, n)) || (rc = ensure(c, lstart, n + 1)) || (rc = ensure(c, leaf_of, n)) ||
+        (rc = ensure(c, cloud_lf, 2)) || (rc = ensure(c, dcl, 1)) || (rc = ensure(c, cnt, 1)) ||
+        (rc = ensure(c, c->feat, (size_t)n * 8)) || (rc = ensure(c, c->pred, (size_t)n)) ||
+        (rc = ensure(c, c->ls, (size_t)n)))
+        return rc;
+    Cloud cl = c->hcl[0];
+    HIPCHK(c, hipMemcpyAsync(dcl.p, &cl, sizeof(Cloud), hipMemcpyHostToDevice, s));
+    launch_zero_u32(reinterpret_cast<uint32_t*>(cnt.p), sizeof(Counters) / sizeof(uint32_t), s);
+    launch_rescale_keys(c->xyz, dcl.p, 1, n, c->dim, c->mbits, c->P, c->resc.p, keys0.p, false, s);
+    radix_sort(keys0.p, vals0.p, keys1.p, vals1.p, n, sort_key_bits(c), true, c->hist.p, c->scan_tmp.p, s);
+    launch_gather_sorted(c->resc.p, vals0.p, n, c->dim, pts.p, inv.p, ids.p, s);
+    launch_leaves(keys0.p, n, dcl.p, 1, c->bucket, vals1.p, reinterpret_cast<uint32_t*>(keys1.p), c->scan_tmp.p,
+                  lstart.p, leaf_of.p, cloud_lf.p, c->P, cnt.p, false, s);
+    LAUNCHCHK(c);
+    int32_t lf[2] = {0, 0};
+    HIPCHK(c, hipMemcpyAsync(lf, cloud_lf.p, sizeof(lf), hipMemcpyDeviceToHost, s));
+    HIPCHK(c, hipStreamSynchronize(s));
+    cl.lfirst = lf[0];
+    cl.nl = lf[1] - lf[0];
+    cl.lbase = 0;
+    cl.L = 1;
+    while (cl.L < cl.nl) cl.L <<= 1;
+    if ((rc = ensure(c, nodes, 2 * (size_t)cl.L))) return rc;
+    HIPCHK(c, hipMemcpyAsync(dcl.p, &cl, sizeof(Cloud), hipMemcpyHostToDevice, s));
+    if (c->grouped) {
+        // the leaf boxes leave out group members, as in the search's build
+        if ((rc = ensure(c, rep, n)) || (rc = ensure(c, runs, n)) || (rc = ensure(c, list, n)) ||
+            (rc = ensure(c, gslot, n)))
+            return rc;
+        launch_dup_groups(keys0.p, pts.p, n, rep.p, runs.p, list.p, gslot.p, cnt.p, s);
+    }
+    const LeafTable lt{lstart.p, leaf_of.p};
+    launch_build_tree(pts.p, dcl.p, 1, cl.L, cl.L, lt, nodes.p, rep.p, s);
+    launch_radius_features(c->dim, pts.p, nodes.p, cl.L, lt, n, c->feat.p, c->ls.p, s);
+    launch_radius_targets(c->K, n, c->cand_key.p, ids.p, c->inv.p, c->ls.p, c->pred.p, s);
+    LAUNCHCHK(c);
+    if (feat) HIPCHK(c, hipMemcpyAsync(feat, c->feat.p, sizeof(float) * n * 8, hipMemcpyDeviceToHost, s));
+    if (target) HIPCHK(c, hipMemcpyAsync(target, c->pred.p, sizeof(float) * n, hipMemcpyDeviceToHost, s));
+    HIPCHK(c, hipStreamSynchronize(s));
     return EMST_OK;
 }
 
@@ -1705,17 +1769,7 @@ int emst_get_radius_samples(emst_ctx* c, float* feat, float* target, int64_t* m)
     if (*m < n) { *m = n; return fail(c, EMST_E_ARG, "sample arrays too small"); }
     *m = n;
     if (n == 0) return EMST_OK;
-    if ((rc = ensure(c, c->feat, (size_t)n * 8)) || (rc = ensure(c, c->pred, (size_t)n)) ||
-        (rc = ensure(c, c->ls, (size_t)n)))
-        return rc;
-    hipStream_t s = c->stream;
-    launch_radius_features(c->dim, c->pts.p, c->nodes.p, c->L, leaf_table(c), n, c->feat.p, c->ls.p, s);
-    launch_radius_targets(c->K, n, c->cand_key.p, c->ls.p, c->pred.p, s);
-    LAUNCHCHK(c);
-    if (feat) HIPCHK(c, hipMemcpyAsync(feat, c->feat.p, sizeof(float) * n * 8, hipMemcpyDeviceToHost, s));
-    if (target) HIPCHK(c, hipMemcpyAsync(target, c->pred.p, sizeof(float) * n, hipMemcpyDeviceToHost, s));
-    HIPCHK(c, hipStreamSynchronize(s));
-    return EMST_OK;
+    return morton_samples(c, feat, target);
 }
 
 int emst_get_search_stats(emst_ctx* c, int64_t* stats, int32_t* n_stats)

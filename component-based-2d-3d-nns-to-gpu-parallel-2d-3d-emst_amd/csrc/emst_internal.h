@@ -16,7 +16,7 @@ struct Params {
     double unit_x;          // rescale factor (A2), double as computed
     float unit_xf;          // (float)unit_x, the factor applied per coordinate
     float newmax[3];        // rescaled extremes (newmin is 0 by monotonicity)
-    float qscale;           // Morton quantisation scale
+    float qscale;           // key quantisation scale
     uint32_t nonfinite;     // set when a coordinate is NaN or Inf
     uint32_t pad[3];
 };
@@ -37,7 +37,7 @@ struct Counters {
     // tested, leaves entered, leaf points read per packet, lane-point pairs
     unsigned long long packets, nodes, leaves, leaf_points, pairs;
     // coincident-point groups (set once per build, not reset by the rounds)
-    uint32_t dup_runs;      // runs of >= 2 equal Morton keys
+    uint32_t dup_runs;      // runs of >= 2 equal keys
     uint32_t dup_points;    // points with an identical twin (group members + representatives)
     uint32_t dup_overflow;  // a run too long to split into groups: grouping off
     uint32_t grouped;       // grouping on (dup_points > 0 and no overflow)
@@ -143,7 +143,7 @@ struct Cloud {
 };
 
 // Leaves of the search hierarchy: the maximal cells of the binary prefix tree
-// of the sorted keys (Morton prefixes) that hold at most `bucket` points; a
+// of the sorted keys (curve prefixes) that hold at most `bucket` points; a
 // run of more than `bucket` equal keys, which no key bit splits, is cut every
 // `bucket` points from its start.  Numbered in sorted order, cloud by cloud:
 // leaf g holds the sorted positions [start[g], start[g + 1]); of[p] = the
@@ -154,7 +154,7 @@ struct LeafTable {
     const int32_t* of;      // n
 };
 
-// Search-hierarchy node: tight box of a contiguous range of Morton-sorted points.
+// Search-hierarchy node: tight box of a contiguous range of sorted points.
 struct alignas(32) Node {
     float lo[3];
     float hi[3];
@@ -167,12 +167,13 @@ struct alignas(32) Node {
 
 // ---- launch wrappers (emst_kernels.hip); all asynchronous on `s` ----
 // Per cloud: bounding box (A1), rescale parameters (A2); per point: rescaled
-// coordinates and the sort key (cloud index above mbits-per-axis Morton bits;
-// no cloud bits for a single cloud).  N = total points, P[ncl].
+// coordinates and the sort key (cloud index above mbits-per-axis bits of the
+// point's cell along a Hilbert or a Morton curve; no cloud bits for a single
+// cloud).  N = total points, P[ncl].
 void launch_bbox(const float* xyz, const Cloud* cl, int ncl, int64_t N, int dim, Params* P, hipStream_t s);
 void launch_params(Params* P, const Cloud* cl, int ncl, int dim, int mbits, hipStream_t s);
-void launch_rescale_morton(const float* xyz, const Cloud* cl, int ncl, int64_t N, int dim, int mbits,
-                           const Params* P, float* resc, uint64_t* keys, hipStream_t s);
+void launch_rescale_keys(const float* xyz, const Cloud* cl, int ncl, int64_t N, int dim, int mbits,
+                           const Params* P, float* resc, uint64_t* keys, bool hilbert, hipStream_t s);
 // LSD radix sort of (keys, vals) by bits [0, bits); result lands in (k0, v0).
 // vals_identity: values start as 0..n-1 (v0 is not read).
 void radix_sort(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, int64_t n, int bits,
@@ -352,7 +353,8 @@ void launch_cell_grid(const float* resc, int64_t n, int dim, int pstride, const 
 // X: n x 8 model features, LS: n x log(leaf spacing s0)
 void launch_radius_features(int dim, const float4* pts, const Node* nodes, int64_t L, LeafTable lt, int64_t n,
                             float* X, float* LS, hipStream_t s);
-void launch_radius_targets(int K, int64_t n, const uint64_t* cand_key, const float* LS, float* T, hipStream_t s);
+void launch_radius_targets(int K, int64_t n, const uint64_t* cand_key, const uint32_t* ids, const int32_t* inv,
+                           const float* LS, float* T, hipStream_t s);
 void launch_radius_seed(int64_t n, const float* model, const float* X, const float* LS, float* Y, float* R,
                         hipStream_t s);
 void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* tmp,

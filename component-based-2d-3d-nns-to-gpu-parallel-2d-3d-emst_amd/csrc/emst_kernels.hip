@@ -2,8 +2,8 @@
 //
 // Stages (reference rows they implement, paths relative to the reference root):
 //   bbox / params / rescale ..... InputRW.h:541-559, SolutionEMST.cu:305-379
-//   Morton keys + radix sort .... the cell-grid build (count, wave-level scan,
-//                                 scatter); cells are Morton prefixes
+//   curve keys + radix sort ..... the cell-grid build (count, wave-level scan,
+//                                 scatter); cells are key prefixes
 //   gather / tree ............... leaf cells of <= bucket points with tight boxes
 //   cone search ................. NodeComputeOctantMD::computeOctants
 //                                 (NodeEMST.h:1018-1296): per point, the nearest
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(kBlock) void k_bbox(const float* __restrict__ xyz, 
 // wg = (double)(pMax.x - pMin.x) etc. are float subtractions widened to double,
 // _wnd / unitX in double (SolutionEMST.cu:305-342).  The rescaled extremes are
 // the rescaled box corners: the map p -> (p - pMin) * unitXf is monotone.
-// One thread per cloud; Morton quantisation uses mbits bits per axis.
+// One thread per cloud; key quantisation uses mbits bits per axis.
 __global__ void k_params(Params* Pa, const Cloud* __restrict__ cl, int ncl, int dim, int mbits)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -238,7 +238,7 @@ __global__ void k_params(Params* Pa, const Cloud* __restrict__ cl, int ncl, int 
     P->qscale = mx > 0 ? (float)(maxq / (double)mx) : 0.f;
 }
 
-// ------------------------------------------ rescale + Morton keys (A2, A5)
+// ------------------------------------------- rescale + curve keys (A2, A5)
 __device__ __forceinline__ uint64_t spread3(uint64_t x)
 {
     x &= 0x1fffff;
@@ -260,13 +260,53 @@ __device__ __forceinline__ uint64_t spread2(uint64_t x)
     return x;
 }
 
+// Hilbert index of D coordinates of `bits` bits (Skilling, "Programming the
+// Hilbert curve", 2004: undo the rotations from the top bit down, Gray-code,
+// interleave).  Like a Morton key its prefixes are boxes, halved one bit at a
+// time, but consecutive cells share a face: the points of a run of sorted
+// positions (a packet of 64 queries, its groups of 8, a leaf) lie in one
+// compact piece of space, where a Morton run jumps at every cell boundary.
+// Measured against Morton keys of the same bits: cone search 5.9 -> 4.5 ms at
+// 10^6 uniform 3D points, 6.1 -> 4.4 at 3*10^6 in the 2.5D mode, 23.3 -> 18.5
+// at 4*10^6 clustered ones; neighbour lists of 10^7 clustered points 5.2 ->
+// 4.2 ms.  The key itself takes 0.05 ms more at 10^7 points.
 template <int D>
-__global__ __launch_bounds__(kBlock) void k_rescale_morton(const float* __restrict__ xyz,
+__device__ __forceinline__ uint64_t hilbert_key(uint32_t x[D], int bits)
+{
+    for (int q = bits - 1; q > 0; --q) {
+        const uint32_t low = (1u << q) - 1u;
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            // bit q set: invert x[0]'s low bits; clear: exchange them with x[i]'s
+            const uint32_t inv = (uint32_t)((int32_t)(x[i] << (31 - q)) >> 31) & low;
+            const uint32_t t = (x[0] ^ x[i]) & (low ^ inv);
+            x[0] ^= t | inv;
+            if (i > 0) x[i] ^= t;
+        }
+    }
+#pragma unroll
+    for (int i = 1; i < D; ++i) x[i] ^= x[i - 1];
+    uint32_t t = x[D - 1];          // then bit j of t: the parity of x[D - 1]'s bits above j
+    t ^= t >> 1;
+    t ^= t >> 2;
+    t ^= t >> 4;
+    t ^= t >> 8;
+    t ^= t >> 16;
+    t >>= 1;
+    uint64_t code = 0;
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+        code |= (D == 3 ? spread3(x[i] ^ t) : spread2(x[i] ^ t)) << (D - 1 - i);
+    return code;
+}
+
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_rescale_keys(const float* __restrict__ xyz,
                                                            const Cloud* __restrict__ cl, int ncl,
                                                            int64_t N, int mbits,
                                                            const Params* __restrict__ Pa,
                                                            float* __restrict__ resc,
-                                                           uint64_t* __restrict__ keys)
+                                                           uint64_t* __restrict__ keys, int hilbert)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
@@ -276,15 +316,19 @@ __global__ __launch_bounds__(kBlock) void k_rescale_morton(const float* __restri
     const float fu = P->unit_xf;
     const float qs = P->qscale;
     const uint32_t maxq = (uint32_t)((1ull << mbits) - 1);
-    uint64_t code = 0;
+    uint32_t cell[D];
     for (int k = 0; k < D; ++k) {
         float d = q[k] - P->pmin[k];                // PointE::operator- (Node.h:574-580)
         float v = d * fu;                           // PointE::operator*(float) (Node.h:588-593)
         resc[i * D + k] = v;
         float qf = v * qs;
-        uint32_t qq = qf >= (float)maxq ? maxq : (uint32_t)qf;
-        code |= (D == 3 ? spread3(qq) : spread2(qq)) << k;
+        cell[k] = qf >= (float)maxq ? maxq : (uint32_t)qf;
     }
+    uint64_t code = 0;
+    if (hilbert)
+        code = hilbert_key<D>(cell, mbits);
+    else
+        for (int k = 0; k < D; ++k) code |= (D == 3 ? spread3(cell[k]) : spread2(cell[k])) << k;
     if (ncl > 1) code |= (uint64_t)c << (mbits * D);
     keys[i] = code;
 }
@@ -516,7 +560,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_sorted(const float* __restric
 }
 
 // ------------------------------------------------ coincident-point groups
-// Identical points share a Morton key, so each group lies inside one run of
+// Identical points share a key, so each group lies inside one run of
 // equal keys; the sort is stable over input order, so within a run positions
 // ascend with input id and a group's first position holds its smallest id.
 constexpr int kMixedRunMax = 1024;   // longest run holding >= 2 locations that is split
@@ -716,7 +760,7 @@ __global__ __launch_bounds__(kBlock) void k_dup_runs(const uint64_t* __restrict_
 
 // One wave per run (grid-stride over the queued runs).  A run at one location
 // is one group; a run over several locations (distinct points closer than a
-// Morton cell) of at most kMixedRunMax points is split by pairwise
+// key cell) of at most kMixedRunMax points is split by pairwise
 // comparison; a longer one sets dup_overflow, which turns grouping off.
 // A run of more than kBigRun points (a heavily repeated location: one wave
 // would walk it alone while the grid idles) gets its group slot and list
@@ -884,7 +928,7 @@ __global__ __launch_bounds__(kBlock) void k_level(Node* __restrict__ nodes, cons
 }
 
 // --------------------------------------------------------- cone search
-// One wave = 64 query points (consecutive in Morton order, or a query list).
+// One wave = 64 query points (consecutive in sorted order, or a query list).
 // The wave walks the binary hierarchy together (packet traversal): a node is
 // entered when any lane may still improve a cone from it; leaf points are
 // read with wave-uniform (scalar) loads and every lane tests them against its
@@ -3974,16 +4018,16 @@ void launch_params(Params* P, const Cloud* cl, int ncl, int dim, int mbits, hipS
     hipLaunchKernelGGL(k_params, dim3(nblocks(ncl)), dim3(kBlock), 0, s, P, cl, ncl, dim, mbits);
 }
 
-void launch_rescale_morton(const float* xyz, const Cloud* cl, int ncl, int64_t N, int dim, int mbits,
-                           const Params* P, float* resc, uint64_t* keys, hipStream_t s)
+void launch_rescale_keys(const float* xyz, const Cloud* cl, int ncl, int64_t N, int dim, int mbits,
+                           const Params* P, float* resc, uint64_t* keys, bool hilbert, hipStream_t s)
 {
     if (N <= 0) return;
     if (dim == 3)
-        hipLaunchKernelGGL(k_rescale_morton<3>, dim3(nblocks(N)), dim3(kBlock), 0, s, xyz, cl, ncl, N, mbits, P,
-                           resc, keys);
+        hipLaunchKernelGGL(k_rescale_keys<3>, dim3(nblocks(N)), dim3(kBlock), 0, s, xyz, cl, ncl, N, mbits, P,
+                           resc, keys, hilbert ? 1 : 0);
     else
-        hipLaunchKernelGGL(k_rescale_morton<2>, dim3(nblocks(N)), dim3(kBlock), 0, s, xyz, cl, ncl, N, mbits, P,
-                           resc, keys);
+        hipLaunchKernelGGL(k_rescale_keys<2>, dim3(nblocks(N)), dim3(kBlock), 0, s, xyz, cl, ncl, N, mbits, P,
+                           resc, keys, hilbert ? 1 : 0);
 }
 
 size_t scan_tmp_words(int64_t n) { return (size_t)((n + kScanTile - 1) / kScanTile) + 1; }

@@ -351,7 +351,8 @@ __global__ void k_adam(float* __restrict__ P, float* __restrict__ G, float* __re
 // Features of every sorted point for the seed model, all free of the cloud's
 // scale (ratios of lengths, fractions), and LS = log s0, the leaf spacing the
 // target and the seed are measured in.  Neighbours are the 8 nearest sorted
-// positions (Morton order).
+// positions, on the order of pts (Morton for samples; a run's seeds take them
+// on the run's own order).
 __global__ __launch_bounds__(256) void k_radius_features(int dim, const float4* __restrict__ pts,
                                                         const Node* __restrict__ nodes, int64_t L,
                                                         LeafTable lt, int64_t n, float* __restrict__ X,
@@ -435,15 +436,19 @@ __global__ __launch_bounds__(256) void k_radius_features(int dim, const float4* 
 }
 
 // Target: log(R / s0), R = sqrt(largest non-empty cone best d2) of the point,
-// s0 = exp(LS) its leaf spacing.  Points with no candidate get -20.
+// s0 = exp(LS) its leaf spacing.  Points with no candidate get -20.  ids: the
+// input id of each target; inv: id -> position of its candidates.
 __global__ __launch_bounds__(256) void k_radius_targets(int K, int64_t n, const uint64_t* __restrict__ cand_key,
+                                                       const uint32_t* __restrict__ ids,
+                                                       const int32_t* __restrict__ inv,
                                                        const float* __restrict__ LS, float* __restrict__ T)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
+    const int64_t q = inv[ids[p]];
     float mx = -1.f;
     for (int k = 0; k < K; ++k) {
-        const uint64_t key = cand_key[(int64_t)k * n + p];
+        const uint64_t key = cand_key[(int64_t)k * n + q];
         if (key != kEmptyKey) mx = fmaxf(mx, __uint_as_float((uint32_t)(key >> 32)));
     }
     const float r = mx > 0.f ? sqrtf(mx) : 0.f;
@@ -467,10 +472,12 @@ void launch_radius_features(int dim, const float4* pts, const Node* nodes, int64
                        lt, n, X, LS);
 }
 
-void launch_radius_targets(int K, int64_t n, const uint64_t* cand_key, const float* LS, float* T, hipStream_t s)
+void launch_radius_targets(int K, int64_t n, const uint64_t* cand_key, const uint32_t* ids, const int32_t* inv,
+                           const float* LS, float* T, hipStream_t s)
 {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_radius_targets, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, K, n, cand_key, LS, T);
+    hipLaunchKernelGGL(k_radius_targets, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, K, n, cand_key,
+                       ids, inv, LS, T);
 }
 
 void launch_radius_seed(int64_t n, const float* model, const float* X, const float* LS, float* Y, float* R,

@@ -295,7 +295,8 @@ int emst_get_search_stats(emst_ctx* ctx, int64_t* stats, int32_t* n_stats);
  * w3[64] | b3 | feature mean[8] | feature 1/std[8] | seed offset.
  * Features (per point, all independent of the cloud's scale): log(d / s0),
  * d = distance to the nearest of the 8 nearest sorted (Morton-order)
- * positions; log(s1/s0), log(s2/s1), log(s3/s2) for the 1st..3rd enclosing
+ * positions (a run's own searches take it on their sort order, a Hilbert
+ * curve); log(s1/s0), log(s2/s1), log(s3/s2) for the 1st..3rd enclosing
  * cells; log aspect of the leaf box; distance to the leaf box boundary / s0;
  * log(median distance to those 8 neighbours / s0); length of the sum of the 8
  * neighbour offsets / sum of their lengths.  Normalised features are clamped
