@@ -424,6 +424,13 @@ int copy_out(emst_ctx* c, std::initializer_list<OutSeg> segs)
 
 int read_counters(emst_ctx* c, Counters* h) { return copy_out(c, {{h, c->C, sizeof(Counters)}}); }
 
+int64_t work_total(const Counters& h, int kind)
+{
+    unsigned long long t = 0;
+    for (int j = 0; j < kWorkSlots; ++j) t += h.work[kind][j];
+    return (int64_t)t;
+}
+
 float elapsed(hipEvent_t a, hipEvent_t b)
 {
     float ms = 0;
@@ -614,8 +621,7 @@ SplitScratch split_scratch(emst_ctx* c)
     sc.list = c->list.p;
     sc.list2 = c->list2.p;
     sc.defer = c->defer.p;
-    sc.after = 0;
-    sc.compact_frac = 0.10;
+    sc.compact_frac = 1.0;
     return sc;
 }
 
@@ -746,23 +752,24 @@ int build(emst_ctx* c)
     }
     LAUNCHCHK(c);
     HIPCHK(c, hipEventRecord(c->ev[1], s));
-    // 3D cones over 2^21 points or more: pass 0 over all queries, the open
-    // ones then resumed from a compacted list when at most 10% remain, else
-    // in place.  Measured at 10^7 points: 8% open on the clustered cloud
-    // gains 5%, 7% on a uniform one 6%.  At 10^6 points (12% open) the second
-    // launch costs more than it saves (-5%), and in 2D (8 cheap cones,
-    // 16-point leaves) the single launch is faster at every open share
-    // measured (10-26%).
+    // Full-dimensional cones over many points: pass 0 over all queries by
+    // k_cone_first, the open ones then resumed from a compacted list (resumed
+    // in place they were 4-20% slower).  Fewer points run every pass in one
+    // launch: the search then takes as long as its longest packet, and two
+    // launches have two of those.  One launch against two, ms (seed 3.5): 3D
+    // uniform 1.37 / 0.98 at 2*10^5 points and 2.22 / 1.55 at 4*10^5,
+    // clustered 2.95 / 3.57 and 3.84 / 3.58; 2D uniform 0.33 / 0.37 and
+    // 0.48 / 0.42, clustered 0.67 / 0.80 and 0.85 / 0.89.
     SplitScratch split{};
     split.open_mask = c->open_mask.p;
     split.cnt = c->open_cnt.p;
     split.off = c->open_cnt.p + ((n + 63) / 64 + 1);
     split.tmp = c->open_tmp.p;
     split.list = c->list.p;     // free until the rounds' research queue
-    split.after = 0;
     const int mode = c->opt.search_split;
-    split.compact_frac = mode == 2 ? -1.0 : (mode == 3 ? 1.0 : 0.10);
-    const bool use_split = mode == 2 || mode == 3 || (mode == 0 && c->cdim == 3 && n >= ((int64_t)1 << 21));
+    split.compact_frac = mode == 2 ? -1.0 : 1.0;
+    const bool many = c->cdim == c->dim && n >= ((int64_t)1 << (c->dim == 3 ? 18 : 19));
+    const bool use_split = mode == 2 || mode == 3 || (mode == 0 && many);
     launch_cone_search(c->dim, c->cdim, c->pts.p, c->nodes.p, c->dcl.p, c->ncl, c->bucket, leaf_table(c), n, nullptr, n,
                        c->label.p, false, c->inv.p, seed_r, c->seed_scale, c->cand_key.p, c->cand_pos.p, nullptr, c->corr.p,
                        c->corr_key.p, c->C, true, dup, use_split ? &split : nullptr, s);
@@ -795,11 +802,7 @@ int build(emst_ctx* c)
         return build(c);
     }
     c->zero_or_empty = h.zero_or_empty;
-    c->stats[0] = (int64_t)h.packets;
-    c->stats[1] = (int64_t)h.nodes;
-    c->stats[2] = (int64_t)h.leaves;
-    c->stats[3] = (int64_t)h.leaf_points;
-    c->stats[4] = (int64_t)h.pairs;
+    for (int k = 0; k < 5; ++k) c->stats[k] = work_total(h, kWorkConePackets + k);
     c->stats[5] = (int64_t)h.dup_points;
     c->stats[6] = c->grouped ? 1 : 0;
     c->stats[7] = 0;
@@ -902,11 +905,7 @@ void absorb_counters(emst_ctx* c, const Counters& h)
     c->rounds = (int)h.round;
     c->stats[7] = (int64_t)h.cycles_cut;
     c->stats[9] = (int64_t)h.comp_queries;
-    for (int k = 0; k < kWorkKinds; ++k) {
-        unsigned long long t = 0;
-        for (int j = 0; j < kWorkSlots; ++j) t += h.work[k][j];
-        c->stats[10 + k] = (int64_t)t;
-    }
+    for (int k = 0; k < kWorkCompKinds; ++k) c->stats[10 + k] = work_total(h, k);
     if (h.done == 1u) c->finished = true;
 }
 

@@ -24,8 +24,12 @@ struct Params {
 constexpr int kWorkSlots = 64;
 enum {
     kWorkCompNodes, kWorkCompLeaves, kWorkCompPairs, kWorkKnnNodes, kWorkKnnLeaves, kWorkKnnPairs,
-    kWorkCompWalks, kWorkKnnWalks, kWorkKinds
+    kWorkCompWalks, kWorkKnnWalks,
+    // the last full cone search: packets, node-test steps, leaves entered,
+    // leaf points read per packet, point pairs
+    kWorkConePackets, kWorkConeNodes, kWorkConeLeaves, kWorkConePoints, kWorkConePairs, kWorkKinds
 };
+constexpr int kWorkCompKinds = kWorkConePackets;    // the component search's kinds come first
 
 // Round counters, one device struct per context.
 struct Counters {
@@ -33,9 +37,6 @@ struct Counters {
     uint32_t research;      // points queued for a repeated cone search
     uint32_t zero_or_empty; // points holding a zero-distance or no candidate
     uint32_t unflat;        // flatten stopped at its step cap (run it again)
-    // cone-search counters of the last full search: packets (waves), nodes
-    // tested, leaves entered, leaf points read per packet, lane-point pairs
-    unsigned long long packets, nodes, leaves, leaf_points, pairs;
     // coincident-point groups (set once per build, not reset by the rounds)
     uint32_t dup_runs;      // runs of >= 2 equal keys
     uint32_t dup_points;    // points with an identical twin (group members + representatives)
@@ -217,7 +218,6 @@ struct SplitScratch {
     int32_t* list;          // n
     int32_t* list2;         // n (component search: the queries left open after pass 0)
     uint64_t* defer;        // n (component search: queries handed to the per-query pass)
-    int after;              // the first launch runs passes 0..after
     double compact_frac;    // resume from a compacted list when at most this share of the queries is open
 };
 // dim: point dimension (distances); cdim: cone dimension (cdim = 2 with dim =

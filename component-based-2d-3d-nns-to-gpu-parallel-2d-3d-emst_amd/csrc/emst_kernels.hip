@@ -1065,6 +1065,24 @@ __device__ __forceinline__ int32_t key_bound(unsigned long long k)
 }
 
 constexpr int kMaxCappedPasses = 6;
+// packets of a cone search, at least (launch_cone_search), and the resumed
+// queries up to which their packets take kConeFewPacket each
+constexpr int64_t kConePackets = 2500;
+constexpr int64_t kConeFewLeft = 65536;
+constexpr int kConeFewPacket = 16;
+
+// a packet's work counters (slots: the adds of all packets do not queue on
+// one address)
+__device__ __forceinline__ void cone_work(Counters* ctr, uint32_t nodes, uint32_t leaves, uint32_t points,
+                                          unsigned long long pairs)
+{
+    const int slot = (int)(blockIdx.x % kWorkSlots);
+    atomicAdd(&ctr->work[kWorkConePackets][slot], 1ull);
+    atomicAdd(&ctr->work[kWorkConeNodes][slot], (unsigned long long)nodes);
+    atomicAdd(&ctr->work[kWorkConeLeaves][slot], (unsigned long long)leaves);
+    atomicAdd(&ctr->work[kWorkConePoints][slot], (unsigned long long)points);
+    atomicAdd(&ctr->work[kWorkConePairs][slot], pairs);
+}
 
 // Cone search, exact, by iterative deepening (the tree form of the Elias ring
 // expansion).  Pass k caps every open cone's bound at R_k^2 (R_0 = the seed,
@@ -1113,14 +1131,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DC == 3 ? 3 
                                                    uint64_t* __restrict__ open_out,
                                                    const uint32_t* __restrict__ nq_dev,
                                                    const uint64_t* __restrict__ resume_mask,
-                                                   int64_t compact_max)
+                                                   int64_t compact_max, int qpp)
 {
     using C = ConeCfg<DC>;
     bool compacted = true;
     if (nq_dev) {
         nq = *nq_dev;
         compacted = nq <= compact_max;
-        if (compacted ? (int64_t)blockIdx.x * 64 >= nq : resume_mask[blockIdx.x] == 0ull)
+        // few queries left: narrower packets (the grid covers 64 to a packet
+        // of every query; 41213 left of 200003 1.23 -> 0.97 ms for the search,
+        // while 145434 left of 10^6 lose 0.3)
+        if (compacted && nq <= kConeFewLeft && nq <= (int64_t)gridDim.x * kConeFewPacket) qpp = kConeFewPacket;
+        if (compacted ? (int64_t)blockIdx.x * qpp >= nq : resume_mask[blockIdx.x] == 0ull)
             return;     // nothing to resume in this packet
     }
     __shared__ unsigned long long best[C::K][64];
@@ -1128,11 +1150,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DC == 3 ? 3 
     __shared__ int32_t stk_ver[64];
     __shared__ unsigned long long stk_mask[64];
     const int lane = __lane_id();
-    const int64_t qi = (int64_t)blockIdx.x * 64 + lane;
+    const int64_t qi = (int64_t)blockIdx.x * (compacted ? qpp : 64) + lane;
     bool active;
     int64_t p;
     if (compacted) {
-        active = qi < nq;
+        active = lane < qpp && qi < nq;
         p = active ? (qlist ? (int64_t)qlist[qi] : qi) : 0;
     } else {
         active = (resume_mask[blockIdx.x] >> lane) & 1ull;     // set bits are points of this packet
@@ -1206,6 +1228,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DC == 3 ? 3 
 #pragma unroll
             for (int c = 0; c < C::K; ++c)
                 if (mine && key_bound(best[c][lane]) > inner) open |= 1u << c;
+            // no point found so far: the passes before pass_lo saw an empty
+            // ball, or left the query out (k_cone_first); it starts over
+            bool none = true;
+#pragma unroll
+            for (int c = 0; c < C::K; ++c) none = none && best[c][lane] == kEmptyKey;
+            if (none) {
+                inner = -1;
+                r2 = r * r;
+            }
         }
         int32_t bound[C::K];
         int32_t maxb = -1;
@@ -1384,11 +1415,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DC == 3 ? 3 
         if (mine) open_final = open;
     }
     if (collect_stats && lane == 0) {
-        atomicAdd(&ctr->packets, 1ull);
-        atomicAdd(&ctr->nodes, (unsigned long long)st_nodes);
-        atomicAdd(&ctr->leaves, (unsigned long long)st_leaves);
-        atomicAdd(&ctr->leaf_points, (unsigned long long)st_pts);
-        atomicAdd(&ctr->pairs, (unsigned long long)st_pairs);
+        cone_work(ctr, st_nodes, st_leaves, st_pts, st_pairs);
     }
     if (__ballot(underflow) != 0ull && lane == 0) atomicOr(&ctr->underflow, 1u);
     if (open_out) {
@@ -1427,6 +1454,488 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DC == 3 ? 3 
         first_corr[p] = pmin >= 0 ? pmin : -2;
         first_key[p] = kmin;
     }
+}
+
+// minimum over the wave, the same in every lane
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v)
+{
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false));     // quad_perm [1,0,3,2]
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false));     // quad_perm [2,3,0,1]
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, false));    // row_half_mirror
+    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, false));    // row_mirror
+    // one value per row of 16
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    return min(min(a, b), min(c, d));
+}
+
+__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
+{
+    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, m);
+    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), m);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// A gathering starts from every node of depth min(6, leaf depth), 64 at most,
+// one per lane: the levels above would each take a dependent step for a few
+// nodes.  Returns the count written to work[].
+__device__ __forceinline__ int gather_start(int64_t L, int32_t* work)
+{
+    int d0 = 0;
+    while (d0 < 6 && ((int64_t)2 << d0) <= L) ++d0;
+    const int cnt = 1 << d0;
+    const int lane = __lane_id();
+    if (lane < cnt) work[lane] = cnt + lane;
+    __builtin_amdgcn_wave_barrier();
+    return cnt;
+}
+
+// The gathering's next nodes from the inner nodes that passed: each hands on
+// its 4 grandchildren (one 128-byte line of the heap), or its 2 children when
+// those are leaves.  Every gathering test (box distance, far side, component
+// label, empty) is monotone under box inclusion, so a grandchild whose parent
+// would have failed fails too: the same nodes pass as level by level, in half
+// the dependent steps.  Writes the entries at work[tail ..] and their count to
+// add; false (nothing written) when they would pass cap.
+__device__ __forceinline__ bool push_inner(bool pass, int nd, int64_t L, int32_t* work, int tail, int cap,
+                                           int& add)
+{
+    const bool deep = pass && 2 * (int64_t)nd < L;     // its children are inner nodes
+    const uint64_t m4 = __ballot(deep), m2 = __ballot(pass && !deep);
+    add = 4 * __popcll(m4) + 2 * __popcll(m2);
+    if (tail + add > cap) return false;
+    const uint64_t lt = lanemask_lt();
+    const int r = tail + 4 * __popcll(m4 & lt) + 2 * __popcll(m2 & lt);
+    if (deep) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) work[r + k] = 4 * nd + k;
+    } else if (pass) {
+        work[r] = 2 * nd;
+        work[r + 1] = 2 * nd + 1;
+    }
+    return true;
+}
+
+// ascending bitonic sort of one 64-bit key per lane across the wave
+__device__ __forceinline__ uint64_t wave_sort_u64(uint64_t e)
+{
+    const int lane = __lane_id();
+#pragma unroll
+    for (int k = 2; k <= 64; k <<= 1) {
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            const uint64_t o = shfl_xor_u64(e, j);
+            const bool keep_min = ((lane & j) == 0) == ((lane & k) == 0);
+            e = keep_min ? (o < e ? o : e) : (o > e ? o : e);
+        }
+    }
+    return e;
+}
+
+// ---- first pass of the cone search over every query (k_cone_first) ----
+//
+// One wave per 64 consecutive positions; each lane is one query with its cone
+// bests in its own column of LDS.  The wave gathers the leaves within the
+// lanes' first radius R_0 of the packet's box (64 node tests a step), keeps
+// per leaf the 8-lane groups whose box it can matter to, and then takes the
+// leaf points one at a time, at one address for the whole wave: every lane
+// pairs the point with its own query.  A point enters only when it lies
+// within the largest radius of a needed group from that group's box.
+//
+// Against one query at a time per leaf (k_cone_search), where 64 lanes pair a
+// leaf's 25-50 points with each query that needs the leaf: the pairs that lie
+// beyond every radius are dropped 64 at a time, no query state is broadcast,
+// and a lane's minimum goes to its own column, where no other lane's atomic
+// waits on the same address.
+//
+// Cones are kept as axis * 2^D + octant (the signs of the offset): that
+// index comes from three sign bits and two compares.  An offset on a boundary
+// between cones (a zero coordinate, or equal largest coordinates) lies in
+// several and takes cone_octants.
+//
+// A query with a cone whose best lies beyond R_0 stores its bests and is left
+// open (open_out) for k_cone_search, which goes on from pass 1.  A packet
+// whose gathering outgrows the LDS lists (a thin point's radius over a dense
+// cluster) is left open without a best, and k_cone_search starts it over: a
+// wave that took all those points one by one was the kernel's tail.  (The
+// search of 4*10^6 clustered points, seed 3.5: lists of 256 leaves 15.0 ms,
+// of 128 11.0; trying halves of such a packet again, down to 32 or 8 lanes,
+// 11.0 and 12.7.)
+//
+// Bound by VALU issue: 32000 instructions a packet of uniform 3D points (60
+// leaves, 930 points a lane, 24 instructions a pair; seed 3.5), 71% of the
+// cycles busy; 12.5 KB of bests and lists and 1 KB of batch allow 11 waves per
+// CU.  Points through scalar loads instead of LDS waited on the scalar cache
+// (1.25 times as long); four streams of 16 lanes with a list of points each
+// took 18% fewer steps and as long.  The whole search against k_cone_search
+// alone: 10^6 uniform points 4.4 -> 2.9 ms in 3D, 0.95 -> 0.79 in 2D; 4*10^6
+// clustered ones 18.2 -> 12.4 (with the seed model 17.3 -> 12.8), power-law
+// ones in 2D 4.2 -> 3.6.
+constexpr int kFirstWork = 1024;
+constexpr int kFirstLeaves = 128;
+constexpr int kFirstChunks = kFirstLeaves / 64;
+
+// the cones of an offset as bits axis * 2^D + octant: the face of every
+// axis whose |d| is the largest, with both signs of each zero coordinate off
+// that axis (cone_mask in the other numbering)
+template <int D>
+__device__ __forceinline__ uint32_t cone_octants(float dx, float dy, float dz)
+{
+    const float ax = fabsf(dx), ay = fabsf(dy), az = D == 3 ? fabsf(dz) : 0.f;
+    const float m = fmaxf(fmaxf(ax, ay), az);
+    constexpr uint32_t all = D == 3 ? 0xffu : 0xfu;
+    const uint32_t px = 0x55u & all, py = 0x33u & all, pz = 0x0fu;      // octants of '+' signs
+    const uint32_t sx = dx < 0.f ? all ^ px : px, sy = dy < 0.f ? all ^ py : py;
+    const uint32_t sz = D == 3 ? (dz < 0.f ? all ^ pz : pz) : all;
+    const uint32_t ex = dx == 0.f ? all : sx, ey = dy == 0.f ? all : sy;
+    const uint32_t ez = D == 3 && dz == 0.f ? all : sz;
+    uint32_t r = 0;
+    if (ax >= m) r |= sx & ey & ez;
+    if (ay >= m) r |= (ex & sy & ez) << (1 << D);
+    if (D == 3 && az >= m) r |= (ex & ey & sz) << (2 << D);
+    return r;
+}
+
+// the row of cone c (face * 2^(D-1) + slab) in that numbering
+template <int D>
+__device__ __forceinline__ constexpr int cone_row(int c)
+{
+    const int face = c / ConeCfg<D>::NS, slab = c % ConeCfg<D>::NS;
+    const int axis = face / 2;
+    int oct = (face & 1) << axis, bit = 0;
+    for (int k = 0; k < D; ++k)
+        if (k != axis) oct |= ((slab >> bit++) & 1) << k;
+    return axis * (1 << D) + oct;
+}
+
+template <int D>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D == 3 ? 3 : 4))) void k_cone_first(
+    const float4* __restrict__ pts, const Node* __restrict__ nodes, const Cloud* __restrict__ clouds, int ncl,
+    int bucket, LeafTable lt, int64_t n, const int32_t* __restrict__ inv, const float* __restrict__ seed_r,
+    float seed_scale, uint64_t* __restrict__ cand_key, int32_t* __restrict__ cand_pos,
+    int32_t* __restrict__ first_corr, uint64_t* __restrict__ first_key, Counters* __restrict__ ctr,
+    int collect_stats, DupState dup, uint64_t* __restrict__ open_out)
+{
+    using C = ConeCfg<D>;
+    static_assert(C::K == D * (1 << D), "one row per axis and octant");
+    // the gathering's lists and the cone bests take turns in the same LDS
+    constexpr int kListWords = kFirstLeaves + kFirstWork / 2;
+    constexpr int kBestWords = C::K * 64;
+    __shared__ unsigned long long lds[kBestWords > kListWords ? kBestWords : kListWords];
+    __shared__ float4 gbox[16];             // per 8-lane group: lo (xyz), hi (xyz)
+    __shared__ float4 batch[64];            // leaf points waiting to be paired
+    unsigned long long* best = lds;         // [row][lane]
+    unsigned long long* gathered = lds;
+    int32_t* work = reinterpret_cast<int32_t*>(lds + kFirstLeaves);
+    const int lane = __lane_id();
+    const int64_t p = (int64_t)blockIdx.x * 64 + lane;
+    bool active = p < n;
+    // grouping on: as in k_cone_search, members do not search and no point
+    // takes a candidate at its own location
+    const bool grouped = dup.rep != nullptr;
+    bool is_rep = false;
+    if (grouped && active) {
+        const int32_t r = dup.rep[p];
+        active = r < 0 || r == (int32_t)p;
+        is_rep = r == (int32_t)p;
+    }
+    const float4 me = pts[p < n ? p : n - 1];
+    const float px = me.x, py = me.y, pz = me.z;
+    const int my_cl = active ? find_cloud(clouds, ncl, p) : -1;
+    const int lb = 31 - __builtin_clz(bucket);      // log2
+    const int per_step = 64 >> lb;                  // leaves per step of 64 lanes
+    uint32_t st_nodes = 0, st_leaves = 0, st_pts = 0, st_pairs = 0;
+    bool underflow = false;
+    uint64_t open_lanes = 0;
+    uint64_t pending = __ballot(active);
+    while (pending) {
+        const int cl = __builtin_amdgcn_readfirstlane(__shfl(my_cl, (int)__builtin_ctzll(pending)));
+        const bool mine = my_cl == cl;
+        pending &= ~__ballot(mine);
+        const int64_t L = clouds[cl].L, lfirst = clouds[cl].lfirst;
+        const Node* __restrict__ tree = nodes + 2 * clouds[cl].lbase;
+        float r = 1.f;
+        if (!mine) {
+            // not this traversal's query
+        } else if (seed_r) {
+            r = seed_r[p];
+            if (!positive_finite(r)) r = 1e-6f;
+        } else {
+            const int64_t lf = lt.of[p];
+            const Node own = tree[L + (lf - lfirst)];
+            const float cnt = (float)(lt.start[lf + 1] - lt.start[lf]);
+            float vol = 1.f, ext = 0.f;
+            for (int k = 0; k < D; ++k) {
+                const float e = own.hi[k] - own.lo[k];
+                vol *= e;
+                ext = fmaxf(ext, e);
+            }
+            float sp = vol > 0.f ? powf(vol / cnt, 1.f / D) : ext / cnt;
+            if (!positive_finite(sp)) sp = 1e-6f;
+            r = seed_scale * sp;
+        }
+        const float r2 = r * r;
+        // boxes of the lanes and of each 8-lane group
+        float qlo[3] = {mine ? px : INFINITY, mine ? py : INFINITY, mine ? pz : INFINITY};
+        float qhi[3] = {mine ? px : -INFINITY, mine ? py : -INFINITY, mine ? pz : -INFINITY};
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                qlo[k] = fminf(qlo[k], __shfl_xor(qlo[k], off));
+                qhi[k] = fmaxf(qhi[k], __shfl_xor(qhi[k], off));
+            }
+            if (off == 4 && (lane & 7) == 0) {
+                gbox[2 * (lane >> 3)] = make_float4(qlo[0], qlo[1], qlo[2], 0.f);
+                gbox[2 * (lane >> 3) + 1] = make_float4(qhi[0], qhi[1], qhi[2], 0.f);
+            }
+        }
+        // the bound per lane, the groups' largest (a group without lanes:
+        // its box is empty), and the largest of all
+        float cap = mine ? r2 : -1.f;
+        uint32_t t8 = group8_max_u32(mine ? __float_as_uint(r2) : 0u);
+        uint32_t B = t8;
+#pragma unroll
+        for (int off = 8; off < 64; off <<= 1) B = max(B, (uint32_t)__shfl_xor((int)B, off));
+        B = (uint32_t)__builtin_amdgcn_readfirstlane((int)B);
+        __builtin_amdgcn_wave_barrier();
+        auto group_d2 = [&](int g, float x0, float y0, float z0, float x1, float y1, float z1) {
+            const float4 a = gbox[2 * g], b = gbox[2 * g + 1];
+            const float m0 = fmaxf(fmaxf(x0 - b.x, a.x - x1), 0.f);
+            const float m1 = fmaxf(fmaxf(y0 - b.y, a.y - y1), 0.f);
+            const float m2 = fmaxf(fmaxf(z0 - b.z, a.z - z1), 0.f);
+            return __float_as_uint(D == 3 ? d2_of(m0, m1, m2) : d2_of(m0, m1));
+        };
+        // gather: key = (box d2 bits without the low 8 | group mask) << 32 | node
+        int head = 0, tail = gather_start(L, work), ngl = 0;
+        bool over = B >= 0x7f800000u;       // (an unbounded first radius: not a capped pass)
+        __builtin_amdgcn_wave_barrier();
+        while (head < tail && !over) {
+            const int take = min(64, tail - head);
+            const int nd = lane < take ? work[head + lane] : 0;
+            head += take;
+            ++st_nodes;
+            bool pass = false, leaf = false;
+            uint32_t bd = 0, gm = 0;
+            if (lane < take) {
+                const Node x = tree[nd];
+                float m[3];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) m[k] = fmaxf(fmaxf(x.lo[k] - qhi[k], qlo[k] - x.hi[k]), 0.f);
+                bd = __float_as_uint(D == 3 ? d2_of(m[0], m[1], m[2]) : d2_of(m[0], m[1]));
+                leaf = nd >= L;
+                pass = bd <= B && bd < 0x7f800000u;     // (an empty box lies at infinity)
+                if (pass && leaf) {
+#pragma unroll
+                    for (int g = 0; g < 8; ++g) {
+                        const uint32_t tg = (uint32_t)__builtin_amdgcn_readlane((int)t8, 8 * g);
+                        const uint32_t d = group_d2(g, x.lo[0], x.lo[1], x.lo[2], x.hi[0], x.hi[1], x.hi[2]);
+                        gm |= d <= tg ? 1u << g : 0u;
+                    }
+                    pass = gm != 0u;
+                }
+            }
+            const uint64_t ml = __ballot(pass && leaf);
+            const int nlf = __popcll(ml);
+            int add;
+            if (!push_inner(pass && !leaf, nd, L, work, tail, kFirstWork, add) || ngl + nlf > kFirstLeaves) {
+                over = true;
+                break;
+            }
+            if (pass && leaf)
+                gathered[ngl + __popcll(ml & lanemask_lt())] =
+                    ((uint64_t)((bd & 0xffffff00u) | gm) << 32) | (uint32_t)nd;
+            tail += add;
+            ngl += nlf;
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (over) {
+            // too far for the lists: left open without a best
+            if (mine)
+                for (int c = 0; c < C::K; ++c) cand_key[(int64_t)c * n + p] = kEmptyKey;
+            open_lanes |= __ballot(mine);
+            continue;
+        }
+        // the leaves, nearest first 64 at a time, now in registers
+        uint64_t ent[kFirstChunks];
+#pragma unroll
+        for (int k = 0; k < kFirstChunks; ++k) {
+            ent[k] = kEmptyKey;
+            if (64 * k < ngl) {
+                const uint64_t e = 64 * k + lane < ngl ? gathered[64 * k + lane] : kEmptyKey;
+                ent[k] = wave_sort_u64(e);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int c = 0; c < C::K; ++c) best[c * 64 + lane] = kEmptyKey;
+        __builtin_amdgcn_wave_barrier();
+        st_leaves += (uint32_t)ngl;
+        const uint32_t nin = (uint32_t)__popcll(__ballot(mine));
+        // one leaf point against every lane's query; true where it lies
+        // on a boundary between cones (lower_all)
+        auto pair = [&](const float4 q) {
+            const float dx = q.x - px, dy = q.y - py, dz = q.z - pz;
+            const float d2 = D == 3 ? d2_of(dx, dy, dz) : d2_of(dx, dy);
+            const float ax = fabsf(dx), ay = fabsf(dy), az = fabsf(dz);
+            float m, second, least;
+            if (D == 3) {
+                m = fmaxf(fmaxf(ax, ay), az);
+                second = __builtin_amdgcn_fmed3f(ax, ay, az);
+                least = fminf(fminf(ax, ay), az);
+            } else {
+                m = fmaxf(ax, ay);
+                second = least = fminf(ax, ay);
+            }
+            uint32_t row = D == 3 ? __float_as_uint(dz) >> 31 : 0u;
+            row = (row << 1) | (__float_as_uint(dy) >> 31);
+            row = (row << 1) | (__float_as_uint(dx) >> 31);
+            if (D == 3) row |= ax == m ? 0u : (ay == m ? 8u : 16u);
+            else row |= ax == m ? 0u : 4u;
+            const bool near = d2 <= cap;
+            const bool plain = least > 0.f && second < m;
+            if (near && plain)
+                atomicMin(&best[row * 64 + lane],
+                          ((unsigned long long)__float_as_uint(d2) << 32) | __float_as_uint(q.w));
+            return near && !plain;
+        };
+        auto lower_all = [&](const float4 q) {
+            const float dx = q.x - px, dy = q.y - py, dz = q.z - pz;
+            const float d2 = D == 3 ? d2_of(dx, dy, dz) : d2_of(dx, dy);
+            const bool self = __float_as_uint(q.w) == __float_as_uint(me.w);
+            const bool here = dx == 0.f && dy == 0.f && dz == 0.f;
+            if (d2 <= cap && !(grouped ? here : self)) {
+                uint32_t rows = cone_octants<D>(dx, dy, dz);
+                while (rows) {
+                    const int row = __builtin_ctz(rows);
+                    rows &= rows - 1;
+                    atomicMin(&best[row * 64 + lane],
+                              ((unsigned long long)__float_as_uint(d2) << 32) | __float_as_uint(q.w));
+                }
+            }
+        };
+        // the points kept so far, padded to a multiple of 4 with points
+        // beyond every bound
+        int held = 0;
+        auto drain = [&]() {
+            if (lane < 3 && held + lane < 64) batch[held + lane] = make_float4(INFINITY, INFINITY, INFINITY, me.w);
+            __builtin_amdgcn_wave_barrier();
+            for (int j = 0; j < held; j += 4) {
+                float4 q[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) q[u] = batch[j + u];
+                bool tie = false;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) tie |= pair(q[u]);
+                // (every query meets itself here once, a zero offset)
+                if (__ballot(tie) != 0ull) {
+#pragma unroll 1
+                    for (int u = 0; u < 4; ++u) if (tie) lower_all(batch[j + u]);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            held = 0;
+        };
+        for (int c0 = 0; c0 < ngl; c0 += 64) {
+            const int cn = min(64, ngl - c0);
+            const int ck = c0 >> 6;
+            uint64_t e = ent[0];
+#pragma unroll
+            for (int k = 1; k < kFirstChunks; ++k) e = ck == k ? ent[k] : e;
+            const int e_node = (int)(uint32_t)e;
+            const uint32_t e_gm = (uint32_t)(e >> 32) & 0xffu;
+            // this lane's leaf point of the step's leaves
+            auto fetch = [&](int i, bool& has, float4& w) {
+                const int idx = i + (lane >> lb);
+                const int node = __shfl(e_node, idx & 63);
+                has = false;
+                w = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (idx < cn) {
+                    const int64_t lf = lfirst + (node - L);
+                    const int32_t s0 = lt.start[lf] + (lane & (bucket - 1));
+                    has = s0 < lt.start[lf + 1];
+                    if (has) w = pts[s0];
+                }
+            };
+            bool has, nhas;
+            float4 w, nw;
+            fetch(0, nhas, nw);
+            for (int i = 0; i < cn; i += per_step) {
+                has = nhas;
+                w = nw;
+                if (i + per_step < cn) fetch(i + per_step, nhas, nw);
+                uint32_t gm = 0;
+                for (int k = i; k < min(cn, i + per_step); ++k) gm |= (uint32_t)__builtin_amdgcn_readlane((int)e_gm, k);
+                // the points within reach of a needed group
+                bool keep = false;
+                while (gm) {
+                    const int g = __builtin_ctz(gm);
+                    gm &= gm - 1;
+                    const uint32_t tg = (uint32_t)__builtin_amdgcn_readlane((int)t8, 8 * g);
+                    keep = keep || group_d2(g, w.x, w.y, w.z, w.x, w.y, w.z) <= tg;
+                }
+                keep = keep && has;
+                const uint64_t cand = __ballot(keep);
+                const int steps = __popcll(cand);
+                st_pts += (uint32_t)__popcll(__ballot(has));
+                st_pairs += (uint32_t)steps * nin;
+                if (held + steps > 64) {
+                    drain();
+                    // a lane whose cones all hold a point searches no
+                    // farther than the farthest of them
+                    uint32_t far = 0;
+#pragma unroll
+                    for (int c = 0; c < C::K; ++c) far = max(far, (uint32_t)(best[c * 64 + lane] >> 32));
+                    if (mine && far < __float_as_uint(cap)) cap = __uint_as_float(far);
+                    t8 = group8_max_u32(mine ? __float_as_uint(cap) : 0u);
+                }
+                if (keep) batch[held + __popcll(cand & lanemask_lt())] = w;
+                held += steps;
+            }
+        }
+        if (held > 0) drain();
+        __builtin_amdgcn_wave_barrier();
+        // results of these lanes: open when a cone's best lies beyond R_0
+        bool open = false;
+        uint64_t kmin = kEmptyKey;
+#pragma unroll
+        for (int c = 0; c < C::K; ++c) {
+            const uint64_t k = best[cone_row<D>(c) * 64 + lane];
+            open = open || key_bound(k) > (int32_t)__float_as_uint(r2);
+            kmin = k < kmin ? k : kmin;
+        }
+        open = open && mine;
+        open_lanes |= __ballot(open);
+        // distinct points at float distance 0 break the grouping's
+        // premise; the caller then searches ungrouped
+        if (grouped && mine && (kmin >> 32) == 0u) underflow = true;
+        if (mine) {
+            const int64_t gs = is_rep ? (int64_t)dup.gslot[p] : 0;
+            int32_t pmin = -1;
+            for (int c = 0; c < C::K; ++c) {
+                const uint64_t k = best[cone_row<D>(c) * 64 + lane];
+                cand_key[(int64_t)c * n + p] = k;
+                if (open) continue;
+                const int32_t q = k == kEmptyKey ? -1 : inv[(uint32_t)k];
+                cand_pos[(int64_t)c * n + p] = q;
+                if (k == kmin) pmin = q;
+                if (is_rep && ((c / C::NS) & 1) == 0) {
+                    const int64_t b = (int64_t)((c / C::NS / 2) * C::NS + c % C::NS) * dup.ngroups + gs;
+                    dup.bkey[b] = k;
+                    dup.bpos[b] = q;
+                }
+            }
+            if (!open && first_corr) {
+                first_corr[p] = pmin >= 0 ? pmin : -2;
+                first_key[p] = kmin;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (lane == 0) open_out[blockIdx.x] = open_lanes;
+    if (collect_stats && lane == 0) cone_work(ctr, st_nodes, st_leaves, st_pts, st_pairs);
+    if (__ballot(underflow) != 0ull && lane == 0) atomicOr(&ctr->underflow, 1u);
 }
 
 // Queries left open by a split cone search, in position order: per-packet
@@ -1662,7 +2171,6 @@ __global__ __launch_bounds__(kBlock) void k_round_init(int64_t n, int32_t* __res
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
         C->edges = 0; C->research = 0; C->zero_or_empty = 0; C->unflat = 0;
-        C->packets = C->nodes = C->leaves = C->leaf_points = C->pairs = 0;
         C->round = 0; C->done = C->invalid ? 1u : 0u; C->edges_prev = 0; C->dup_settled = 0; C->nsamples = 0;
         C->comp_queries = 0;
         C->deferred = 0;
@@ -2541,82 +3049,6 @@ constexpr int kSmallPacket = 8;
 // largest K-th distance after its own leaves, so they reach further
 constexpr int kKnnGatherWork = 1024;
 constexpr int kKnnGatherLeaves = 256;
-
-// minimum over the wave, the same in every lane
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v)
-{
-    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false));     // quad_perm [1,0,3,2]
-    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false));     // quad_perm [2,3,0,1]
-    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, false));    // row_half_mirror
-    v = min(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, false));    // row_mirror
-    // one value per row of 16
-    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
-    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
-    return min(min(a, b), min(c, d));
-}
-
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
-{
-    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, m);
-    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), m);
-    return ((uint64_t)hi << 32) | lo;
-}
-
-// A gathering starts from every node of depth min(6, leaf depth), 64 at most,
-// one per lane: the levels above would each take a dependent step for a few
-// nodes.  Returns the count written to work[].
-__device__ __forceinline__ int gather_start(int64_t L, int32_t* work)
-{
-    int d0 = 0;
-    while (d0 < 6 && ((int64_t)2 << d0) <= L) ++d0;
-    const int cnt = 1 << d0;
-    const int lane = __lane_id();
-    if (lane < cnt) work[lane] = cnt + lane;
-    __builtin_amdgcn_wave_barrier();
-    return cnt;
-}
-
-// The gathering's next nodes from the inner nodes that passed: each hands on
-// its 4 grandchildren (one 128-byte line of the heap), or its 2 children when
-// those are leaves.  Every gathering test (box distance, far side, component
-// label, empty) is monotone under box inclusion, so a grandchild whose parent
-// would have failed fails too: the same nodes pass as level by level, in half
-// the dependent steps.  Writes the entries at work[tail ..] and their count to
-// add; false (nothing written) when they would pass cap.
-__device__ __forceinline__ bool push_inner(bool pass, int nd, int64_t L, int32_t* work, int tail, int cap,
-                                           int& add)
-{
-    const bool deep = pass && 2 * (int64_t)nd < L;     // its children are inner nodes
-    const uint64_t m4 = __ballot(deep), m2 = __ballot(pass && !deep);
-    add = 4 * __popcll(m4) + 2 * __popcll(m2);
-    if (tail + add > cap) return false;
-    const uint64_t lt = lanemask_lt();
-    const int r = tail + 4 * __popcll(m4 & lt) + 2 * __popcll(m2 & lt);
-    if (deep) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) work[r + k] = 4 * nd + k;
-    } else if (pass) {
-        work[r] = 2 * nd;
-        work[r + 1] = 2 * nd + 1;
-    }
-    return true;
-}
-
-// ascending bitonic sort of one 64-bit key per lane across the wave
-__device__ __forceinline__ uint64_t wave_sort_u64(uint64_t e)
-{
-    const int lane = __lane_id();
-#pragma unroll
-    for (int k = 2; k <= 64; k <<= 1) {
-#pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            const uint64_t o = shfl_xor_u64(e, j);
-            const bool keep_min = ((lane & j) == 0) == ((lane & k) == 0);
-            e = keep_min ? (o < e ? o : e) : (o > e ? o : e);
-        }
-    }
-    return e;
-}
 
 // nearest point in another component, for the points of qlist (count in
 // nq_dev): packet traversal as in the cone search, one best per query, by
@@ -4116,27 +4548,43 @@ void launch_cone_search(int dim, int cdim, const float4* pts, const Node* nodes,
     const unsigned g = nblocks(nq, 64);
     const int cs = collect_stats ? 1 : 0;
     auto kern = dim == 3 ? (cdim == 2 ? k_cone_search<3, 2> : k_cone_search<3, 3>) : k_cone_search<2, 2>;
-    if (!split || qlist || split->after < 0 || split->after >= kMaxCappedPasses) {
-        hipLaunchKernelGGL(kern, dim3(g), dim3(64), 0, s, pts, nodes, cl, ncl, bucket, lt, n, qlist, nq, label,
-                           check_labels ? 1 : 0, inv, seed_r, seed_scale, cand_key, cand_pos, revive, first_corr,
+    if (!split || qlist) {
+        // Few queries: fewer to a packet, so that there are some 2500 packets
+        // at least (ten waves a CU) and each is shorter: a launch of few
+        // packets takes as long as one of them (2D / 3D, ms, 64 to a packet
+        // against this rule: 1379 points 0.20 / 0.47 and 0.07 / 0.14, 10^4
+        // 0.21 / 0.68 and 0.12 / 0.29, 3*10^4 0.23 / 0.75 and 0.16 / 0.51;
+        // 10^5 points take 64).
+        int qpp = 1;
+        while (qpp < 64 && (int64_t)qpp * kConePackets < nq) qpp <<= 1;
+        hipLaunchKernelGGL(kern, dim3(nblocks(nq, qpp)), dim3(64), 0, s, pts, nodes, cl, ncl, bucket, lt, n, qlist,
+                           nq, label, check_labels ? 1 : 0, inv, seed_r, seed_scale, cand_key, cand_pos, revive, first_corr,
                            first_key, C, cs, dup, 0, kMaxCappedPasses, (uint64_t*)nullptr,
-                           (const uint32_t*)nullptr, (const uint64_t*)nullptr, (int64_t)0);
+                           (const uint32_t*)nullptr, (const uint64_t*)nullptr, (int64_t)0, qpp);
         return;
     }
-    // passes 0..after over every query, then the open ones compacted into full waves
+    // pass 0 over every query, then the open ones compacted into full waves.
+    // The wedges of the 2.5D mode are unbounded in z, so their bests tighten
+    // early and the per-face node test drops most of what a radius would keep:
+    // k_cone_search stays faster there (4.3 against 6.2 ms, 3*10^6 points).
     const int64_t P = (int64_t)g;
-    hipLaunchKernelGGL(kern, dim3(g), dim3(64), 0, s, pts, nodes, cl, ncl, bucket, lt, n, qlist, nq, label,
-                       check_labels ? 1 : 0, inv, seed_r, seed_scale, cand_key, cand_pos, revive, first_corr,
-                       first_key, C, cs, dup, 0, split->after, split->open_mask, (const uint32_t*)nullptr,
-                       (const uint64_t*)nullptr, (int64_t)0);
+    if (cdim == dim)
+        hipLaunchKernelGGL(dim == 3 ? (k_cone_first<3>) : (k_cone_first<2>), dim3(g), dim3(64), 0, s, pts, nodes, cl,
+                           ncl, bucket, lt, n, inv, seed_r, seed_scale, cand_key, cand_pos, first_corr, first_key, C,
+                           cs, dup, split->open_mask);
+    else
+        hipLaunchKernelGGL(kern, dim3(g), dim3(64), 0, s, pts, nodes, cl, ncl, bucket, lt, n, qlist, nq, label,
+                           check_labels ? 1 : 0, inv, seed_r, seed_scale, cand_key, cand_pos, revive, first_corr,
+                           first_key, C, cs, dup, 0, 0, split->open_mask, (const uint32_t*)nullptr,
+                           (const uint64_t*)nullptr, (int64_t)0, 64);
     hipLaunchKernelGGL(k_open_count, dim3(nblocks(P + 1)), dim3(kBlock), 0, s, split->open_mask, P, split->cnt);
     exclusive_scan_u32(split->cnt, split->off, P + 1, split->tmp, s);
     hipLaunchKernelGGL(k_open_fill, dim3((unsigned)P), dim3(64), 0, s, split->open_mask, split->off, split->list);
     hipLaunchKernelGGL(kern, dim3(g), dim3(64), 0, s, pts, nodes, cl, ncl, bucket, lt, n,
                        (const int32_t*)split->list, nq, label, check_labels ? 1 : 0, inv, seed_r, seed_scale,
-                       cand_key, cand_pos, revive, first_corr, first_key, C, cs, dup, split->after + 1, kMaxCappedPasses,
+                       cand_key, cand_pos, revive, first_corr, first_key, C, cs, dup, 1, kMaxCappedPasses,
                        (uint64_t*)nullptr, (const uint32_t*)(split->off + P), (const uint64_t*)split->open_mask,
-                       (int64_t)(split->compact_frac * (double)nq));
+                       (int64_t)(split->compact_frac * (double)nq), 64);
 }
 
 void launch_leaves(const uint64_t* keys, int64_t n, Cloud* cl, int ncl, int bucket, uint32_t* mark,

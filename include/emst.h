@@ -66,9 +66,8 @@ typedef struct {
                                skips that round's hook (emst_get_search_stats entry 7 counts
                                these).  Not with the learned seed radius. */
     int32_t search_split;   /* round-1 cone search launches (changes work, never results):
-                               0 auto (3D cones and >= 2^21 points: 3 when at most 10% of the
-                               queries are left with open cones after the first pass, else 2;
-                               otherwise 1); 1 one launch for
+                               0 auto (3 from 2^18 points in 3D and 2^19 in 2D, not in the
+                               2.5D mode; otherwise 1); 1 one launch for
                                every pass; 2 first pass, then the open queries resumed in place;
                                3 first pass, then the open queries compacted into full waves */
     int32_t round_search;   /* 0: round-1 cone search, candidates reused by every round (the
@@ -260,9 +259,10 @@ int emst_get_times(emst_ctx* ctx, float* times, int32_t* n_times);
 int emst_get_round_ends(emst_ctx* ctx, float* ms, int32_t* n);
 
 /* Counters of the last full cone search (the work behind its bytes):
- * [0] packets (64-point waves), [1] hierarchy nodes tested, [2] leaf cells
- * entered, [3] leaf points read (summed over packets), [4] point pairs
- * evaluated (leaf points x lanes that needed the leaf), [5] points sharing
+ * [0] packets (waves of at most 64 queries), [1] node-test steps (a hierarchy
+ * node against a packet's queries, or up to 64 nodes against the packet's
+ * box), [2] leaf cells entered, [3] leaf points read (summed over packets), [4] point pairs
+ * evaluated (leaf points x lanes that took them), [5] points sharing
  * their location with another point, [6] 1 when those were searched as
  * groups (one search per location), 0 when every point searched itself,
  * [7] hooks withheld by the 2.5D mode's cycle rule over the rounds run so far,
