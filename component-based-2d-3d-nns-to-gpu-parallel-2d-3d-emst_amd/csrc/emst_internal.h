@@ -175,10 +175,12 @@ void launch_bbox(const float* xyz, const Cloud* cl, int ncl, int64_t N, int dim,
 void launch_params(Params* P, const Cloud* cl, int ncl, int dim, int mbits, hipStream_t s);
 void launch_rescale_keys(const float* xyz, const Cloud* cl, int ncl, int64_t N, int dim, int mbits,
                            const Params* P, float* resc, uint64_t* keys, bool hilbert, hipStream_t s);
-// LSD radix sort of (keys, vals) by bits [0, bits); result lands in (k0, v0).
-// vals_identity: values start as 0..n-1 (v0 is not read).
-void radix_sort(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, int64_t n, int bits,
-                bool vals_identity, uint32_t* hist, uint32_t* scan_tmp, hipStream_t s);
+// LSD radix sort of (keys, vals) by bits [0, bits), at most 64; true: the
+// result lies in (k1, v1), else in (k0, v0) (always so for an even number of
+// 8-bit digits).  vals_identity: values start as 0..n-1 (v0 is not read).
+// hist: radix_hist_words(n).
+bool radix_sort(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, int64_t n, int bits, bool vals_identity,
+                uint32_t* hist, hipStream_t s);
 size_t radix_hist_words(int64_t n);
 size_t scan_tmp_words(int64_t n);
 void launch_gather_sorted(const float* resc, const uint32_t* perm, int64_t n, int dim, float4* pts,
@@ -340,10 +342,10 @@ void launch_labels_out(int64_t n, const int32_t* label, const float4* pts, const
                        int32_t* out, hipStream_t s);
 void launch_cands_out(int K, int64_t n, const uint64_t* cand_key, const int32_t* inv,
                       int32_t* cand, float* cd2, hipStream_t s);
-void launch_edge_keys(const int32_t* eu, const int32_t* ev, int64_t m, uint64_t* keys,
-                      hipStream_t s);
-void launch_edges_out(const uint64_t* keys, const uint32_t* idx, const float* ed2, int64_t m,
-                      int32_t* u, int32_t* v, float* d2, hipStream_t s);
+// bits: of an id (2^bits >= the number of points)
+void launch_edge_keys(const int32_t* eu, const int32_t* ev, int64_t m, int bits, uint64_t* keys, hipStream_t s);
+void launch_edges_out(const uint64_t* keys, const uint32_t* idx, const float* ed2, int64_t m, int bits, int32_t* u,
+                      int32_t* v, float* d2, hipStream_t s);
 // Reference cellular matrix (findCell + CSR).
 // geo: int32[16] = ext_dual[3], PC[3], pc[3], R, dim (host-computed, see emst_api.hip).
 // dim = grid dimension, pstride = floats per point (3 for the 2.5D mode's 2D grid).
