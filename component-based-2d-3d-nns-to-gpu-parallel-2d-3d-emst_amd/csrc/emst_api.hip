@@ -158,9 +158,8 @@ struct emst_ctx {
     DevBuf<uint32_t> dup_m2;
     DevBuf<uint64_t> dup_bkey;
     // cycle rule of the 2.5D mode (CycleState)
-    DevBuf<int32_t> cy_j0, cy_j, cy_roots;
-    DevBuf<uint64_t> cy_kh;
-    DevBuf<uint32_t> cy_kl;
+    DevBuf<int32_t> cy_j0, cy_roots;
+    DevBuf<uint64_t> cy_st;
     DevBuf<uint8_t> cy_onc, cy_cut;
     DevBuf<unsigned long long> visit;  // arrival state of the bottom-up node passes
     DevBuf<int32_t> list2;             // queries open after pass 0 (per-round component search)
@@ -310,9 +309,7 @@ int alloc_all(emst_ctx* c)
     if (c->cdim < c->dim) {
         ENS(cy_j0, n);
         ENS(cy_roots, n);
-        ENS(cy_j, 2 * n);
-        ENS(cy_kh, 2 * n);
-        ENS(cy_kl, 2 * n);
+        ENS(cy_st, 2 * n);
         ENS(cy_onc, n);
         ENS(cy_cut, n);
     }
@@ -549,18 +546,12 @@ CycleState cycle_state(emst_ctx* c)
     const int64_t n = c->n;
     y.j0 = c->cy_j0.p;
     y.roots = c->cy_roots.p;
-    y.j[0] = c->cy_j.p;
-    y.j[1] = c->cy_j.p + n;
-    y.kh[0] = c->cy_kh.p;
-    y.kh[1] = c->cy_kh.p + n;
-    y.kl[0] = c->cy_kl.p;
-    y.kl[1] = c->cy_kl.p + n;
+    y.st[0] = c->cy_st.p;
+    y.st[1] = c->cy_st.p + n;
     y.onc = c->cy_onc.p;
     y.cut = c->cy_cut.p;
     y.inv = c->inv.p;
-    int steps = 1;
-    while (steps < 62 && ((int64_t)1 << steps) < n) ++steps;
-    y.steps = steps;
+    y.steps = cycle_steps((uint64_t)n);
     return y;
 }
 
@@ -999,7 +990,7 @@ std::vector<uintptr_t> graph_key(emst_ctx* c)
             (uintptr_t)c->open_tmp.p, (uintptr_t)c->list.p, (uintptr_t)c->nodes.p, (uintptr_t)c->dcl.p,
             (uintptr_t)c->nleaves, (uintptr_t)c->lstart.p, (uintptr_t)c->leaf_of.p, (uintptr_t)c->bucket,
             (uintptr_t)__builtin_bit_cast(uint32_t, c->seed_scale),
-            (uintptr_t)y.j[0], (uintptr_t)y.kh[0], (uintptr_t)y.kl[0], (uintptr_t)y.onc, (uintptr_t)y.cut,
+            (uintptr_t)y.st[0], (uintptr_t)y.onc, (uintptr_t)y.cut,
             (uintptr_t)c->grouped, (uintptr_t)d.npoints,
             (uintptr_t)d.ngroups, (uintptr_t)c->C, (uintptr_t)c->pts.p, (uintptr_t)c->cand_key.p,
             (uintptr_t)c->cand_pos.p, (uintptr_t)c->label.p, (uintptr_t)c->label2.p, (uintptr_t)c->corr.p,

@@ -77,6 +77,8 @@ struct Counters {
     // then needs no keep, prep, node labels or second key, and its hook takes
     // every point with a target as its singleton component's winner
     uint32_t knn_round1;
+    // listed roots whose walk was too long this round (2.5D cycle rule)
+    uint32_t walk_left;
 };
 
 // Coincident-point groups.  Points with identical rescaled coordinates form a
@@ -106,24 +108,33 @@ struct DupState {
 // chain.  Per round, over the component roots: j0 = the root that the chosen
 // edge leads to (the root itself when it has no outgoing candidate or chose
 // the same edge as that root: a mutual pair, which the hook resolves); the
-// roots with another target are listed (roots, Counters::nroots); pointer
-// doubling over the list (j, kh/kl ping-pong, S steps with 2^S > listed
-// roots, at most `steps`) gives the largest chosen edge (kh = d2 bits << 32 |
-// min id, kl = max id) on the path of 2^S hops, which for a root on a cycle
-// is the cycle's largest; onc marks the roots on cycles, cut the root whose
-// own edge is its cycle's largest: that root does not hook this round.
+// roots with another target are listed (roots, Counters::nroots); onc marks
+// the roots on cycles, cut the root whose own edge is its cycle's largest:
+// that root does not hook this round.  A walk along the choices settles each
+// root (k_cycle_walk); when one is too long, all of them are settled by
+// pointer jumping (st, two buffers: root reached << 32 | the root on the way
+// to it with the largest chosen edge; `steps` launches at most).
 // j0 == nullptr: off.
 struct CycleState {
     int32_t* roots;         // listed roots (n)
     int32_t* j0;
-    int32_t* j[2];
-    uint64_t* kh[2];
-    uint32_t* kl[2];
+    uint64_t* st[2];
     uint8_t* onc;
     uint8_t* cut;
     const int32_t* inv;     // global id -> sorted position
     int steps;
 };
+constexpr int kCyHops = 64;     // hops of one launch of the pointer jumping
+constexpr int kCyWalk = 256;    // hops of a walk, at most
+
+// launches of the pointer jumping after which any path of r listed roots has
+// ended on a cycle or at a root with no target: kCyHops^S > r
+__host__ __device__ inline int cycle_steps(uint64_t r)
+{
+    int s = 0;
+    for (uint64_t reach = 1; reach <= r; reach *= kCyHops) ++s;
+    return s;
+}
 
 // One point cloud of a context (a context holds one cloud, or a batch of
 // independent clouds of one dimension run together, packed back to back in

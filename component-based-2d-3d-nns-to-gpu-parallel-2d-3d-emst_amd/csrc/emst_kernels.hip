@@ -2458,6 +2458,7 @@ __global__ void k_round_begin(Counters* C)
     C->round += 1;
     C->edges_prev = C->edges;
     C->nroots = 0;
+    C->walk_left = 0;
     C->deferred = 0;
 }
 
@@ -4354,10 +4355,9 @@ __global__ __launch_bounds__(64) void k_knn_first(int64_t n, const float4* __res
 // so the rule starts at round 2.
 //
 // k_cycle_init: per root, its target j0 (itself when it has no outgoing
-// candidate or is in a mutual pair), both doubling buffers, onc = cut = 0;
-// the roots with another target are listed (cy.roots, C->nroots), one
+// candidate or is in a mutual pair) and cut = 0; the roots with another target are listed (cy.roots, C->nroots), one
 // block-wide reservation per chunk of kCyChunk points.
-constexpr int kCyChunk = 8192;
+constexpr int kCyChunk = 2048;                 // (8192: 315 us over those rounds, 2048: 193)
 constexpr int kCyPer = kCyChunk / kBlock;      // points per thread, one bit each
 
 __global__ __launch_bounds__(kBlock) void k_cycle_init(int64_t n, const int32_t* __restrict__ label,
@@ -4382,16 +4382,7 @@ __global__ __launch_bounds__(kBlock) void k_cycle_init(int64_t n, const int32_t*
             const int32_t o = la == (int32_t)r ? lb : la;
             if (!(comp1[o] == k1 && comp2[o] == k2)) t = o;     // else a mutual pair
         }
-        const uint64_t h = t == (int32_t)r ? 0ull : k1;
-        const uint32_t l = t == (int32_t)r ? 0u : k2;
         cy.j0[r] = t;
-        cy.j[0][r] = t;
-        cy.j[1][r] = t;
-        cy.kh[0][r] = h;
-        cy.kh[1][r] = h;
-        cy.kl[0][r] = l;
-        cy.kl[1][r] = l;
-        cy.onc[r] = 0;
         cy.cut[r] = 0;
         if (t != (int32_t)r) bits |= 1u << i;
     }
@@ -4420,38 +4411,88 @@ __global__ __launch_bounds__(kBlock) void k_cycle_init(int64_t n, const int32_t*
         if ((bits >> i) & 1u) cy.roots[at++] = (int32_t)(c0 + (int64_t)i * kBlock + threadIdx.x);
 }
 
-// number of doubling steps for R listed roots: 2^S > R covers any path of
-// listed roots, which ends on a cycle or at a root with no target
-__device__ __forceinline__ int cycle_steps(uint32_t R, int max_steps)
+// the chosen edge of root a is larger than that of root b
+__device__ __forceinline__ bool cycle_above(const uint64_t* comp1, const uint32_t* comp2, int32_t a, int32_t b)
 {
-    int S = 0;
-    while (S < max_steps && (1ull << S) <= (uint64_t)R) ++S;
-    return S;
+    const uint64_t ka = comp1[a], kb = comp1[b];
+    return ka > kb || (ka == kb && comp2[a] > comp2[b]);
 }
 
-// doubling step k (reads buffer k & 1): hop 2^k further, keep the largest
-// edge key on the way; steps past cycle_steps do nothing
-__global__ __launch_bounds__(kBlock) void k_cycle_step(CycleState cy, int k, const Counters* C)
+// A listed root is cut when its choices lead back to it past smaller edges
+// only, so each walks along them until an edge larger than its own, a root
+// with no target, itself, or a root met before (a cycle without it: the last
+// power-of-two hop is remembered).  Edges mostly shrink along the choices, so
+// walks are short: over the 12 rounds of a 3*10^6-point terrain they take
+// 171 us in all, and the launches behind them, idle, 245.  (Pointer doubling
+// alone took 22 launches a round there, 1.57 ms.)
+__global__ __launch_bounds__(kBlock) void k_cycle_walk(const uint64_t* __restrict__ comp1,
+                                                      const uint32_t* __restrict__ comp2, CycleState cy,
+                                                      Counters* C)
 {
     if (C->done || C->round <= 1u) return;
     const uint32_t R = C->nroots;
-    if (k >= cycle_steps(R, cy.steps)) return;
-    const int src = k & 1, dst = src ^ 1;
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (int64_t)R;
          t += (int64_t)gridDim.x * blockDim.x) {
         const int32_t r = cy.roots[t];
-        const int32_t j = cy.j[src][r];
-        uint64_t h = cy.kh[src][r];
-        uint32_t l = cy.kl[src][r];
-        const uint64_t h2 = cy.kh[src][j];
-        const uint32_t l2 = cy.kl[src][j];
-        if (h2 > h || (h2 == h && l2 > l)) {
-            h = h2;
-            l = l2;
+        int32_t x = cy.j0[r], met = r;
+        int hops = 0, next = 1;
+        bool cut = false, left = false;
+        for (;;) {
+            if (x == r) {
+                cut = true;
+                break;
+            }
+            if (x == met || cycle_above(comp1, comp2, x, r)) break;
+            if (++hops == kCyWalk) {
+                left = true;
+                break;
+            }
+            if (hops == next) {
+                met = x;
+                next *= 2;
+            }
+            const int32_t y = cy.j0[x];
+            if (y == x) break;
+            x = y;
         }
-        cy.j[dst][r] = cy.j[src][j];
-        cy.kh[dst][r] = h;
-        cy.kl[dst][r] = l;
+        if (cut) {
+            cy.cut[r] = 1;
+            atomicAdd(&C->cycles_cut, 1u);
+        }
+        if (left) C->walk_left = 1u;
+    }
+}
+
+// Pointer jumping over the listed roots, when a walk was too long: launch k
+// goes kCyHops hops of the last launch's states (launch 0: of the choices
+// themselves) and keeps the root on the way whose edge is largest.
+__global__ __launch_bounds__(kBlock) void k_cycle_step(const uint64_t* __restrict__ comp1,
+                                                      const uint32_t* __restrict__ comp2, CycleState cy, int k,
+                                                      const Counters* C)
+{
+    if (C->done || C->round <= 1u || !C->walk_left) return;
+    const uint32_t R = C->nroots;
+    if (k >= cycle_steps(R)) return;
+    const uint64_t* src = cy.st[k & 1];
+    uint64_t* dst = cy.st[(k & 1) ^ 1];
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (int64_t)R;
+         t += (int64_t)gridDim.x * blockDim.x) {
+        const int32_t r = cy.roots[t];
+        int32_t j = r, top = r;
+        for (int hop = 0; hop < kCyHops; ++hop) {
+            const int32_t y = cy.j0[j];
+            if (y == j) break;
+            int32_t to = y, on = j;
+            if (k > 0) {
+                const uint64_t st = src[j];
+                to = (int32_t)(st >> 32);
+                on = (int32_t)(uint32_t)st;
+            }
+            if (on != top && cycle_above(comp1, comp2, on, top)) top = on;
+            j = to;
+        }
+        dst[r] = (uint64_t)(uint32_t)j << 32 | (uint32_t)top;
+        if (k == 0) cy.onc[r] = 0;
     }
 }
 
@@ -4459,27 +4500,26 @@ __global__ __launch_bounds__(kBlock) void k_cycle_step(CycleState cy, int k, con
 // root with no target), and every root of a cycle is such a target
 __global__ __launch_bounds__(kBlock) void k_cycle_mark(CycleState cy, const Counters* C)
 {
-    if (C->done || C->round <= 1u) return;
+    if (C->done || C->round <= 1u || !C->walk_left) return;
     const uint32_t R = C->nroots;
-    const int fin = cycle_steps(R, cy.steps) & 1;
+    const uint64_t* fin = cy.st[cycle_steps(R) & 1];
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (int64_t)R;
          t += (int64_t)gridDim.x * blockDim.x)
-        cy.onc[cy.j[fin][cy.roots[t]]] = 1;
+        cy.onc[fin[cy.roots[t]] >> 32] = 1;
 }
 
-__global__ __launch_bounds__(kBlock) void k_cycle_cut(const uint64_t* __restrict__ comp1,
-                                                     const uint32_t* __restrict__ comp2, CycleState cy,
-                                                     Counters* C)
+// (those that their walk has cut are cut here again, and not counted twice)
+__global__ __launch_bounds__(kBlock) void k_cycle_cut(CycleState cy, Counters* C)
 {
-    if (C->done || C->round <= 1u) return;
+    if (C->done || C->round <= 1u || !C->walk_left) return;
     const uint32_t R = C->nroots;
-    const int fin = cycle_steps(R, cy.steps) & 1;
+    const uint64_t* fin = cy.st[cycle_steps(R) & 1];
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (int64_t)R;
          t += (int64_t)gridDim.x * blockDim.x) {
         const int32_t r = cy.roots[t];
-        const bool cut = cy.onc[r] && comp1[r] == cy.kh[fin][r] && comp2[r] == cy.kl[fin][r];
-        cy.cut[r] = cut ? 1 : 0;
-        if (cut) atomicAdd(&C->cycles_cut, 1u);
+        if (!cy.onc[r] || (int32_t)(uint32_t)fin[r] != r || cy.cut[r]) continue;
+        cy.cut[r] = 1;
+        atomicAdd(&C->cycles_cut, 1u);
     }
 }
 
@@ -5050,10 +5090,13 @@ void launch_round_phase(int phase, int K, int64_t n, const uint32_t* ids, const 
             const unsigned gc = (unsigned)std::min<int64_t>(g, 1024);
             hipLaunchKernelGGL(k_cycle_init, dim3((unsigned)((n + kCyChunk - 1) / kCyChunk)), dim3(kBlock), 0, s, n,
                                label, comp1, comp2, cy, C);
-            for (int k = 0; k < cy.steps; ++k)
-                hipLaunchKernelGGL(k_cycle_step, dim3(gc), dim3(kBlock), 0, s, cy, k, C);
-            hipLaunchKernelGGL(k_cycle_mark, dim3(gc), dim3(kBlock), 0, s, cy, C);
-            hipLaunchKernelGGL(k_cycle_cut, dim3(gc), dim3(kBlock), 0, s, comp1, comp2, cy, C);
+            hipLaunchKernelGGL(k_cycle_walk, dim3(gc), dim3(kBlock), 0, s, comp1, comp2, cy, C);
+            if (n > kCyWalk) {
+                for (int k = 0; k < cy.steps; ++k)
+                    hipLaunchKernelGGL(k_cycle_step, dim3(gc), dim3(kBlock), 0, s, comp1, comp2, cy, k, C);
+                hipLaunchKernelGGL(k_cycle_mark, dim3(gc), dim3(kBlock), 0, s, cy, C);
+                hipLaunchKernelGGL(k_cycle_cut, dim3(gc), dim3(kBlock), 0, s, cy, C);
+            }
         }
         hipLaunchKernelGGL(k_round_hook, dim3(nblocks(n, kHookBlock)), dim3(kHookBlock), 0, s, n, ids, label,
                            label2, corr, corr_key, comp1, comp2, C, eu, ev, ed2, eround, cy.j0 ? cy.cut : nullptr);
