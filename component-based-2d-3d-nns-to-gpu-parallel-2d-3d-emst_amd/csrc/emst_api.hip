@@ -149,6 +149,11 @@ struct emst_ctx {
     DevBuf<uint8_t> cursor;            // per-point scan position in its ranked candidates
     DevBuf<uint64_t> open_mask;        // split cone search (SplitScratch)
     DevBuf<uint32_t> open_cnt, open_tmp;
+    DevBuf<int32_t> reach;              // late cones (k_late_mark)
+    bool late = false;                  // points may hold late cones
+    bool no_late = false;               // a choice of theirs failed its check: exact cones
+    bool late_tree = false;             // this build's nodes hold their smallest ids
+    const float* seed_r = nullptr;      // the build's learned seeds
     DevBuf<Params> params;
     DevBuf<double> cloud_w;
     DevBuf<int32_t> cloud_e, cloud_r;
@@ -640,7 +645,106 @@ NbrList nbr_list(emst_ctx* c)
     return NbrList{c->knn_pos.p, c->knn_key.p, c->knn_cur.p};
 }
 
-int build(emst_ctx* c)
+// First radius of a search that may leave cones late (k_late_mark), as a
+// multiple of the plain seed and of a model's (which aims at every cone), and
+// the fewest points of one.  (Factors, ms per run of 10^6 uniform / 4*10^6
+// clustered points: 0.7 2.27 / 11.7, 0.5 2.10 / 10.1, 0.4 2.09 / 9.9, 0.3 5.4 /
+// 17.5, where a twentieth of the points sees no other; with a model 0.5 12.7,
+// 0.35 11.3.  Fewer points, exact cones first / late: uniform 4000 0.61 /
+// 0.59, 2048 0.52 / 0.51, clustered 4000 0.86 / 0.81, 2048 0.60 / 0.68.)
+constexpr float kLateSeed = 0.5f, kLateLearned = 0.35f;
+constexpr int64_t kLateMin = 1 << 12;
+
+ConeRest cone_rest(emst_ctx* c)
+{
+    ConeRest a{};
+    a.pts = c->pts.p;
+    a.nodes = c->nodes.p;
+    a.clouds = c->dcl.p;
+    a.ncl = c->ncl;
+    a.bucket = c->bucket;
+    a.lt = leaf_table(c);
+    a.n = c->n;
+    a.list = c->list.p;
+    a.inv = c->inv.p;
+    a.cand_key = c->cand_key.p;
+    a.cand_pos = c->cand_pos.p;
+    a.reach = c->reach.p;
+    a.ids = c->ids.p;
+    a.label = c->label.p;
+    a.corr = c->corr.p;
+    a.corr_key = c->corr_key.p;
+    a.comp1 = c->comp1.p;
+    a.rkey = c->rkey.p;
+    a.rpos = c->rpos.p;
+    a.cursor = c->cursor.p;
+    a.C = c->C;
+    return a;
+}
+
+// The cone search over every point.  first: writes round 1's targets.
+int search_cones(emst_ctx* c, bool first)
+{
+    const int64_t n = c->n;
+    hipStream_t s = c->stream;
+    // Full-dimensional cones over many points: pass 0 over all queries by
+    // k_cone_first, the open ones then resumed from a compacted list (resumed
+    // in place they were 4-20% slower).  Fewer points run every pass in one
+    // launch: the search then takes as long as its longest packet, and two
+    // launches have two of those.  One launch against two, ms (seed 3.5): 3D
+    // uniform 1.37 / 0.98 at 2*10^5 points and 2.22 / 1.55 at 4*10^5,
+    // clustered 2.95 / 3.57 and 3.84 / 3.58; 2D uniform 0.33 / 0.37 and
+    // 0.48 / 0.42, clustered 0.67 / 0.80 and 0.85 / 0.89.
+    SplitScratch split{};
+    split.open_mask = c->open_mask.p;
+    split.cnt = c->open_cnt.p;
+    split.off = c->open_cnt.p + ((n + 63) / 64 + 1);
+    split.tmp = c->open_tmp.p;
+    split.list = c->list.p;     // free until the rounds' research queue
+    const int mode = c->opt.search_split;
+    split.compact_frac = mode == 2 ? -1.0 : 1.0;
+    const bool many = c->cdim == c->dim && n >= ((int64_t)1 << (c->dim == 3 ? 18 : 19));
+    const bool use_split = c->late || mode == 2 || mode == 3 || (mode == 0 && many);
+    launch_cone_search(c->dim, c->cdim, c->pts.p, c->nodes.p, c->dcl.p, c->ncl, c->bucket, leaf_table(c), n, nullptr,
+                       n, c->label.p, false, c->inv.p, c->seed_r, c->seed_scale,
+                       !c->late ? 1.f : c->seed_r ? kLateLearned : kLateSeed, c->cand_key.p, c->cand_pos.p, nullptr,
+                       first ? c->corr.p : nullptr, first ? c->corr_key.p : nullptr, c->C, true, dup_state(c),
+                       use_split ? &split : nullptr, c->late ? c->reach.p : nullptr, s);
+    LAUNCHCHK(c);
+    HIPCHK(c, hipEventRecord(c->ev[2], s));
+    // read with the counters (into the context, which outlives any early
+    // return while the copy is queued)
+    c->resumed_h = 0;
+    if (use_split && !c->late && n > 0)
+        HIPCHK(c, hipMemcpyAsync(&c->resumed_h, split.off + (n + 63) / 64, sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                 s));
+    return EMST_OK;
+}
+
+// Every cone exact, for callers that read them, count their search or repeat
+// it: the search again from full seeds (going on from the late points' small
+// radius instead tests twice as many nodes).
+int complete_cones(emst_ctx* c)
+{
+    if (!c->late) return EMST_OK;
+    hipStream_t s = c->stream;
+    c->late = false;
+    launch_zero_u32(reinterpret_cast<uint32_t*>(c->C->work[kWorkConePackets]),
+                    2 * (int64_t)(kWorkKinds - kWorkConePackets) * kWorkSlots, s);
+    int rc = search_cones(c, false);
+    if (rc) return rc;
+    launch_rank_cones(c->cdim, c->n, c->cand_key.p, c->cand_pos.p, nullptr, c->n, c->rkey.p, c->rpos.p, c->cursor.p,
+                      nullptr, nullptr, s);
+    launch_revive(c->n, c->corr.p, s);
+    LAUNCHCHK(c);
+    Counters h{};
+    if ((rc = read_counters(c, &h))) return rc;
+    for (int k = 0; k < 5; ++k) c->stats[k] = work_total(h, kWorkConePackets + k);
+    c->stats[8] = c->resumed_h;
+    return EMST_OK;
+}
+
+int build(emst_ctx* c, bool all_cones)
 {
     const int64_t n = c->n;
     hipStream_t s = c->stream;
@@ -669,6 +773,8 @@ int build(emst_ctx* c)
     c->groups_settled = false;
     c->knn_built = false;
     c->dup_points = c->dup_groups = 0;
+    bool any_dup = c->no_grouping;
+    c->late = false;
     const bool comp = c->opt.round_search == 1;
     if (!c->no_grouping && !comp) {
         launch_dup_groups(c->keys0.p, c->pts.p, n, c->dup_rep.p, c->dup_runs.p, c->dup_list.p,
@@ -677,6 +783,7 @@ int build(emst_ctx* c)
         Counters h{};
         int rc0 = read_counters(c, &h);
         if (rc0) return rc0;
+        any_dup = h.dup_points > 0 || h.dup_overflow != 0;
         if (h.grouped) {
             const int K2 = c->K / 2;
             if ((rc0 = ensure(c, c->dup_m2, h.dup_groups)) ||
@@ -733,7 +840,7 @@ int build(emst_ctx* c)
         c->trace.clear();
         return EMST_OK;
     }
-    const float* seed_r = nullptr;
+    c->seed_r = nullptr;
     if (c->learned && c->ncl == 1 && c->cdim == c->dim) {
         int rc2;
         if ((rc2 = ensure(c, c->feat, (size_t)n * 8)) || (rc2 = ensure(c, c->pred, (size_t)n)) ||
@@ -741,43 +848,28 @@ int build(emst_ctx* c)
             return rc2;
         launch_radius_features(c->dim, c->pts.p, c->nodes.p, c->L, leaf_table(c), n, c->feat.p, c->ls.p, s);
         launch_radius_seed(n, c->model.p, c->feat.p, c->ls.p, c->pred.p, c->seed.p, s);
-        seed_r = c->seed.p;
+        c->seed_r = c->seed.p;
     }
     LAUNCHCHK(c);
     HIPCHK(c, hipEventRecord(c->ev[1], s));
-    // Full-dimensional cones over many points: pass 0 over all queries by
-    // k_cone_first, the open ones then resumed from a compacted list (resumed
-    // in place they were 4-20% slower).  Fewer points run every pass in one
-    // launch: the search then takes as long as its longest packet, and two
-    // launches have two of those.  One launch against two, ms (seed 3.5): 3D
-    // uniform 1.37 / 0.98 at 2*10^5 points and 2.22 / 1.55 at 4*10^5,
-    // clustered 2.95 / 3.57 and 3.84 / 3.58; 2D uniform 0.33 / 0.37 and
-    // 0.48 / 0.42, clustered 0.67 / 0.80 and 0.85 / 0.89.
-    SplitScratch split{};
-    split.open_mask = c->open_mask.p;
-    split.cnt = c->open_cnt.p;
-    split.off = c->open_cnt.p + ((n + 63) / 64 + 1);
-    split.tmp = c->open_tmp.p;
-    split.list = c->list.p;     // free until the rounds' research queue
-    const int mode = c->opt.search_split;
-    split.compact_frac = mode == 2 ? -1.0 : 1.0;
-    const bool many = c->cdim == c->dim && n >= ((int64_t)1 << (c->dim == 3 ? 18 : 19));
-    const bool use_split = mode == 2 || mode == 3 || (mode == 0 && many);
-    launch_cone_search(c->dim, c->cdim, c->pts.p, c->nodes.p, c->dcl.p, c->ncl, c->bucket, leaf_table(c), n, nullptr, n,
-                       c->label.p, false, c->inv.p, seed_r, c->seed_scale, c->cand_key.p, c->cand_pos.p, nullptr, c->corr.p,
-                       c->corr_key.p, c->C, true, dup, use_split ? &split : nullptr, s);
-    LAUNCHCHK(c);
-    HIPCHK(c, hipEventRecord(c->ev[2], s));
-    // read with the counters below (into the context, which outlives any
-    // early return while the copy is queued)
-    c->resumed_h = 0;
-    if (use_split && n > 0)
-        HIPCHK(c, hipMemcpyAsync(&c->resumed_h, split.off + (n + 63) / 64, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                 s));
+    // Late cones (k_late_mark) in 3D, where most of the search's time goes to
+    // cones that no round asks for: not where points coincide (their groups
+    // share cones), and 2D cones cost less than the rounds that ask for them
+    // (10^6 uniform points 1.85 ms a run without, 1.80 with, 3*10^5 clustered
+    // ones 1.37 and 2.8).  3D, without / with, ms a run: uniform 10^4 0.69 /
+    // 0.58, 2*10^5 2.10 / 1.03, 10^6 4.3 / 2.1; clustered 10^4 1.22 / 1.06,
+    // 5*10^4 2.03 / 1.96, 2*10^5 3.6 / 2.2, 10^6 6.7 / 4.8, 4*10^6 16.7 /
+    // 10.1, with a seed model 17.6 / 11.3.
+    c->late = !all_cones && !c->no_late && c->opt.search_split == 0 && c->ncl == 1 && c->cdim == 3 && n >= kLateMin &&
+              !any_dup;
+    c->late_tree = false;
+    int rc4;
+    if (c->late && (rc4 = ensure(c, c->reach, (size_t)n))) return rc4;
+    if ((rc4 = search_cones(c, true))) return rc4;
     launch_dup_fill(c->cdim, n, c->label.p, c->pts.p, c->inv.p, c->cand_key.p, c->cand_pos.p, nullptr, c->corr.p,
                     c->corr_key.p, c->C, dup, s);
     launch_rank_cones(c->cdim, n, c->cand_key.p, c->cand_pos.p, nullptr, n, c->rkey.p, c->rpos.p, c->cursor.p,
-                      nullptr, s);
+                      c->late ? c->reach.p : nullptr, nullptr, s);
     LAUNCHCHK(c);
     // while grouping is on only group points can hold a zero-distance or no
     // candidate, and k_dup_fill refreshes those; the queue serves the
@@ -785,7 +877,7 @@ int build(emst_ctx* c)
     // (a point's smallest cone key, which the search leaves as round 1's, is at
     // distance zero or empty exactly when some cone is: one key a point is
     // read instead of K, 0.16 -> 0.01 ms at 4*10^6 3D points)
-    if (!c->grouped) launch_flag_research(1, n, c->corr_key.p, c->list.p, c->C, s);
+    if (!c->grouped) launch_flag_research(1, n, c->corr_key.p, c->list.p, c->late ? c->reach.p : nullptr, c->C, s);
     LAUNCHCHK(c);
     HIPCHK(c, hipEventRecord(c->ev[3], s));
     Counters h{};
@@ -795,7 +887,7 @@ int build(emst_ctx* c)
         // distinct points at float distance 0: the groups would merge
         // candidates that the per-point rule keeps apart; search ungrouped
         c->no_grouping = true;
-        return build(c);
+        return build(c, all_cones);
     }
     c->zero_or_empty = h.zero_or_empty;
     for (int k = 0; k < 5; ++k) c->stats[k] = work_total(h, kWorkConePackets + k);
@@ -811,6 +903,8 @@ int build(emst_ctx* c)
     c->edges = 0;
     c->finished = c->target_edges == 0;
     c->trace.clear();
+    // repeated searches start from exact cones
+    if (c->zero_or_empty > 0) return complete_cones(c);
     return EMST_OK;
 }
 
@@ -838,11 +932,11 @@ constexpr int kOneLaunchRounds = 16;
 // The kernels of one Boruvka round (SolutionEMST::activate).  Round control
 // lives on the device (k_round_begin / k_round_end), so a round issued after
 // the run has finished does nothing.  trace: events after each phase.
-void issue_round(emst_ctx* c, bool tr, unsigned long long* stamps = nullptr)
+void issue_round(emst_ctx* c, bool tr, unsigned long long* stamps = nullptr, bool begin = true)
 {
     hipStream_t s = c->stream;
-    launch_round_begin(c->C, s);
-    if (tr) (void)hipEventRecord(c->ev[3], s);
+    if (begin) launch_round_begin(c->C, s);
+    if (begin && tr) (void)hipEventRecord(c->ev[3], s);
     // group points: zero-distance '+' cones while the group spans several
     // components, the representative's own cones once it is one (the
     // repeated search of NodeEMST.h:1051-1077, without searching again); the
@@ -852,7 +946,7 @@ void issue_round(emst_ctx* c, bool tr, unsigned long long* stamps = nullptr)
         launch_dup_fill(c->cdim, c->n, c->label.p, c->pts.p, c->inv.p, c->cand_key.p, c->cand_pos.p, c->corr.p,
                         nullptr, nullptr, c->C, d, s);
         launch_rank_cones(c->cdim, c->n, c->cand_key.p, c->cand_pos.p, d.list, d.npoints, c->rkey.p, c->rpos.p,
-                          c->cursor.p, c->C, s);
+                          c->cursor.p, nullptr, c->C, s);
     }
     const CycleState cy = cycle_state(c);
     for (int ph = 0; ph < 4; ++ph) {
@@ -868,6 +962,7 @@ void issue_round(emst_ctx* c, bool tr, unsigned long long* stamps = nullptr)
                            c->label.p, c->label2.p,
                            c->corr.p, c->corr_key.p, c->comp1.p, c->comp2.p, c->C, c->eu.p,
                            c->ev_.p, c->ed2.p, c->eround.p, cy, s);
+        if (ph == 0 && c->late) launch_late_cones(cone_rest(c), s);
         if (tr) (void)hipEventRecord(c->ev[4 + ph], s);
     }
     launch_round_end(c->C, c->grouped, s, stamps, kOneLaunchRounds);
@@ -895,12 +990,40 @@ int resume_flatten(emst_ctx* c, Counters* h)
     return read_counters(c, h);
 }
 
+// A round paused by its late points (done == 3): their search, then the rest
+// of the round.
+int resume_late(emst_ctx* c, Counters* h)
+{
+    hipStream_t s = c->stream;
+    int rc;
+    if ((rc = ensure(c, c->list2, (size_t)c->n)) || (rc = ensure(c, c->defer, (size_t)c->n)) ||
+        (rc = ensure(c, c->visit, 2 * (size_t)c->nleaves)))
+        return rc;
+    launch_late_search(cone_rest(c), c->nodes.p, c->visit.p, c->nleaves, !c->late_tree,
+                       kCompSeedScale3D, split_scratch(c), s);
+    c->late_tree = true;
+    const bool tr = c->opt.trace != 0;
+    if (tr) HIPCHK(c, hipEventRecord(c->ev[4], s));
+    const CycleState cy = cycle_state(c);
+    for (int ph = 1; ph < 4; ++ph) {
+        launch_round_phase(ph, c->K, c->n, c->ids.p, c->rkey.p, c->rpos.p, c->cursor.p, c->label.p, c->label2.p,
+                           c->corr.p, c->corr_key.p, c->comp1.p, c->comp2.p, c->C, c->eu.p, c->ev_.p, c->ed2.p,
+                           c->eround.p, cy, s);
+        if (tr) HIPCHK(c, hipEventRecord(c->ev[4 + ph], s));
+    }
+    launch_round_end(c->C, c->grouped, s);
+    LAUNCHCHK(c);
+    if ((rc = read_counters(c, h))) return rc;
+    if (h->done == 2u) rc = resume_flatten(c, h);
+    return rc;
+}
+
 void absorb_counters(emst_ctx* c, const Counters& h)
 {
     c->edges = h.edges;
     c->rounds = (int)h.round;
     c->stats[7] = (int64_t)h.cycles_cut;
-    c->stats[9] = (int64_t)h.comp_queries;
+    c->stats[9] = c->opt.round_search == 1 ? (int64_t)h.comp_queries : 0;
     for (int k = 0; k < kWorkCompKinds; ++k) c->stats[10 + k] = work_total(h, k);
     if (h.done == 1u) c->finished = true;
 }
@@ -924,17 +1047,18 @@ int round_once(emst_ctx* c, int32_t* finished)
     } else if (c->rounds > 0 && c->zero_or_empty > 0) {
         // research and zero_or_empty restart for this round
         HIPCHK(c, hipMemsetAsync(&c->C->research, 0, 2 * sizeof(uint32_t), s));
-        launch_flag_research(c->K, n, c->cand_key.p, c->list.p, c->C, s);
+        launch_flag_research(c->K, n, c->cand_key.p, c->list.p, nullptr, c->C, s);
         LAUNCHCHK(c);
         Counters h{};
         int rc = read_counters(c, &h);
         if (rc) return rc;
         if (h.research > 0) {
             launch_cone_search(c->dim, c->cdim, c->pts.p, c->nodes.p, c->dcl.p, c->ncl, c->bucket, leaf_table(c), n, c->list.p,
-                               h.research, c->label.p, true, c->inv.p, nullptr, c->seed_scale, c->cand_key.p,
-                               c->cand_pos.p, c->corr.p, nullptr, nullptr, c->C, false, DupState{}, nullptr, s);
+                               h.research, c->label.p, true, c->inv.p, nullptr, c->seed_scale, 1.f, c->cand_key.p,
+                               c->cand_pos.p, c->corr.p, nullptr, nullptr, c->C, false, DupState{}, nullptr, nullptr,
+                               s);
             launch_rank_cones(c->cdim, n, c->cand_key.p, c->cand_pos.p, c->list.p, h.research, c->rkey.p, c->rpos.p,
-                              c->cursor.p, nullptr, s);
+                              c->cursor.p, nullptr, nullptr, s);
         }
         LAUNCHCHK(c);
         searched = h.zero_or_empty;
@@ -948,9 +1072,19 @@ int round_once(emst_ctx* c, int32_t* finished)
     if (tr && c->opt.round_search == 1 && n > 0)
         c->comp_search_ms += elapsed(c->ev[8], c->ev[9]) + elapsed(c->ev[10], c->ev[11]);
     if (h.done == 2u && (rc = resume_flatten(c, &h))) return rc;
+    if (h.done == 3u && (rc = resume_late(c, &h))) return rc;
+    if (h.done == 4u) {
+        // the rounds so far again, with exact cones, and this one
+        const int before = c->rounds;
+        c->no_late = true;
+        if ((rc = build(c, true))) return rc;
+        for (int k = 0; k <= before && rc == EMST_OK; ++k) rc = round_once(c, finished);
+        return rc;
+    }
     absorb_counters(c, h);
     // the component search: queries of this round's two dispatches
     if (c->opt.round_search == 1) searched = c->stats[9] - queries_before;
+    else if (c->late && c->rounds > 1) searched = h.late;
     c->groups_settled = h.dup_settled != 0u;
     if (tr) {
         emst_round_trace row{};
@@ -990,6 +1124,7 @@ std::vector<uintptr_t> graph_key(emst_ctx* c)
             (uintptr_t)c->open_tmp.p, (uintptr_t)c->list.p, (uintptr_t)c->nodes.p, (uintptr_t)c->dcl.p,
             (uintptr_t)c->nleaves, (uintptr_t)c->lstart.p, (uintptr_t)c->leaf_of.p, (uintptr_t)c->bucket,
             (uintptr_t)__builtin_bit_cast(uint32_t, c->seed_scale),
+            (uintptr_t)c->late, (uintptr_t)c->reach.p,
             (uintptr_t)y.st[0], (uintptr_t)y.onc, (uintptr_t)y.cut,
             (uintptr_t)c->grouped, (uintptr_t)d.npoints,
             (uintptr_t)d.ngroups, (uintptr_t)c->C, (uintptr_t)c->pts.p, (uintptr_t)c->cand_key.p,
@@ -998,6 +1133,17 @@ std::vector<uintptr_t> graph_key(emst_ctx* c)
             (uintptr_t)c->eu.p, (uintptr_t)c->ev_.p, (uintptr_t)c->ed2.p, (uintptr_t)c->eround.p,
             (uintptr_t)c->inv.p, (uintptr_t)c->rkey.p, (uintptr_t)c->rpos.p, (uintptr_t)c->cursor.p, (uintptr_t)d.rep, (uintptr_t)d.list, (uintptr_t)d.gslot, (uintptr_t)d.m2,
             (uintptr_t)d.bkey, (uintptr_t)d.bpos, (uintptr_t)c->ids.p, (uintptr_t)c->alloc_gen};
+}
+
+int run_rounds(emst_ctx* c);
+
+// a chosen edge failed its check (launch_late_search): the run again, with
+// exact cones
+int restart_exact(emst_ctx* c)
+{
+    c->no_late = true;
+    const int rc = build(c, true);
+    return rc ? rc : run_rounds(c);
 }
 
 int run_graph(emst_ctx* c)
@@ -1021,12 +1167,25 @@ int run_graph(emst_ctx* c)
         }
         c->graph_key = key;
     }
+    // a round paused by late points idles the rest of its replay, and the
+    // next ones mostly pause too: one round at a time from there
+    bool paused = false;
     while (!c->finished) {
-        HIPCHK(c, hipGraphLaunch(c->graph, s));
+        if (paused) {
+            issue_round(c, false);
+            LAUNCHCHK(c);
+        } else {
+            HIPCHK(c, hipGraphLaunch(c->graph, s));
+        }
         Counters h{};
         int rc = read_counters(c, &h);
         if (rc) return rc;
         if (h.done == 2u && (rc = resume_flatten(c, &h))) return rc;
+        if (h.done == 3u) {
+            paused = true;
+            if ((rc = resume_late(c, &h))) return rc;
+        }
+        if (h.done == 4u) return restart_exact(c);
         absorb_counters(c, h);
         c->groups_settled = h.dup_settled != 0u;
     }
@@ -1114,7 +1273,7 @@ int run_one_launch(emst_ctx* c)
     if (rc) return rc;
     c->grouped = false;
     c->groups_settled = false;
-    c->no_grouping = false;
+    c->no_grouping = c->no_late = false;
     c->knn_built = true;
     c->dup_points = c->dup_groups = 0;
     std::vector<uintptr_t> key = graph_key(c);
@@ -1165,7 +1324,7 @@ int run_one_launch(emst_ctx* c)
             }
         // more leaves than slots: the eager build lays the hierarchy out exactly
         c->built = false;
-        if ((rc = build(c))) return rc;
+        if ((rc = build(c, false))) return rc;
         return run_rounds(c);
     }
     c->zero_or_empty = 0;
@@ -1265,12 +1424,13 @@ int need_points(emst_ctx* c)
     return EMST_OK;
 }
 
-int ensure_built(emst_ctx* c)
+// cones: the caller reads the cone candidates, all of them exact
+int ensure_built(emst_ctx* c, bool cones = false)
 {
     int rc = need_points(c);
     if (rc) return rc;
-    if (!c->built) return build(c);
-    return EMST_OK;
+    if (!c->built) return build(c, cones);
+    return cones ? complete_cones(c) : EMST_OK;
 }
 
 // The rounds of a built context, to the end; times[2] = their device time.
@@ -1432,7 +1592,7 @@ int emst_set_clouds(emst_ctx* c, int32_t ncl, const int64_t* npts, const float* 
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->have_points = true;
     c->built = false;
-    c->no_grouping = false;
+    c->no_grouping = c->no_late = false;
     c->finished = false;
     c->rounds = 0;
     c->edges = 0;
@@ -1457,18 +1617,26 @@ int emst_autotune(emst_ctx* c, int32_t* best_bucket, float* best_scale, float* b
     // the cone search's leaf size, seed and form are tuned on the cone form
     const int rs0 = c->opt.round_search;
     c->opt.round_search = 0;
-    float best = 0.f;
+    // each choice by its whole run: with late cones the build's search is a
+    // part of the search
+    auto whole = [&](float* build_ms) {
+        c->no_grouping = c->no_late = false;
+        int r = build(c, false);
+        *build_ms = c->times[0] + c->times[1];
+        return r ? r : run_rounds(c);
+    };
+    float best = 0.f, bms = 0.f, ms = 0.f;
     int bb = 64;
     float bs = c->seed_scale;
     for (int b : {16, 32, 64})
         for (float sc : {2.f, 3.f, 4.f}) {
             if ((rc = layout_clouds(c, b))) break;
             c->seed_scale = sc;
-            c->no_grouping = false;
-            if ((rc = build(c))) break;
-            const float t = c->times[0] + c->times[1];
+            if ((rc = whole(&ms))) break;
+            const float t = c->times[0] + c->times[1] + c->times[2];
             if (best == 0.f || t < best) {
                 best = t;
+                bms = ms;
                 bb = b;
                 bs = sc;
             }
@@ -1482,11 +1650,11 @@ int emst_autotune(emst_ctx* c, int32_t* best_bucket, float* best_scale, float* b
         c->seed_scale = bs;
         for (int sp : {1, 2, 3}) {
             c->opt.search_split = sp;
-            c->no_grouping = false;
-            if ((rc = build(c))) break;
-            const float t = c->times[0] + c->times[1];
+            if ((rc = whole(&ms))) break;
+            const float t = c->times[0] + c->times[1] + c->times[2];
             if (t < best) {
                 best = t;
+                bms = ms;
                 bsplit = sp;
             }
         }
@@ -1506,8 +1674,8 @@ int emst_autotune(emst_ctx* c, int32_t* best_bucket, float* best_scale, float* b
             c->seed_scale = rs == 1 && c->dim == 3 ? kCompSeedScale3D : bs;
             // the component search at its own leaf size, 64 points
             const int bk = rs == 1 ? 64 : bb;
-            c->no_grouping = false;
-            if ((rc = layout_clouds(c, bk)) || (rc = build(c)) || (rc = run_rounds(c))) break;
+            c->no_grouping = c->no_late = false;
+            if ((rc = layout_clouds(c, bk)) || (rc = build(c, false)) || (rc = run_rounds(c))) break;
             const float t = c->times[0] + c->times[1] + c->times[2];
             if (tbest == 0.f || t < tbest) {
                 tbest = t;
@@ -1532,7 +1700,7 @@ int emst_autotune(emst_ctx* c, int32_t* best_bucket, float* best_scale, float* b
     c->trace.clear();
     if (best_bucket) *best_bucket = bb;
     if (best_scale) *best_scale = bs;
-    if (best_ms) *best_ms = best;
+    if (best_ms) *best_ms = bms;
     return EMST_OK;
 }
 
@@ -1691,7 +1859,7 @@ int emst_get_trace(emst_ctx* c, emst_round_trace* rows, int32_t* nrows)
 
 int emst_get_candidates(emst_ctx* c, int32_t* cand, float* cd2, int32_t* k)
 {
-    int rc = ensure_built(c);
+    int rc = ensure_built(c, true);
     if (rc) return rc;
     if (c->opt.round_search == 1) return fail(c, EMST_E_STATE, "the per-round component search keeps no cone candidates");
     if (k) *k = c->K;
@@ -1843,7 +2011,7 @@ int emst_set_radius_model(emst_ctx* c, const float* model)
 int emst_get_radius_samples(emst_ctx* c, float* feat, float* target, int64_t* m)
 {
     if (!m) return fail(c, EMST_E_ARG, "m must not be NULL");
-    int rc = ensure_built(c);
+    int rc = ensure_built(c, true);
     if (rc) return rc;
     if (c->ncl != 1) return fail(c, EMST_E_STATE, "radius samples come from a single-cloud context");
     if (c->cdim != c->dim) return fail(c, EMST_E_STATE, "radius samples come from full-dimensional cones");
@@ -1878,6 +2046,11 @@ int emst_get_radius_samples(emst_ctx* c, float* feat, float* target, int64_t* m)
 int emst_get_search_stats(emst_ctx* c, int64_t* stats, int32_t* n_stats)
 {
     if (!c || !stats || !n_stats) return EMST_E_ARG;
+    if (c->built && c->late) {
+        HIPCHK(c, hipSetDevice(c->opt.device));
+        const int rc = complete_cones(c);
+        if (rc) return rc;
+    }
     const int32_t k = std::min<int32_t>(*n_stats, 18);
     for (int i = 0; i < k; ++i) stats[i] = c->stats[i];
     *n_stats = k;

@@ -49,7 +49,8 @@ struct Counters {
     // round control, on the device so that rounds can run back to back
     // (captured in a graph) and stop by themselves
     uint32_t round;         // rounds run so far
-    uint32_t done;          // 0 running, 1 finished, 2 paused: flatten needs another launch
+    uint32_t done;          // 0 running, 1 finished, 2 paused: flatten needs another launch, 3 paused: late
+                            // points need a search, 4 stopped: the run needs exact cones
     uint32_t edges_prev;    // edges before the current round
     uint32_t target;        // sum over clouds of (points - 1)
     uint32_t max_rounds;
@@ -79,6 +80,9 @@ struct Counters {
     uint32_t knn_round1;
     // listed roots whose walk was too long this round (2.5D cycle rule)
     uint32_t walk_left;
+    // late cones (k_late_mark): points listed this round
+    uint32_t late;
+    uint32_t late_checks;   // targets to check (k_late_settle)
 };
 
 // Coincident-point groups.  Points with identical rescaled coordinates form a
@@ -238,10 +242,39 @@ struct SplitScratch {
 // over every pass) applies to full searches (qlist == nullptr).
 void launch_cone_search(int dim, int cdim, const float4* pts, const Node* nodes, const Cloud* cl, int ncl, int bucket,
                         LeafTable lt, int64_t n, const int32_t* qlist, int64_t nq, const int32_t* label,
-                        bool check_labels, const int32_t* inv, const float* seed_r, float seed_scale,
+                        bool check_labels, const int32_t* inv, const float* seed_r, float seed_scale, float seed_mul,
                         uint64_t* cand_key, int32_t* cand_pos, int32_t* revive, int32_t* first_corr,
                         uint64_t* first_key, Counters* C, bool collect_stats, DupState dup,
-                        const SplitScratch* split, hipStream_t s);
+                        const SplitScratch* split, int32_t* reach, hipStream_t s);
+// Late cones (k_late_mark; 3D, one cloud): the cloud, the points listed, their
+// cones and the rounds' arrays.
+struct ConeRest {
+    const float4* pts;
+    const Node* nodes;
+    const Cloud* clouds;
+    int ncl, bucket;
+    LeafTable lt;
+    int64_t n;
+    int32_t* list;
+    const int32_t* inv;
+    uint64_t* cand_key;
+    int32_t* cand_pos;
+    int32_t* reach;
+    const uint32_t* ids;
+    const int32_t* label;
+    int32_t* corr;
+    uint64_t* corr_key;
+    uint64_t* comp1;
+    uint64_t* rkey;
+    int32_t* rpos;
+    uint8_t* cursor;
+    Counters* C;
+};
+enum { kRestRound, kRestCheck };        // k_cone_rest: a point's cones, or the check of its target
+void launch_late_cones(const ConeRest& a, hipStream_t s);
+void launch_late_search(const ConeRest& a, Node* nodes, unsigned long long* visit, int64_t nleaves, bool first,
+                        float seed_scale, const SplitScratch& sc, hipStream_t s);
+void launch_revive(int64_t n, int32_t* corr, hipStream_t s);
 // Phase 0 of a round of the per-round component search (the alternative to
 // the round-1 cone search): node component labels (into Node::pad[1]; visit:
 // the arrival words of launch_node_min_ids), kept targets, and a search for
@@ -324,7 +357,7 @@ void launch_round_init(int64_t n, int32_t* label, int32_t* label2, int32_t* eu, 
 // dim: the cone dimension.
 void launch_rank_cones(int dim, int64_t n, const uint64_t* cand_key, const int32_t* cand_pos,
                        const int32_t* qlist, int64_t nq, uint64_t* rkey, int32_t* rpos, uint8_t* cursor,
-                       const Counters* C, hipStream_t s);
+                       const int32_t* reach, const Counters* C, hipStream_t s);
 // rkey / rpos: the ranked candidates of k_rank_cones (point-major, K per point)
 void launch_round_phase(int phase, int K, int64_t n, const uint32_t* ids, const uint64_t* rkey,
                         const int32_t* rpos, uint8_t* cursor, int32_t* label,
@@ -340,7 +373,7 @@ void launch_round_end(Counters* C, bool grouped, hipStream_t s, unsigned long lo
 // the device's constant-rate clock (hipDeviceAttributeWallClockRate) into *at
 void launch_stamp(unsigned long long* at, hipStream_t s);
 // Queue the points holding a zero-distance or no candidate.
-void launch_flag_research(int K, int64_t n, const uint64_t* cand_key, int32_t* list,
+void launch_flag_research(int K, int64_t n, const uint64_t* cand_key, int32_t* list, const int32_t* reach,
                           Counters* C, hipStream_t s);
 void launch_weight(const float* xyz, int dim, const int32_t* eu, const int32_t* ev, int64_t m,
                    double* partial, int nblocks, hipStream_t s);

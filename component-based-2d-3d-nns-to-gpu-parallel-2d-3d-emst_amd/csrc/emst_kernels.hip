@@ -1318,6 +1318,7 @@ __device__ __forceinline__ int32_t key_bound(unsigned long long k)
 }
 
 constexpr int kMaxCappedPasses = 6;
+constexpr int32_t kReachAll = 0x7fffffff;       // every cone of the point is exact
 // packets of a cone search, at least (launch_cone_search), and the resumed
 // queries up to which their packets take kConeFewPacket each
 constexpr int64_t kConePackets = 2500;
@@ -1865,9 +1866,9 @@ template <int D>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D == 3 ? 3 : 4))) void k_cone_first(
     const float4* __restrict__ pts, const Node* __restrict__ nodes, const Cloud* __restrict__ clouds, int ncl,
     int bucket, LeafTable lt, int64_t n, const int32_t* __restrict__ inv, const float* __restrict__ seed_r,
-    float seed_scale, uint64_t* __restrict__ cand_key, int32_t* __restrict__ cand_pos,
+    float seed_scale, float seed_mul, uint64_t* __restrict__ cand_key, int32_t* __restrict__ cand_pos,
     int32_t* __restrict__ first_corr, uint64_t* __restrict__ first_key, Counters* __restrict__ ctr,
-    int collect_stats, DupState dup, uint64_t* __restrict__ open_out)
+    int collect_stats, DupState dup, uint64_t* __restrict__ open_out, int32_t* __restrict__ reach)
 {
     using C = ConeCfg<D>;
     static_assert(C::K == D * (1 << D), "one row per axis and octant");
@@ -1927,6 +1928,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D == 3 ? 3 :
             if (!positive_finite(sp)) sp = 1e-6f;
             r = seed_scale * sp;
         }
+        r *= seed_mul;
         const float r2 = r * r;
         // boxes of the lanes and of each 8-lane group
         float qlo[3] = {mine ? px : INFINITY, mine ? py : INFINITY, mine ? pz : INFINITY};
@@ -2005,8 +2007,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D == 3 ? 3 :
         }
         if (over) {
             // too far for the lists: left open without a best
-            if (mine)
+            if (mine) {
                 for (int c = 0; c < C::K; ++c) cand_key[(int64_t)c * n + p] = kEmptyKey;
+                if (reach) {
+                    reach[p] = -1;
+                    first_corr[p] = -2;
+                    first_key[p] = kEmptyKey;
+                }
+            }
             open_lanes |= __ballot(mine);
             continue;
         }
@@ -2159,6 +2167,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D == 3 ? 3 :
             kmin = k < kmin ? k : kmin;
         }
         open = open && mine;
+        if (reach) {
+            // late cones (k_late_mark): nothing is left open here
+            if (mine) reach[p] = open ? (int32_t)__float_as_uint(r2) : kReachAll;
+            open = false;
+        }
         open_lanes |= __ballot(open);
         // distinct points at float distance 0 break the grouping's
         // premise; the caller then searches ungrouped
@@ -2180,13 +2193,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D == 3 ? 3 :
                 }
             }
             if (!open && first_corr) {
+                // (bests lie within R_0, so the smallest is exact)
                 first_corr[p] = pmin >= 0 ? pmin : -2;
                 first_key[p] = kmin;
             }
         }
         __builtin_amdgcn_wave_barrier();
     }
-    if (lane == 0) open_out[blockIdx.x] = open_lanes;
+    if (lane == 0 && open_out) open_out[blockIdx.x] = open_lanes;
     if (collect_stats && lane == 0) cone_work(ctr, st_nodes, st_leaves, st_pts, st_pairs);
     if (__ballot(underflow) != 0ull && lane == 0) atomicOr(&ctr->underflow, 1u);
 }
@@ -2459,6 +2473,8 @@ __global__ void k_round_begin(Counters* C)
     C->edges_prev = C->edges;
     C->nroots = 0;
     C->walk_left = 0;
+    C->late = 0;
+    C->late_checks = 0;
     C->deferred = 0;
 }
 
@@ -2491,11 +2507,12 @@ __global__ void k_stamp(unsigned long long* at)
 // at all (NodeEMST.h:1051-1077).
 __global__ __launch_bounds__(kBlock) void k_flag_research(int K, int64_t n,
                                                          const uint64_t* __restrict__ cand_key,
-                                                         int32_t* __restrict__ list, Counters* C)
+                                                         int32_t* __restrict__ list,
+                                                         const int32_t* __restrict__ reach, Counters* C)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
-    bool zero = false, any = false;
+    bool zero = false, any = reach && reach[p] != kReachAll;    // (late cones: not known to be empty)
     for (int k = 0; k < K; ++k) {
         const uint64_t key = cand_key[(int64_t)k * n + p];
         if (key == kEmptyKey) continue;
@@ -2588,6 +2605,7 @@ __global__ __launch_bounds__(kBlock) void k_rank_cones(int64_t n, const uint64_t
                                                       const int32_t* __restrict__ qlist, int64_t nq,
                                                       uint64_t* __restrict__ rkey, int32_t* __restrict__ rpos,
                                                       uint8_t* __restrict__ cursor,
+                                                      const int32_t* __restrict__ reach,
                                                       const Counters* __restrict__ C)
 {
     using CC = ConeCfg<D>;
@@ -2597,6 +2615,7 @@ __global__ __launch_bounds__(kBlock) void k_rank_cones(int64_t n, const uint64_t
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nq) return;
     const int64_t p = qlist ? (int64_t)qlist[t] : t;
+    const int32_t upto = reach ? reach[p] : kReachAll;
     uint64_t key[P];
     int32_t pos[P];
 #pragma unroll
@@ -2604,6 +2623,14 @@ __global__ __launch_bounds__(kBlock) void k_rank_cones(int64_t n, const uint64_t
         key[c] = c < CC::K ? cand_key[(int64_t)c * n + p] : kEmptyKey;
         pos[c] = c < CC::K ? cand_pos[(int64_t)c * n + p] : -1;
     }
+    // a late point's cones past its first radius are not exact yet
+    if (upto != kReachAll)
+#pragma unroll
+        for (int c = 0; c < P; ++c)
+            if (key_bound(key[c]) > upto) {
+                key[c] = kEmptyKey;
+                pos[c] = -1;
+            }
 #pragma unroll
     for (int k = 2; k <= P; k <<= 1)
 #pragma unroll
@@ -2640,6 +2667,78 @@ __global__ __launch_bounds__(kBlock) void k_rank_cones(int64_t n, const uint64_t
 // differs: the cones are ranked once (k_rank_cones) and cursor[p] skips the
 // ones already found inside the component, which never leave it (components
 // only merge), so each candidate is looked at about once over all rounds.
+__device__ __forceinline__ void round_min_point(bool inb, int64_t p, int K, const uint32_t* __restrict__ ids,
+                                                const uint64_t* __restrict__ rkey,
+                                                const int32_t* __restrict__ rpos, uint8_t* __restrict__ cursor,
+                                                const int32_t* __restrict__ label, int32_t* __restrict__ corr,
+                                                uint64_t* __restrict__ corr_key, uint64_t* __restrict__ comp1)
+{
+    int32_t lp = 0;
+    uint64_t key1 = kEmptyKey;
+    bool valid = false;
+    if (inb) {
+        lp = label[p];
+        int32_t c = corr[p];
+        uint64_t ck = corr_key[p];
+        // corr == -2: every cone candidate already inside the component;
+        // since components only merge, the point never has an outgoing
+        // candidate again (until a repeated cone search or a group
+        // refresh gives it new candidates)
+        if (c != -2 && !(c >= 0 && label[c] != lp)) {
+            c = -1;
+            ck = kEmptyKey;
+            // kStep ranks per step, their loads independent of each other,
+            // so a long run of candidates inside the component costs few
+            // round trips to memory
+            constexpr int kStep = 4;
+            int r = cursor[p];
+            bool more = r < K;
+            const uint64_t* __restrict__ kr = rkey + p * (int64_t)K;
+            const int32_t* __restrict__ pr = rpos + p * (int64_t)K;
+            while (more) {
+                uint64_t key[kStep];
+                int32_t q[kStep], lq[kStep];
+#pragma unroll
+                for (int i = 0; i < kStep; ++i) {
+                    key[i] = kEmptyKey;
+                    q[i] = -1;
+                    if (r + i < K) {
+                        key[i] = kr[r + i];
+                        q[i] = pr[r + i];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < kStep; ++i) lq[i] = key[i] != kEmptyKey ? label[q[i]] : lp;
+#pragma unroll
+                for (int i = 0; i < kStep; ++i) {
+                    if (!more) continue;
+                    if (key[i] == kEmptyKey) {      // ranked last: no outgoing candidate left
+                        r = K;
+                        more = false;
+                    } else if (lq[i] != lp) {
+                        ck = key[i];
+                        c = q[i];
+                        more = false;
+                    } else {
+                        ++r;
+                    }
+                }
+                more = more && r < K;
+            }
+            cursor[p] = (uint8_t)r;
+            corr[p] = c == -1 ? -2 : c;
+            corr_key[p] = ck;
+        }
+        if (c >= 0) {
+            const uint32_t pid = ids[p];
+            const uint32_t qid = (uint32_t)ck;
+            key1 = (ck & 0xffffffff00000000ull) | (uint64_t)min(pid, qid);
+            valid = true;
+        }
+    }
+    atomic_min_grouped(comp1, lp, key1, valid);
+}
+
 __global__ __launch_bounds__(kBlock) void k_round_min(int K, int64_t n, const uint32_t* __restrict__ ids,
                                                      const uint64_t* __restrict__ rkey,
                                                      const int32_t* __restrict__ rpos,
@@ -2650,80 +2749,351 @@ __global__ __launch_bounds__(kBlock) void k_round_min(int K, int64_t n, const ui
                                                      uint64_t* __restrict__ comp1, const Counters* C)
 {
     if (C->done) return;
-    {
-        const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-        const bool inb = p < n;
-        int32_t lp = 0;
-        uint64_t key1 = kEmptyKey;
-        bool valid = false;
-        if (inb) {
-            lp = label[p];
-            int32_t c = corr[p];
-            uint64_t ck = corr_key[p];
-            // corr == -2: every cone candidate already inside the component;
-            // since components only merge, the point never has an outgoing
-            // candidate again (until a repeated cone search or a group
-            // refresh gives it new candidates)
-            if (c != -2 && !(c >= 0 && label[c] != lp)) {
-                c = -1;
-                ck = kEmptyKey;
-                // kStep ranks per step, their loads independent of each other,
-                // so a long run of candidates inside the component costs few
-                // round trips to memory
-                constexpr int kStep = 4;
-                int r = cursor[p];
-                bool more = r < K;
-                const uint64_t* __restrict__ kr = rkey + p * (int64_t)K;
-                const int32_t* __restrict__ pr = rpos + p * (int64_t)K;
-                while (more) {
-                    uint64_t key[kStep];
-                    int32_t q[kStep], lq[kStep];
-#pragma unroll
-                    for (int i = 0; i < kStep; ++i) {
-                        key[i] = kEmptyKey;
-                        q[i] = -1;
-                        if (r + i < K) {
-                            key[i] = kr[r + i];
-                            q[i] = pr[r + i];
-                        }
-                    }
-#pragma unroll
-                    for (int i = 0; i < kStep; ++i) lq[i] = key[i] != kEmptyKey ? label[q[i]] : lp;
-#pragma unroll
-                    for (int i = 0; i < kStep; ++i) {
-                        if (!more) continue;
-                        if (key[i] == kEmptyKey) {      // ranked last: no outgoing candidate left
-                            r = K;
-                            more = false;
-                        } else if (lq[i] != lp) {
-                            ck = key[i];
-                            c = q[i];
-                            more = false;
-                        } else {
-                            ++r;
-                        }
-                    }
-                    more = more && r < K;
-                }
-                cursor[p] = (uint8_t)r;
-                corr[p] = c == -1 ? -2 : c;
-                corr_key[p] = ck;
-            }
-            if (c >= 0) {
-                const uint32_t pid = ids[p];
-                const uint32_t qid = (uint32_t)ck;
-                key1 = (ck & 0xffffffff00000000ull) | (uint64_t)min(pid, qid);
-                valid = true;
-            }
-        }
-        atomic_min_grouped(comp1, lp, key1, valid);
-    }
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    round_min_point(p < n, p, K, ids, rkey, rpos, cursor, label, corr, corr_key, comp1);
 }
 
 // a member's edge key, high part: (d2, min id); the max id completes it
 __device__ __forceinline__ uint64_t edge_key1(uint64_t ck, uint32_t pid)
 {
     return (ck & 0xffffffff00000000ull) | (uint64_t)min(pid, (uint32_t)ck);
+}
+
+// Late cones.  A first pass of the cone search leaves a point late when a cone
+// of it has no point within R_0: its cones are exact up to reach[p] (the bits
+// of R_0^2; -1: none is known; kReachAll: all are exact), and only the exact
+// ones are ranked.  The rounds go on without the rest: a late point matters
+// only in a round in which every exact candidate of its has joined its
+// component while the component's smallest edge is beyond what the point has
+// seen (its reach, or the nearest outside point that an earlier round found,
+// corr_key).  Those points are listed here, after the round's minima.  Few of
+// them get their cones searched to the end (k_cone_rest).  More of them pause
+// the round, and their nearest points outside the component are searched
+// instead (launch_late_search).
+constexpr int kLateChunk = 2048;        // points per block: one list reservation each
+constexpr int kLatePer = kLateChunk / kBlock;
+
+__global__ __launch_bounds__(kBlock) void k_late_mark(int64_t n, const int32_t* __restrict__ label,
+                                                     const int32_t* __restrict__ corr,
+                                                     uint64_t* __restrict__ corr_key,
+                                                     const uint64_t* __restrict__ comp1,
+                                                     const int32_t* __restrict__ reach,
+                                                     int32_t* __restrict__ list, Counters* C)
+{
+    if (C->done) return;
+    __shared__ uint32_t wsum[kBlock / 64];
+    __shared__ uint32_t base;
+    const int64_t c0 = (int64_t)blockIdx.x * kLateChunk + (int64_t)(threadIdx.x / 64) * 64 * kLatePer + __lane_id();
+    uint32_t bits = 0, tot = 0;
+    uint32_t at[kLatePer];
+#pragma unroll
+    for (int i = 0; i < kLatePer; ++i) {
+        const int64_t p = c0 + i * 64;
+        bool need = false;
+        if (p < n && corr[p] == -2) {
+            const int32_t r = reach[p];
+            if (r != kReachAll) {
+                // no outside point's d2 is below `seen`
+                const uint32_t lo = (uint32_t)(corr_key[p] >> 32);
+                const int32_t seen = max(r, lo == 0xffffffffu ? -1 : (int32_t)lo);
+                const uint32_t edge = (uint32_t)(comp1[label[p]] >> 32);
+                need = seen < 0 || edge > (uint32_t)seen;
+                if (need && seen >= 0) corr_key[p] = ((uint64_t)(uint32_t)seen << 32) | 0xffffffffull;
+            }
+        }
+        const uint64_t m = __ballot(need);
+        at[i] = tot + (uint32_t)__popcll(m & lanemask_lt());
+        tot += (uint32_t)__popcll(m);
+        if (need) bits |= 1u << i;
+    }
+    const int w = threadIdx.x / 64;
+    if (__lane_id() == 0) wsum[w] = tot;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (int j = 0; j < kBlock / 64; ++j) {
+            const uint32_t x = wsum[j];
+            wsum[j] = t;
+            t += x;
+        }
+        base = t ? atomicAdd(&C->late, t) : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kLatePer; ++i)
+        if ((bits >> i) & 1u) list[base + wsum[w] + at[i]] = (int32_t)(c0 + i * 64);
+}
+
+// points without a candidate left look again (their cones are exact now)
+__global__ __launch_bounds__(kBlock) void k_revive(int64_t n, int32_t* __restrict__ corr)
+{
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < n && corr[p] == -2) corr[p] = -1;
+}
+
+// After the search of the listed points' nearest points outside their
+// components: a point whose edge is its component's smallest keeps it as its
+// target and is listed for k_cone_rest's check (not in round 1, where every
+// point is a component and its nearest point is the smallest cone candidate);
+// the others wait, their nearest outside point's d2 a lower bound.  A pair at
+// distance zero is left to the exact cones (done = 4), with its rule of
+// repeated searches.
+__global__ __launch_bounds__(kBlock) void k_late_settle(const int32_t* __restrict__ list,
+                                                       const uint32_t* __restrict__ ids,
+                                                       const int32_t* __restrict__ label,
+                                                       int32_t* __restrict__ corr,
+                                                       const uint64_t* __restrict__ corr_key,
+                                                       const uint64_t* __restrict__ comp1,
+                                                       int32_t* __restrict__ check, Counters* C)
+{
+    if (C->done) return;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool on = t < (int64_t)C->late;
+    bool keep = false;
+    int32_t p = 0;
+    if (on) {
+        p = list[t];
+        if (corr[p] >= 0) {
+            const uint64_t ck = corr_key[p];
+            keep = edge_key1(ck, ids[p]) == comp1[label[p]];
+            if ((ck >> 32) == 0u) C->done = 4u;
+        }
+        if (!keep) corr[p] = -2;
+    }
+    const bool add = keep && C->round > 1u;
+    const uint64_t m = __ballot(add);
+    if (m == 0ull) return;
+    uint32_t base = 0;
+    if (__lane_id() == (int)__builtin_ctzll(m)) base = atomicAdd(&C->late_checks, (uint32_t)__popcll(m));
+    base = (uint32_t)__shfl((int)base, (int)__builtin_ctzll(m));
+    if (add) check[base + (uint32_t)__popcll(m & lanemask_lt())] = p;
+}
+
+// The open cones of listed points, searched to the end: one wave per point,
+// one tree node per lane.  A step takes the 32 nearest-first nodes on top of
+// the stack, tests their 64 children against the cones' bounds, sorts the
+// needed ones by distance, reads the leaves among them (64 points at a time)
+// and pushes the rest, nearest on top.  Lane c keeps cone c; cones exact to
+// reach[p] are closed, the bests found beyond it are bounds.
+//
+// Against packets of 64 queries (k_cone_search from pass 1), whose wave walks
+// the union of their trees one node at a time: a few listed points lie apart,
+// and a packet of 25 took 8 ms; here each takes some 100 us, 20 ns in a full
+// launch.  Packets of neighbouring queries share their walk and are the faster
+// ones for many (400000 points of 10^6: 1.8 against 6.4 ms).
+//
+// kRestCheck: whether a late point's target is its cone's nearest point (the
+// target's cones, up to its distance); if not, done = 4.
+constexpr int kRestStack = 1024;
+constexpr int kRestBlocks = 5120;       // 20 waves a CU
+constexpr int kRestReserve = 64;        // left for a plain descent (one node a step)
+
+__global__ __launch_bounds__(64) void k_cone_rest(ConeRest a, const uint32_t* __restrict__ nq_dev, int64_t few,
+                                                  int mode)
+{
+    using CC = ConeCfg<3>;
+    const int64_t nq = (int64_t)*nq_dev;
+    if ((int64_t)blockIdx.x >= nq || a.C->done) return;
+    if (nq > few) {
+        // too many for one wave each: packets (k_cone_search); a round waits
+        if (mode == kRestRound && blockIdx.x == 0 && threadIdx.x == 0) a.C->done = 3u;
+        return;
+    }
+    __shared__ unsigned long long stk[kRestStack];
+    __shared__ unsigned long long best[CC::K];
+    const int lane = __lane_id();
+    const int64_t n = a.n;
+    const int lb = 31 - __builtin_clz(a.bucket);
+    const int per_step = 64 >> lb;
+    uint32_t st_nodes = 0, st_leaves = 0;
+    for (int64_t qi = blockIdx.x; qi < nq; qi += gridDim.x) {
+        const int32_t p = __builtin_amdgcn_readfirstlane(a.list[qi]);
+        const int cl = find_cloud(a.clouds, a.ncl, p);
+        const int64_t cend = a.clouds[cl].pos + a.clouds[cl].n;
+        const int64_t L = a.clouds[cl].L, lfirst = a.clouds[cl].lfirst, nl = a.clouds[cl].nl;
+        const Node* __restrict__ tree = a.nodes + 2 * a.clouds[cl].lbase;
+        const float4 me = a.pts[p];
+        const float px = me.x, py = me.y, pz = me.z;
+        int32_t inner = -1;
+        unsigned long long mine = kEmptyKey;
+        uint64_t open = 0;
+        if (mode == kRestCheck) {
+            const float4 q = a.pts[a.corr[p]];
+            open = cone_mask<3>(q.x - px, q.y - py, q.z - pz);
+            mine = a.corr_key[p];
+        } else {
+            inner = a.reach[p];
+            if (lane < CC::K) mine = a.cand_key[(int64_t)lane * n + p];
+            open = __ballot(lane < CC::K && key_bound(mine) > inner);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (lane < CC::K) best[lane] = mine;
+        __builtin_amdgcn_wave_barrier();
+        // in a round the cones need be exact only up to the component's edge,
+        // so up to any outside point met (k_late_seen)
+        const int32_t lp = a.label[p];
+        int32_t cap = mode == kRestRound ? key_bound(a.comp1[lp]) : kReachAll;
+        cap = __builtin_amdgcn_readfirstlane(cap);
+        int32_t bound[CC::K];
+        int32_t maxb = -1;
+        auto refresh = [&]() {
+            maxb = -1;
+#pragma unroll
+            for (int c = 0; c < CC::K; ++c) {
+                const int32_t b = (open >> c) & 1ull
+                                      ? min(cap, __builtin_amdgcn_readfirstlane(key_bound(best[c]))) : -1;
+                bound[c] = b;
+                maxb = max(maxb, b);
+            }
+        };
+        refresh();
+        // one step's leaves, in the order of their lanes
+        auto leaves = [&](uint64_t lm, uint64_t key) {
+            while (lm) {
+                // the next per_step leaves; lane -> its leaf's lane
+                int src = -1, got = 0;
+                while (got < per_step && lm) {
+                    const int l = (int)__builtin_ctzll(lm);
+                    lm &= lm - 1;
+                    if ((int32_t)__builtin_amdgcn_readlane((int)(key >> 32), l) > maxb) continue;
+                    if (got == (lane >> lb)) src = l;
+                    ++got;
+                }
+                if (got == 0) break;
+                st_leaves += (uint32_t)got;
+                const int node = __shfl((int)(uint32_t)key, src < 0 ? 0 : src);
+                bool low = false;
+                uint32_t out = 0xffffffffu;
+                if (src >= 0) {
+                    int64_t s0, s1;
+                    leaf_range(a.lt, lfirst, nl, cend, node - L, s0, s1);
+                    s0 += lane & (a.bucket - 1);
+                    if (s0 < s1) {
+                        const float4 v = a.pts[s0];
+                        const float dx = v.x - px, dy = v.y - py, dz = v.z - pz;
+                        const float d2 = d2_of(dx, dy, dz);
+                        const int32_t db = (int32_t)__float_as_uint(d2);
+                        if (s0 != (int64_t)p && db <= maxb && db > inner) {
+                            if (mode == kRestRound && a.label[s0] != lp) out = (uint32_t)db;
+                            uint32_t cm = cone_mask<3>(dx, dy, dz) & (uint32_t)open;
+                            const unsigned long long kk =
+                                ((unsigned long long)__float_as_uint(d2) << 32) | __float_as_uint(v.w);
+                            while (cm) {
+                                const int c = __builtin_ctz(cm);
+                                cm &= cm - 1;
+                                if (kk < best[c]) {
+                                    atomicMin(&best[c], kk);
+                                    low = true;
+                                }
+                            }
+                        }
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();
+                if (__ballot(out < (uint32_t)cap) != 0ull) cap = min(cap, (int32_t)wave_min_u32(out));
+                if (__ballot(low) != 0ull) refresh();
+            }
+        };
+        int sp;
+        if (L == 1) {
+            sp = 0;
+            if (open) leaves(1ull, (uint64_t)1);
+        } else {
+            sp = (int)(L / 2 < 32 ? L / 2 : 32);
+            if (lane < sp) stk[lane] = (unsigned long long)(sp + lane);
+        }
+        if (!open) sp = 0;
+        __builtin_amdgcn_wave_barrier();
+        while (sp > 0) {
+            const int room = kRestStack - kRestReserve - sp;
+            const int take = min(min(sp, 32), max(1, room));
+            const bool on = (lane >> 1) < take;
+            const unsigned long long e = on ? stk[sp - 1 - (lane >> 1)] : kEmptyKey;
+            sp -= take;
+            uint64_t key = kEmptyKey;
+            if (on && (int32_t)(e >> 32) <= maxb) {
+                const int child = 2 * (int)(uint32_t)e + (lane & 1);
+                const Node x = tree[child];
+                if (node_needed<3, 3>(x, px, py, pz, bound, maxb, inner, false)) {
+                    const float m0 = fmaxf(fmaxf(x.lo[0] - px, px - x.hi[0]), 0.f);
+                    const float m1 = fmaxf(fmaxf(x.lo[1] - py, py - x.hi[1]), 0.f);
+                    const float m2 = fmaxf(fmaxf(x.lo[2] - pz, pz - x.hi[2]), 0.f);
+                    const float m = d2_of(m0, m1, m2);
+                    key = (uint64_t)__float_as_uint(m) << 32 | (uint32_t)child;
+                }
+            }
+            ++st_nodes;
+            if (__ballot(key != kEmptyKey) == 0ull) continue;
+            key = wave_sort_u64(key);
+            leaves(__ballot(key != kEmptyKey && (int64_t)(uint32_t)key >= L), key);
+            const bool go = key != kEmptyKey && (int64_t)(uint32_t)key < L && (int32_t)(key >> 32) <= maxb;
+            const uint64_t gm = __ballot(go);
+            const int cnt = __popcll(gm);
+            if (go) stk[sp + cnt - 1 - __popcll(gm & lanemask_lt())] = key;
+            sp += cnt;
+            __builtin_amdgcn_wave_barrier();
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (mode == kRestCheck) {
+            if (__ballot(((open >> lane) & 1ull) && best[lane < CC::K ? lane : 0] == mine) == 0ull && lane == 0)
+                a.C->done = 4u;
+            continue;
+        }
+        // results
+        uint64_t key = kEmptyKey;
+        int32_t pos = -1;
+        if (lane < CC::K) {
+            key = best[lane];
+            pos = key == kEmptyKey ? -1 : a.inv[(uint32_t)key];
+            a.cand_key[(int64_t)lane * n + p] = key;
+            a.cand_pos[(int64_t)lane * n + p] = pos;
+        }
+        if (lane == 0) a.reach[p] = cap;        // (kReachAll without one)
+        key = wave_sort_u64(key_bound(key) <= cap ? key : kEmptyKey);
+        pos = key == kEmptyKey ? -1 : a.inv[(uint32_t)key];
+        if (lane < CC::K) {
+            a.rkey[(int64_t)p * CC::K + lane] = key;
+            a.rpos[(int64_t)p * CC::K + lane] = pos;
+        }
+        // (a pair at distance zero: its rule of repeated searches, as in k_late_settle)
+        if (lane == 0 && (key >> 32) == 0u) a.C->done = 4u;
+        const uint64_t outm = __ballot(pos >= 0 && a.label[pos >= 0 ? pos : 0] != lp);
+        const int first = outm ? (int)__builtin_ctzll(outm) : CC::K;
+        if (lane == (outm ? first : 0)) {
+            a.cursor[p] = (uint8_t)first;
+            // (a target that is still outside was the smallest candidate, and stays it)
+            a.corr[p] = outm ? pos : -2;
+            a.corr_key[p] = outm ? key : kEmptyKey;
+            if (outm) {
+                const uint64_t k1 = (key & 0xffffffff00000000ull) | (uint64_t)min(a.ids[p], (uint32_t)key);
+                atomic_min_if_lower(&a.comp1[lp], k1);
+            }
+        }
+    }
+    if (lane == 0) {
+        const int slot = (int)(blockIdx.x % kWorkSlots);
+        atomicAdd(&a.C->work[kWorkConeNodes][slot], (unsigned long long)st_nodes);
+        atomicAdd(&a.C->work[kWorkConeLeaves][slot], (unsigned long long)st_leaves);
+        atomicAdd(&a.C->work[kWorkConePairs][slot], (unsigned long long)st_leaves * (unsigned long long)a.bucket);
+    }
+}
+
+// A listed point searched up to its nearest outside point without finding a
+// candidate there: a cone's nearest point is one of its component, which lies
+// nearer to that outside point and so has the smaller edge.  The component's
+// edge is then within what the point has seen; if not (in floats), the run
+// needs exact cones.
+__global__ __launch_bounds__(kBlock) void k_late_seen(const int32_t* __restrict__ list,
+                                                     const int32_t* __restrict__ label,
+                                                     const int32_t* __restrict__ corr,
+                                                     const uint64_t* __restrict__ comp1,
+                                                     const int32_t* __restrict__ reach, Counters* C)
+{
+    if (C->done) return;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= C->late) return;
+    const int32_t p = list[t], r = reach[p];
+    if (corr[p] == -2 && r != kReachAll && (r < 0 || (uint32_t)(comp1[label[p]] >> 32) > (uint32_t)r)) C->done = 4u;
 }
 
 // second phase: among members matching (d2, min id), the smallest max id.
@@ -4540,7 +4910,7 @@ __global__ __launch_bounds__(kBlock) void k_round_flatten(int64_t n, int32_t* __
                                                          uint64_t* __restrict__ comp1,
                                                          uint32_t* __restrict__ comp2, Counters* C)
 {
-    if (C->done == 1u) return;      // a paused round (done == 2) still flattens
+    if (C->done & 1u || C->done == 4u) return;      // a round paused here (done == 2) still flattens
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     const int32_t was = label[p];
@@ -4842,10 +5212,10 @@ void launch_build_tree(const float4* pts, const Cloud* cl, int ncl, int64_t nlea
 
 void launch_cone_search(int dim, int cdim, const float4* pts, const Node* nodes, const Cloud* cl, int ncl,
                         int bucket, LeafTable lt, int64_t n, const int32_t* qlist, int64_t nq, const int32_t* label,
-                        bool check_labels, const int32_t* inv, const float* seed_r, float seed_scale,
+                        bool check_labels, const int32_t* inv, const float* seed_r, float seed_scale, float seed_mul,
                         uint64_t* cand_key, int32_t* cand_pos, int32_t* revive, int32_t* first_corr,
                         uint64_t* first_key, Counters* C, bool collect_stats, DupState dup,
-                        const SplitScratch* split, hipStream_t s)
+                        const SplitScratch* split, int32_t* reach, hipStream_t s)
 {
     if (nq <= 0) return;
     const unsigned g = nblocks(nq, 64);
@@ -4873,13 +5243,14 @@ void launch_cone_search(int dim, int cdim, const float4* pts, const Node* nodes,
     const int64_t P = (int64_t)g;
     if (cdim == dim)
         hipLaunchKernelGGL(dim == 3 ? (k_cone_first<3>) : (k_cone_first<2>), dim3(g), dim3(64), 0, s, pts, nodes, cl,
-                           ncl, bucket, lt, n, inv, seed_r, seed_scale, cand_key, cand_pos, first_corr, first_key, C,
-                           cs, dup, split->open_mask);
+                           ncl, bucket, lt, n, inv, seed_r, seed_scale, seed_mul, cand_key, cand_pos, first_corr, first_key, C,
+                           cs, dup, split->open_mask, reach);
     else
         hipLaunchKernelGGL(kern, dim3(g), dim3(64), 0, s, pts, nodes, cl, ncl, bucket, lt, n, qlist, nq, label,
                            check_labels ? 1 : 0, inv, seed_r, seed_scale, cand_key, cand_pos, revive, first_corr,
                            first_key, C, cs, dup, 0, 0, split->open_mask, (const uint32_t*)nullptr,
                            (const uint64_t*)nullptr, (int64_t)0, 64);
+    if (reach) return;          // late cones: the rounds ask for the rest
     hipLaunchKernelGGL(k_open_count, dim3(nblocks(P + 1)), dim3(kBlock), 0, s, split->open_mask, P, split->cnt);
     exclusive_scan_u32(split->cnt, split->off, P + 1, split->tmp, s);
     hipLaunchKernelGGL(k_open_fill, dim3((unsigned)P), dim3(64), 0, s, split->open_mask, split->off, split->list);
@@ -4888,6 +5259,36 @@ void launch_cone_search(int dim, int cdim, const float4* pts, const Node* nodes,
                        cand_key, cand_pos, revive, first_corr, first_key, C, cs, dup, 1, kMaxCappedPasses,
                        (uint64_t*)nullptr, (const uint32_t*)(split->off + P), (const uint64_t*)split->open_mask,
                        (int64_t)(split->compact_frac * (double)nq), 64);
+}
+
+// Points that k_cone_rest takes at most in a round; a round with more pauses.
+// (4096 / 16384, ms per run: clustered 10^4 points 1.50 / 1.06, 2*10^5 2.70 /
+// 2.18, 4*10^6 10.6 / 10.1.)
+constexpr int64_t kRestFew = 16384;
+
+// listed points one wave each: nq_dev of them; none when they are more than
+// `few`
+static void cone_rest(const ConeRest& a, const uint32_t* nq_dev, int64_t few, int mode, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cone_rest, dim3((unsigned)std::min<int64_t>(a.n, kRestBlocks)), dim3(64), 0, s, a, nq_dev,
+                       few, mode);
+}
+
+// Late cones in a round, after its minima (k_late_mark).
+void launch_late_cones(const ConeRest& a, hipStream_t s)
+{
+    if (a.n <= 0) return;
+    hipLaunchKernelGGL(k_late_mark, dim3((unsigned)((a.n + kLateChunk - 1) / kLateChunk)), dim3(kBlock), 0, s, a.n,
+                       a.label, (const int32_t*)a.corr, a.corr_key, (const uint64_t*)a.comp1,
+                       (const int32_t*)a.reach, a.list, a.C);
+    cone_rest(a, &a.C->late, kRestFew, kRestRound, s);
+    hipLaunchKernelGGL(k_late_seen, dim3((unsigned)(kRestFew / kBlock)), dim3(kBlock), 0, s, (const int32_t*)a.list,
+                       a.label, (const int32_t*)a.corr, (const uint64_t*)a.comp1, (const int32_t*)a.reach, a.C);
+}
+
+void launch_revive(int64_t n, int32_t* corr, hipStream_t s)
+{
+    if (n > 0) hipLaunchKernelGGL(k_revive, dim3(nblocks(n)), dim3(kBlock), 0, s, n, corr);
 }
 
 void launch_leaves(const uint64_t* keys, int64_t n, Cloud* cl, int ncl, int bucket, uint32_t* mark,
@@ -4922,6 +5323,73 @@ void launch_comp_seed_init(int64_t n, const float4* pts, int32_t* csize, uint32_
 {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_comp_seed_init, dim3(nblocks(n)), dim3(kBlock), 0, s, n, pts, csize, cbox);
+}
+
+// the component search's dispatches over a list of points (nq of them)
+static void comp_dispatches(int dim, int64_t n, const float4* pts, const Node* nodes, const Cloud* cl, int ncl,
+                            int bucket, LeafTable lt, const SplitScratch& sc, const int32_t* list,
+                            const uint32_t* nq, const int32_t* label, int32_t* corr, uint64_t* corr_key,
+                            uint64_t* comp1, const int32_t* inv, float seed_scale, const float* seed_r, Counters* C,
+                            hipStream_t s, hipEvent_t* ev)
+{
+    const int64_t P = (n + 63) / 64;
+    auto kern = dim == 3 ? (bucket == 64 ? k_comp_search<3, 64> : k_comp_search<3, 0>)
+                         : (bucket == 16 ? k_comp_search<2, 16> : k_comp_search<2, 0>);
+    // (2D at its default 64-point leaves runs the runtime-size instance: a
+    // <2, 64> instance measured 7% slower on the 2D power-law cloud)
+    // pass 0 over the searching points; their open packets' lanes into open_mask
+    if (ev) (void)hipEventRecord(ev[0], s);
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(P, kSearchBlocks)), dim3(64), 0, s, pts,
+                       nodes, cl, ncl, bucket, lt,
+                       list, nq, label, inv, seed_scale, corr, corr_key, comp1, 0, 0,
+                       sc.open_mask, seed_r, sc.defer, C, ev != nullptr ? 1 : 0);
+    if (ev) (void)hipEventRecord(ev[1], s);
+    open_compact(sc.open_mask, P, sc.off, sc.tmp, list, sc.list2, s);
+    if (ev) (void)hipEventRecord(ev[2], s);
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(P, kResumeBlocks)), dim3(64), 0, s, pts,
+                       nodes, cl, ncl, bucket, lt,
+                       (const int32_t*)sc.list2, (const uint32_t*)(sc.off + P), label, inv, seed_scale, corr,
+                       corr_key, comp1, 1, kMaxCappedPasses, (uint64_t*)nullptr, seed_r, sc.defer, C,
+                       ev != nullptr ? 1 : 0);
+    // the queries the packets handed over, one wave each
+    if (sc.defer != nullptr) {
+        auto dk = dim == 3 ? k_comp_search_deferred<3> : k_comp_search_deferred<2>;
+        hipLaunchKernelGGL(dk, dim3(kDeferBlocks), dim3(64 * kDeferWaves), 0, s, pts, nodes, cl, ncl, lt,
+                           (const uint64_t*)sc.defer, label, inv, seed_scale, corr, corr_key, comp1, seed_r, C,
+                           ev != nullptr ? 1 : 0);
+    }
+    if (ev) (void)hipEventRecord(ev[3], s);
+}
+
+// A round that too many late points pause (done == 3): their nearest points
+// outside their components, by the component search.  It finds the smallest
+// edge of every component whose exact candidates may not hold it.  The cones
+// would choose the same edge: a point nearer to p within the cone of p's edge
+// (p, q) is one of p's component and nearer to q than p is.  In floats that
+// last step could fail, so every edge chosen here is checked against its cone
+// (k_cone_rest), and one that fails restarts the run with exact cones
+// (done == 4).
+void launch_late_search(const ConeRest& a, Node* nodes, unsigned long long* visit, int64_t nleaves,
+                        bool first, float seed_scale, const SplitScratch& sc, hipStream_t s)
+{
+    const int64_t n = a.n, P = (n + 63) / 64;
+    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(kBlock), 0, s, &a.C->done, (int64_t)1);
+    hipLaunchKernelGGL(k_zero_u32, dim3(nblocks(2 * P)), dim3(kBlock), 0, s, reinterpret_cast<uint32_t*>(sc.open_mask),
+                       2 * P);
+    if (first) {
+        hipLaunchKernelGGL(k_zero_u32, dim3(nblocks(4 * nleaves)), dim3(kBlock), 0, s,
+                           reinterpret_cast<uint32_t*>(visit), 4 * nleaves);
+        launch_node_min_ids(a.pts, a.clouds, a.ncl, nleaves, a.lt, nodes, visit, s);
+    }
+    hipLaunchKernelGGL(k_nlab_tree, dim3(nblocks(nleaves)), dim3(kBlock), 0, s, a.label, a.clouds, a.ncl, nleaves,
+                       a.lt, nodes, visit, (const Counters*)a.C);
+    comp_dispatches(3, n, a.pts, nodes, a.clouds, a.ncl, a.bucket, a.lt, sc, (const int32_t*)a.list, &a.C->late,
+                    a.label, a.corr, a.corr_key, a.comp1, a.inv, seed_scale, nullptr, a.C, s, nullptr);
+    hipLaunchKernelGGL(k_late_settle, dim3(nblocks(n)), dim3(kBlock), 0, s, (const int32_t*)a.list, a.ids, a.label,
+                       a.corr, (const uint64_t*)a.corr_key, (const uint64_t*)a.comp1, sc.list2, a.C);
+    ConeRest chk = a;
+    chk.list = sc.list2;
+    cone_rest(chk, &a.C->late_checks, n, kRestCheck, s);
 }
 
 void launch_comp_round(int dim, int64_t n, const float4* pts, const uint32_t* ids, Node* nodes,
@@ -4962,32 +5430,8 @@ void launch_comp_round(int dim, int64_t n, const float4* pts, const uint32_t* id
             seed_r = cs.R;
         }
     }
-    auto kern = dim == 3 ? (bucket == 64 ? k_comp_search<3, 64> : k_comp_search<3, 0>)
-                         : (bucket == 16 ? k_comp_search<2, 16> : k_comp_search<2, 0>);
-    // (2D at its default 64-point leaves runs the runtime-size instance: a
-    // <2, 64> instance measured 7% slower on the 2D power-law cloud)
-    // pass 0 over the searching points; their open packets' lanes into open_mask
-    if (ev) (void)hipEventRecord(ev[0], s);
-    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(P, kSearchBlocks)), dim3(64), 0, s, pts,
-                       (const Node*)nodes, cl, ncl, bucket, lt,
-                       (const int32_t*)sc.list, nq, label, inv, seed_scale, corr, corr_key, comp1, 0, 0,
-                       sc.open_mask, seed_r, sc.defer, C, ev != nullptr ? 1 : 0);
-    if (ev) (void)hipEventRecord(ev[1], s);
-    open_compact(sc.open_mask, P, sc.off, sc.tmp, (const int32_t*)sc.list, sc.list2, s);
-    if (ev) (void)hipEventRecord(ev[2], s);
-    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(P, kResumeBlocks)), dim3(64), 0, s, pts,
-                       (const Node*)nodes, cl, ncl, bucket, lt,
-                       (const int32_t*)sc.list2, (const uint32_t*)(sc.off + P), label, inv, seed_scale, corr,
-                       corr_key, comp1, 1, kMaxCappedPasses, (uint64_t*)nullptr, seed_r, sc.defer, C,
-                       ev != nullptr ? 1 : 0);
-    // the queries the packets handed over, one wave each
-    if (sc.defer != nullptr) {
-        auto dk = dim == 3 ? k_comp_search_deferred<3> : k_comp_search_deferred<2>;
-        hipLaunchKernelGGL(dk, dim3(kDeferBlocks), dim3(64 * kDeferWaves), 0, s, pts, (const Node*)nodes, cl, ncl, lt,
-                           (const uint64_t*)sc.defer, label, inv, seed_scale, corr, corr_key, comp1, seed_r, C,
-                           ev != nullptr ? 1 : 0);
-    }
-    if (ev) (void)hipEventRecord(ev[3], s);
+    comp_dispatches(dim, n, pts, nodes, cl, ncl, bucket, lt, sc, (const int32_t*)sc.list, nq, label, corr, corr_key,
+                    comp1, inv, seed_scale, seed_r, C, s, ev);
     // comp1 now holds every component's edge: the sample log of this round
     if (cs.features_on && cs.samples != nullptr)
         hipLaunchKernelGGL(k_comp_samples, dim3(g), dim3(kBlock), 0, s, (const int32_t*)sc.list,
@@ -5051,20 +5495,20 @@ void launch_stamp(unsigned long long* at, hipStream_t s)
     hipLaunchKernelGGL(k_stamp, dim3(1), dim3(1), 0, s, at);
 }
 
-void launch_flag_research(int K, int64_t n, const uint64_t* cand_key, int32_t* list, Counters* C,
-                          hipStream_t s)
+void launch_flag_research(int K, int64_t n, const uint64_t* cand_key, int32_t* list, const int32_t* reach,
+                          Counters* C, hipStream_t s)
 {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_flag_research, dim3(nblocks(n)), dim3(kBlock), 0, s, K, n, cand_key, list, C);
+    hipLaunchKernelGGL(k_flag_research, dim3(nblocks(n)), dim3(kBlock), 0, s, K, n, cand_key, list, reach, C);
 }
 
 void launch_rank_cones(int dim, int64_t n, const uint64_t* cand_key, const int32_t* cand_pos,
                        const int32_t* qlist, int64_t nq, uint64_t* rkey, int32_t* rpos, uint8_t* cursor,
-                       const Counters* C, hipStream_t s)
+                       const int32_t* reach, const Counters* C, hipStream_t s)
 {
     if (nq <= 0) return;
     hipLaunchKernelGGL(dim == 3 ? k_rank_cones<3> : k_rank_cones<2>, dim3(nblocks(nq)), dim3(kBlock), 0, s, n,
-                       cand_key, cand_pos, qlist, nq, rkey, rpos, cursor, C);
+                       cand_key, cand_pos, qlist, nq, rkey, rpos, cursor, reach, C);
 }
 
 void launch_round_phase(int phase, int K, int64_t n, const uint32_t* ids, const uint64_t* rkey,

@@ -66,8 +66,11 @@ typedef struct {
                                skips that round's hook (emst_get_search_stats entry 7 counts
                                these).  Not with the learned seed radius. */
     int32_t search_split;   /* round-1 cone search launches (changes work, never results):
-                               0 auto (3 from 2^18 points in 3D and 2^19 in 2D, not in the
-                               2.5D mode; otherwise 1); 1 one launch for
+                               0 auto: 3D from 2^12 points (one cloud, no two at one place)
+                               the first pass with a smaller radius, the cones beyond it
+                               when a round asks for them; otherwise, and where the cones
+                               themselves are asked for, 3 from 2^18 points in 3D and 2^19
+                               in 2D (not in the 2.5D mode), else 1; 1 one launch for
                                every pass; 2 first pass, then the open queries resumed in place;
                                3 first pass, then the open queries compacted into full waves */
     int32_t round_search;   /* 0: round-1 cone search, candidates reused by every round (the
@@ -157,13 +160,12 @@ int emst_set_clouds(emst_ctx* ctx, int32_t ncl, const int64_t* npts, const float
 int emst_get_cloud_results(emst_ctx* ctx, double* weight, int32_t* edges, int32_t* last_round);
 
 /* Autotuner (no counterpart in the reference, whose cell size is the fixed
- * level radius): times the build and cone search of the context's current
- * points on the device for every leaf size (points per leaf cell: 16, 32,
+ * level radius): times runs of the context's current points on the device
+ * for every leaf size (points per leaf cell: 16, 32,
  * 64) and plain seed scale (2, 3, 4 leaf spacings), then every search_split
- * form (1, 2, 3) for the fastest pair, then whole runs with round_search 0
- * and with 1 at 64-point leaves (not with a learned model set, nor in the
- * 2.5D mode, where the
- * caller's choice stays); keeps the fastest choice in the context (used by
+ * form (1, 2, 3) for the fastest pair, each by whole runs, then round_search 0
+ * and 1 at 64-point leaves (not with a learned model set, nor in the 2.5D
+ * mode, where the caller's choice stays); keeps the fastest choice in the context (used by
  * every later set_points / set_clouds / run) and returns the pair; best_ms =
  * its build + cone search time.  The result of a run never depends on any of
  * them; any output may be NULL. */
@@ -258,7 +260,9 @@ int emst_get_times(emst_ctx* ctx, float* times, int32_t* n_times);
  * counterpart in the reference. */
 int emst_get_round_ends(emst_ctx* ctx, float* ms, int32_t* n);
 
-/* Counters of the last full cone search (the work behind its bytes):
+/* Counters of the last full cone search (the work behind its bytes; a run that
+ * left cones to its rounds, see emst_options.search_split, makes that search
+ * here):
  * [0] packets (waves of at most 64 queries), [1] node-test steps (a hierarchy
  * node against a packet's queries, or up to 64 nodes against the packet's
  * box), [2] leaf cells entered, [3] leaf points read (summed over packets), [4] point pairs
