@@ -110,6 +110,7 @@ struct emst_ctx {
     int ncl = 0;
     std::vector<Cloud> hcl;
     int64_t nleaves = 0, Lmax = 0;
+    int64_t tblocks = 0;                // blocks of the tree build (k_tree_low)
     int mbits = 16;                   // sort key bits per axis
     int64_t target_edges = 0;         // sum over clouds of (points - 1)
     const float* xyz = nullptr;       // input points on the device (AoS)
@@ -459,6 +460,7 @@ int layout_clouds(emst_ctx* c, int bucket)
     for (Cloud& cl : c->hcl) {
         cl.pos = pos;
         cl.lbase = 0;
+        cl.tbase = 0;
         cl.L = 1;
         cl.lfirst = 0;
         cl.nl = 0;
@@ -524,6 +526,7 @@ int make_leaves(emst_ctx* c)
     std::vector<int32_t> lf(c->ncl + 1);
     if ((rc = copy_out(c, {{lf.data(), c->cloud_lf.p, sizeof(int32_t) * (c->ncl + 1)}}))) return rc;
     int64_t lbase = 0, Lmax = 1;
+    c->tblocks = 0;
     for (int k = 0; k < c->ncl; ++k) {
         Cloud& cl = c->hcl[k];
         cl.lfirst = lf[k];
@@ -532,6 +535,8 @@ int make_leaves(emst_ctx* c)
         while (L < cl.nl) L <<= 1;
         cl.L = L;
         cl.lbase = lbase;
+        cl.tbase = c->tblocks;
+        c->tblocks += tree_blocks(L);
         lbase += L;
         Lmax = std::max(Lmax, L);
     }
@@ -796,7 +801,7 @@ int build(emst_ctx* c, bool all_cones)
         }
     }
     const DupState dup = dup_state(c);
-    launch_build_tree(c->pts.p, c->dcl.p, c->ncl, c->nleaves, c->Lmax, leaf_table(c), c->nodes.p, dup.rep, s);
+    launch_build_tree(c->pts.p, c->dcl.p, c->ncl, c->tblocks, c->Lmax, leaf_table(c), c->nodes.p, dup.rep, s);
     launch_round_init(n, c->label.p, c->label2.p, c->eu.p, c->corr.p, c->corr_key.p, c->comp1.p,
                       c->comp2.p, c->C, (uint32_t)c->target_edges, (uint32_t)c->opt.max_rounds, s);
     LAUNCHCHK(c);
@@ -804,7 +809,6 @@ int build(emst_ctx* c, bool all_cones)
         // the per-round component search has no round-1 search: every round
         // searches (launch_comp_round)
         HIPCHK(c, hipMemsetAsync(c->visit.p, 0, sizeof(unsigned long long) * 2 * c->nleaves, s));
-        launch_node_min_ids(c->pts.p, c->dcl.p, c->ncl, c->nleaves, leaf_table(c), c->nodes.p, c->visit.p, s);
         // round 1's targets and the neighbour lists; a run that logs the
         // learned seed's training pairs searches in round 1 as well (its log
         // starts there); the seed itself applies from round 3 on, past the
@@ -1213,6 +1217,7 @@ bool one_launch_on(const emst_ctx* c)
 int one_launch_layout(emst_ctx* c)
 {
     int64_t lbase = 0, Lmax = 1;
+    c->tblocks = 0;
     const int64_t per_slot = std::max(1, c->bucket / 4);
     for (Cloud& cl : c->hcl) {
         const int64_t want = std::max<int64_t>(1, (cl.n + per_slot - 1) / per_slot);
@@ -1220,6 +1225,8 @@ int one_launch_layout(emst_ctx* c)
         while (L < want) L <<= 1;
         cl.L = L;
         cl.lbase = lbase;
+        cl.tbase = c->tblocks;
+        c->tblocks += tree_blocks(L);
         cl.lfirst = 0;
         cl.nl = 0;
         lbase += L;
@@ -1255,11 +1262,10 @@ void issue_one_launch_build(emst_ctx* c)
                   c->scan_tmp.p, c->lstart.p, c->leaf_of.p, c->cloud_lf.p, c->P, c->C, true, s);
     // dup_runs .. cycles_cut start at zero (a kernel: no memset nodes in graphs)
     launch_zero_u32(&c->C->dup_runs, 8, s);
-    launch_build_tree(c->pts.p, c->dcl.p, c->ncl, c->nleaves, c->Lmax, leaf_table(c), c->nodes.p, nullptr, s);
+    launch_build_tree(c->pts.p, c->dcl.p, c->ncl, c->tblocks, c->Lmax, leaf_table(c), c->nodes.p, nullptr, s);
     launch_round_init(n, c->label.p, c->label2.p, c->eu.p, c->corr.p, c->corr_key.p, c->comp1.p,
                       c->comp2.p, c->C, (uint32_t)c->target_edges, (uint32_t)c->opt.max_rounds, s);
     launch_zero_u32(reinterpret_cast<uint32_t*>(c->visit.p), 4 * c->nleaves, s);
-    launch_node_min_ids(c->pts.p, c->dcl.p, c->ncl, c->nleaves, leaf_table(c), c->nodes.p, c->visit.p, s);
     launch_knn_first(c->dim, n, c->pts.p, c->nodes.p, c->dcl.p, c->ncl, c->bucket, leaf_table(c), c->inv.p,
                      c->corr.p, c->corr_key.p, NbrList{c->knn_pos.p, c->knn_key.p, c->knn_cur.p}, c->C, false, s);
 }
@@ -1279,6 +1285,8 @@ int run_one_launch(emst_ctx* c)
     std::vector<uintptr_t> key = graph_key(c);
     key.push_back((uintptr_t)c->xyz);
     key.push_back((uintptr_t)c->ncl);
+    key.push_back((uintptr_t)c->tblocks);
+    key.push_back((uintptr_t)c->Lmax);
     key.push_back((uintptr_t)c->resc.p);
     key.push_back((uintptr_t)c->keys0.p);
     key.push_back((uintptr_t)c->target_edges);
@@ -1397,7 +1405,7 @@ int morton_samples(emst_ctx* c, float* feat, float* target)
     HIPCHK(c, hipStreamSynchronize(s));
     cl.lfirst = lf[0];
     cl.nl = lf[1] - lf[0];
-    cl.lbase = 0;
+    cl.lbase = cl.tbase = 0;
     cl.L = 1;
     while (cl.L < cl.nl) cl.L <<= 1;
     if ((rc = ensure(c, nodes, 2 * (size_t)cl.L))) return rc;
@@ -1410,7 +1418,7 @@ int morton_samples(emst_ctx* c, float* feat, float* target)
         launch_dup_groups(keys0.p, pts.p, n, rep.p, runs.p, list.p, gslot.p, cnt.p, s);
     }
     const LeafTable lt{lstart.p, leaf_of.p};
-    launch_build_tree(pts.p, dcl.p, 1, cl.L, cl.L, lt, nodes.p, rep.p, s);
+    launch_build_tree(pts.p, dcl.p, 1, tree_blocks(cl.L), cl.L, lt, nodes.p, rep.p, s);
     launch_radius_features(c->dim, pts.p, nodes.p, cl.L, lt, n, c->feat.p, c->ls.p, s);
     launch_radius_targets(c->K, n, c->cand_key.p, ids.p, c->inv.p, c->ls.p, c->pred.p, s);
     LAUNCHCHK(c);

@@ -156,7 +156,10 @@ struct Cloud {
     int64_t L;
     int64_t lfirst;
     int64_t nl;
+    int64_t tbase;          // first block of its tree (k_tree_low)
 };
+constexpr int kTreeLeaves = 256;    // leaf slots per block of k_tree_low
+inline int64_t tree_blocks(int64_t L) { return (L + kTreeLeaves - 1) / kTreeLeaves; }
 
 // Leaves of the search hierarchy: the maximal cells of the binary prefix tree
 // of the sorted keys (curve prefixes) that hold at most `bucket` points; a
@@ -206,8 +209,8 @@ void launch_gather_sorted(const float* resc, const uint32_t* perm, int64_t n, in
 void launch_dup_groups(const uint64_t* keys, const float4* pts, int64_t n, int32_t* rep,
                        int32_t* runs, int32_t* list, int32_t* gslot, Counters* C, hipStream_t s);
 // Leaf boxes leave out group members (rep == nullptr: grouping off).
-// nleaves = sum of the clouds' L, Lmax = largest L.
-void launch_build_tree(const float4* pts, const Cloud* cl, int ncl, int64_t nleaves, int64_t Lmax, LeafTable lt,
+// blocks = the clouds' tree_blocks, Lmax = largest L.
+void launch_build_tree(const float4* pts, const Cloud* cl, int ncl, int64_t blocks, int64_t Lmax, LeafTable lt,
                        Node* nodes, const int32_t* rep, hipStream_t s);
 // The leaves of the sorted keys (see LeafTable): mark and idx are n words of
 // scratch, tmp scan_tmp_words(n); start (n + 1 words at most) and of (n) are
@@ -277,7 +280,8 @@ void launch_late_search(const ConeRest& a, Node* nodes, unsigned long long* visi
 void launch_revive(int64_t n, int32_t* corr, hipStream_t s);
 // Phase 0 of a round of the per-round component search (the alternative to
 // the round-1 cone search): node component labels (into Node::pad[1]; visit:
-// the arrival words of launch_node_min_ids), kept targets, and a search for
+// 2 * nleaves words of arrival state, zero before the first round over this
+// hierarchy and kept between rounds), kept targets, and a search for
 // the points whose target joined their component; writes corr / corr_key and
 // the component minima (comp1).  sc: open_mask, cnt, off, tmp, list and
 // list2; pass 0 runs over every searching point, the later passes over those
@@ -305,11 +309,12 @@ struct CompSeed {
 // point p at k * n + p (position -1, key all ones: the cloud has no more
 // points), and per point the entry its current target came from (K: the list
 // is used up).  K = knn_len(dim): longer lists in 3D, where they answer the
-// searches of the early rounds (clustered 3D 10^7: 6 entries 14.6 ms per
-// EMST, 8 13.7, 10 13.5, 12 14.9); 2D is fastest at 6 (12.3 ms; 8: 12.4,
-// 10: 12.6).
+// searches of the early rounds (clustered 3D 10^7: 6 entries 12.2 ms per
+// run, 7 11.9, 8 11.9, 9 11.9, 10 12.2; 512 clouds 10.9, 10.8, 11.1, 11.0,
+// 11.5); 2D is fastest at 6 and 7 (power-law 10^7: 4 11.3, 5 10.9, 6 10.6, 7
+// 10.5).
 constexpr int kKnn2 = 6;
-constexpr int kKnn3 = 10;
+constexpr int kKnn3 = 8;
 __host__ __device__ constexpr int knn_len(int dim) { return dim == 3 ? kKnn3 : kKnn2; }
 struct NbrList {
     int32_t* pos;           // K * n
@@ -323,8 +328,7 @@ void launch_comp_round(int dim, int64_t n, const float4* pts, const uint32_t* id
                        const int32_t* eu, const int32_t* eround, Counters* C, hipStream_t s,
                        hipEvent_t* ev = nullptr);
 // The round-1 targets of the component search and the neighbour lists: one
-// traversal per 64-point packet (after launch_round_init and
-// launch_node_min_ids).  Writes corr / corr_key (every component is one
+// traversal per 64-point packet (after launch_round_init).  Writes corr / corr_key (every component is one
 // point, so the nearest neighbour is the round's exact target) and nb.
 void launch_knn_first(int dim, int64_t n, const float4* pts, const Node* nodes, const Cloud* cl, int ncl,
                       int bucket, LeafTable lt, const int32_t* inv, int32_t* corr, uint64_t* corr_key,
@@ -335,12 +339,6 @@ void launch_comp_seed_init(int64_t n, const float4* pts, int32_t* csize, uint32_
 // MLP inference over X[0..*m_dev) (the comp search's device-side count).
 void launch_mlp_infer_dev(const float* model, const float* X, const uint32_t* m_dev, int64_t m_max, float* Y,
                           hipStream_t s);
-// Smallest point id under every node of the hierarchy, into Node::pad[0]
-// (0xffffffff for a node without points).  visit:
-// 2 * nleaves words of arrival state, zero before the first bottom-up launch
-// over this hierarchy (k_nmin_tree, k_nlab_tree) and kept between them.
-void launch_node_min_ids(const float4* pts, const Cloud* cl, int ncl, int64_t nleaves, LeafTable lt, Node* nodes,
-                         unsigned long long* visit, hipStream_t s);
 // Cones of every group point for the current labels (dim: the cone dimension) (after the grouped
 // cone search, and at the start of each round while a group may still span
 // several components).  Sets C->dup_split when one does.

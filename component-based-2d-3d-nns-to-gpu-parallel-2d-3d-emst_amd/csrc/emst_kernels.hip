@@ -107,6 +107,18 @@ __device__ __forceinline__ int find_cloud_leaf(const Cloud* cl, int ncl, int64_t
     return lo;
 }
 
+// the cloud whose tree block b is (k_tree_low)
+__device__ __forceinline__ int find_cloud_block(const Cloud* cl, int ncl, int64_t b)
+{
+    int lo = 0, hi = ncl - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (cl[mid].tbase <= b) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
 // sorted positions [s0, s1) of leaf slot j of a cloud (empty past its leaves)
 __device__ __forceinline__ void leaf_range(const LeafTable& lt, int64_t lfirst, int64_t nl, int64_t cend, int64_t j,
                                            int64_t& s0, int64_t& s1)
@@ -1131,53 +1143,105 @@ __global__ void k_dup_finish(Counters* C)
 // smallest id, wins every tie at their common location), so they are left out
 // and a leaf of members only keeps the empty box (+inf, -inf), which no node
 // test accepts.
-__global__ __launch_bounds__(kBlock) void k_leaves(const float4* __restrict__ pts,
-                                                  const Cloud* __restrict__ cl, int ncl, int64_t nleaves,
-                                                  LeafTable lt, Node* __restrict__ nodes,
-                                                  const int32_t* __restrict__ rep)
+//
+// One block per kTreeLeaves leaf slots of a cloud, an aligned subtree of it
+// (Cloud::tbase: the cloud's first block): four lanes read a leaf's points,
+// and the subtree's levels are combined in LDS.  The levels above, of clouds
+// with more slots, follow in one launch (k_tree_top).  With each node goes the
+// smallest point id under it (pad[0]): with ties on d2 broken by id, a node
+// at the bound can only matter when it holds a smaller id than the best so
+// far (runs of coincident points).  (A launch per level, a leaf to a lane and
+// the ids by a climb of atomics took 14 launches and 72 us at 131072 points, 20
+// and 296 us at 10^7; now 2, and 14 and 66 us.)
+constexpr int kTreeBlock = 4 * kTreeLeaves;
+
+__global__ __launch_bounds__(kTreeBlock) void k_tree_low(const float4* __restrict__ pts,
+                                                        const Cloud* __restrict__ cl, int ncl, LeafTable lt,
+                                                        Node* __restrict__ nodes, const int32_t* __restrict__ rep)
 {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= nleaves) return;
-    const int c = find_cloud_leaf(cl, ncl, g);
-    const int64_t j = g - cl[c].lbase;          // the cloud's leaf slot j
-    if (j >= cl[c].L) return;               // past the cloud's slots (one-launch capacity)
-    const bool grouped = rep != nullptr;
-    Node nd;
-    for (int k = 0; k < 3; ++k) { nd.lo[k] = INFINITY; nd.hi[k] = -INFINITY; }
-    nd.pad[0] = nd.pad[1] = 0.f;
-    int64_t s0, s1;
-    leaf_range(lt, cl[c].lfirst, cl[c].nl, cl[c].pos + cl[c].n, j, s0, s1);
-    for (int64_t s = s0; s < s1; ++s) {
-        if (grouped) {
-            const int32_t r = rep[s];
-            if (r >= 0 && r != (int32_t)s) continue;
+    __shared__ float lo[3][kTreeLeaves], hi[3][kTreeLeaves];
+    __shared__ uint32_t mid[kTreeLeaves];
+    const int c = find_cloud_block(cl, ncl, (int64_t)blockIdx.x);
+    const int64_t L = cl[c].L, j0 = ((int64_t)blockIdx.x - cl[c].tbase) * kTreeLeaves;
+    if (j0 >= L) return;                    // past the cloud's slots (one-launch capacity)
+    Node* base = nodes + 2 * cl[c].lbase;
+    const int w = (int)(L < kTreeLeaves ? L : kTreeLeaves);
+    const int t = (int)threadIdx.x, slot = t >> 2;
+    auto put = [&](int64_t i, const float* l, const float* h, uint32_t m) {
+        Node nd;
+        for (int k = 0; k < 3; ++k) { nd.lo[k] = l[k]; nd.hi[k] = h[k]; }
+        nd.pad[0] = __uint_as_float(m);
+        nd.pad[1] = 0.f;
+        base[i] = nd;
+    };
+    float l[3] = {INFINITY, INFINITY, INFINITY}, h[3] = {-INFINITY, -INFINITY, -INFINITY};
+    uint32_t m = 0xffffffffu;
+    if (slot < w) {
+        int64_t s0, s1;
+        leaf_range(lt, cl[c].lfirst, cl[c].nl, cl[c].pos + cl[c].n, j0 + slot, s0, s1);
+        for (int64_t s = s0 + (t & 3); s < s1; s += 4) {
+            if (rep != nullptr) {
+                const int32_t r = rep[s];
+                if (r >= 0 && r != (int32_t)s) continue;
+            }
+            const float4 p = pts[s];
+            l[0] = fminf(l[0], p.x); h[0] = fmaxf(h[0], p.x);
+            l[1] = fminf(l[1], p.y); h[1] = fmaxf(h[1], p.y);
+            l[2] = fminf(l[2], p.z); h[2] = fmaxf(h[2], p.z);
+            m = min(m, __float_as_uint(p.w));
         }
-        const float4 p = pts[s];
-        nd.lo[0] = fminf(nd.lo[0], p.x); nd.hi[0] = fmaxf(nd.hi[0], p.x);
-        nd.lo[1] = fminf(nd.lo[1], p.y); nd.hi[1] = fmaxf(nd.hi[1], p.y);
-        nd.lo[2] = fminf(nd.lo[2], p.z); nd.hi[2] = fmaxf(nd.hi[2], p.z);
     }
-    nodes[2 * cl[c].lbase + cl[c].L + j] = nd;
+#pragma unroll
+    for (int off = 1; off < 4; off <<= 1) {
+        for (int k = 0; k < 3; ++k) {
+            l[k] = fminf(l[k], __shfl_xor(l[k], off));
+            h[k] = fmaxf(h[k], __shfl_xor(h[k], off));
+        }
+        m = min(m, (uint32_t)__shfl_xor((int)m, off));
+    }
+    if ((t & 3) == 0 && slot < w) {
+        for (int k = 0; k < 3; ++k) { lo[k][slot] = l[k]; hi[k][slot] = h[k]; }
+        mid[slot] = m;
+        put(L + j0 + slot, l, h, m);
+    }
+    // thread t < ww holds node ((L + j0) >> lev) + t of the level
+    for (int lev = 1, ww = w / 2; ww >= 1; ++lev, ww >>= 1) {
+        __syncthreads();
+        if (t < ww) {
+            for (int k = 0; k < 3; ++k) {
+                l[k] = fminf(lo[k][2 * t], lo[k][2 * t + 1]);
+                h[k] = fmaxf(hi[k][2 * t], hi[k][2 * t + 1]);
+            }
+            m = min(mid[2 * t], mid[2 * t + 1]);
+        }
+        __syncthreads();
+        if (t < ww) {
+            for (int k = 0; k < 3; ++k) { lo[k][t] = l[k]; hi[k][t] = h[k]; }
+            mid[t] = m;
+            put(((L + j0) >> lev) + t, l, h, m);
+        }
+    }
 }
 
-// heap level [lo, 2 lo) of every cloud with more than lo leaves
-__global__ __launch_bounds__(kBlock) void k_level(Node* __restrict__ nodes, const Cloud* __restrict__ cl,
-                                                 int ncl, int64_t lo)
+// the levels above the blocks' subtrees: one block per cloud
+__global__ __launch_bounds__(1024) void k_tree_top(const Cloud* __restrict__ cl, Node* __restrict__ nodes)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)ncl * lo) return;
-    const int c = (int)(t / lo);
-    if (lo >= cl[c].L) return;
+    const int c = (int)blockIdx.x;
     Node* base = nodes + 2 * cl[c].lbase;
-    const int64_t i = lo + t % lo;
-    const Node a = base[2 * i], b = base[2 * i + 1];
-    Node nd;
-    for (int k = 0; k < 3; ++k) {
-        nd.lo[k] = fminf(a.lo[k], b.lo[k]);
-        nd.hi[k] = fmaxf(a.hi[k], b.hi[k]);
+    for (int64_t w = cl[c].L / kTreeLeaves / 2; w >= 1; w >>= 1) {
+        for (int64_t i = w + threadIdx.x; i < 2 * w; i += blockDim.x) {
+            const Node a = base[2 * i], b = base[2 * i + 1];
+            Node nd;
+            for (int k = 0; k < 3; ++k) {
+                nd.lo[k] = fminf(a.lo[k], b.lo[k]);
+                nd.hi[k] = fmaxf(a.hi[k], b.hi[k]);
+            }
+            nd.pad[0] = __uint_as_float(min(__float_as_uint(a.pad[0]), __float_as_uint(b.pad[0])));
+            nd.pad[1] = 0.f;
+            base[i] = nd;
+        }
+        __syncthreads();
     }
-    nd.pad[0] = nd.pad[1] = 0.f;
-    base[i] = nd;
 }
 
 // --------------------------------------------------------- cone search
@@ -3249,18 +3313,13 @@ struct LabelOp {
         return a == kNlabEmpty ? b : (b == kNlabEmpty ? a : (a == b ? a : kNlabMixed));
     }
 };
-struct MinOp {
-    typedef uint32_t T;
-    __device__ static uint32_t combine(uint32_t a, uint32_t b) { return min(a, b); }
-};
-
 // component label of every node: the common label of its points.  A block
 // whose kBlock leaf slots are one aligned subtree of a cloud (every block of a
 // cloud with at least kBlock slots) combines the subtree's 8 lower levels in
 // LDS, and only the subtree's root climbs with atomics: the climb of every
 // leaf through those levels was a chain of dependent atomics per level.  The
 // arrival counts of the nodes inside such a subtree are then left alone,
-// which keeps their parity for the other climbs (k_nmin_tree).
+// which keeps their parity.
 __global__ __launch_bounds__(kBlock) void k_nlab_tree(const int32_t* __restrict__ label,
                                                      const Cloud* __restrict__ cl, int ncl, int64_t nleaves,
                                                      LeafTable lt, Node* __restrict__ nodes,
@@ -3320,36 +3379,6 @@ __global__ __launch_bounds__(kBlock) void k_nlab_tree(const int32_t* __restrict_
         }
     }
     if (t == 0) climb<LabelOp>(v, store, visit + 2 * cl[c].lbase, (L + jb) / kBlock);
-}
-
-// smallest point id under every node (static per build): with ties on d2
-// broken by id, a node at the bound can only matter when it holds a smaller
-// id than the best so far (runs of coincident points)
-__global__ __launch_bounds__(kBlock) void k_nmin_tree(const float4* __restrict__ pts,
-                                                     const Cloud* __restrict__ cl, int ncl, int64_t nleaves,
-                                                     LeafTable lt, Node* __restrict__ nodes,
-                                                     unsigned long long* __restrict__ visit)
-{
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= nleaves) return;
-    const int c = find_cloud_leaf(cl, ncl, g);
-    const int64_t j = g - cl[c].lbase;
-    if (j >= cl[c].L) return;               // past the cloud's slots (one-launch capacity)
-    int64_t s0, s1;
-    leaf_range(lt, cl[c].lfirst, cl[c].nl, cl[c].pos + cl[c].n, j, s0, s1);
-    uint32_t m = 0xffffffffu;
-    int64_t s = s0;
-    for (; s + 4 <= s1; s += 4) {
-        uint32_t v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(pts[s + j].w);
-        m = min(m, min(min(v[0], v[1]), min(v[2], v[3])));
-    }
-    for (; s < s1; ++s) m = min(m, __float_as_uint(pts[s].w));
-    Node* base = nodes + 2 * cl[c].lbase;
-    auto store = [&](int64_t i, uint32_t v) { base[i].pad[0] = __uint_as_float(v); };
-    store(cl[c].L + j, m);
-    climb<MinOp>(m, store, visit + 2 * cl[c].lbase, cl[c].L + j);
 }
 
 // Per point, corr / corr_key between rounds:
@@ -5230,13 +5259,11 @@ void launch_dup_groups(const uint64_t* keys, const float4* pts, int64_t n, int32
     hipLaunchKernelGGL(k_dup_finish, dim3(1), dim3(1), 0, s, C);
 }
 
-void launch_build_tree(const float4* pts, const Cloud* cl, int ncl, int64_t nleaves, int64_t Lmax, LeafTable lt,
+void launch_build_tree(const float4* pts, const Cloud* cl, int ncl, int64_t blocks, int64_t Lmax, LeafTable lt,
                        Node* nodes, const int32_t* rep, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_leaves, dim3(nblocks(nleaves)), dim3(kBlock), 0, s, pts, cl, ncl, nleaves, lt, nodes,
-                       rep);
-    for (int64_t lo = Lmax / 2; lo >= 1; lo /= 2)
-        hipLaunchKernelGGL(k_level, dim3(nblocks((int64_t)ncl * lo)), dim3(kBlock), 0, s, nodes, cl, ncl, lo);
+    hipLaunchKernelGGL(k_tree_low, dim3((unsigned)blocks), dim3(kTreeBlock), 0, s, pts, cl, ncl, lt, nodes, rep);
+    if (Lmax > kTreeLeaves) hipLaunchKernelGGL(k_tree_top, dim3((unsigned)ncl), dim3(1024), 0, s, cl, nodes);
 }
 
 void launch_cone_search(int dim, int cdim, const float4* pts, const Node* nodes, const Cloud* cl, int ncl,
@@ -5340,14 +5367,6 @@ void launch_zero_u32(uint32_t* p, int64_t n, hipStream_t s)
     if (n > 0) hipLaunchKernelGGL(k_zero_u32, dim3(nblocks(n)), dim3(kBlock), 0, s, p, n);
 }
 
-void launch_node_min_ids(const float4* pts, const Cloud* cl, int ncl, int64_t nleaves, LeafTable lt, Node* nodes,
-                         unsigned long long* visit, hipStream_t s)
-{
-    if (nleaves <= 0) return;
-    hipLaunchKernelGGL(k_nmin_tree, dim3(nblocks(nleaves)), dim3(kBlock), 0, s, pts, cl, ncl, nleaves, lt, nodes,
-                       visit);
-}
-
 void launch_comp_seed_init(int64_t n, const float4* pts, int32_t* csize, uint32_t* cbox, hipStream_t s)
 {
     if (n <= 0) return;
@@ -5411,11 +5430,9 @@ void launch_late_search(const ConeRest& a, Node* nodes, unsigned long long* visi
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(kBlock), 0, s, &a.C->done, (int64_t)1);
     hipLaunchKernelGGL(k_zero_u32, dim3(nblocks(2 * P)), dim3(kBlock), 0, s, reinterpret_cast<uint32_t*>(sc.open_mask),
                        2 * P);
-    if (first) {
+    if (first)
         hipLaunchKernelGGL(k_zero_u32, dim3(nblocks(4 * nleaves)), dim3(kBlock), 0, s,
                            reinterpret_cast<uint32_t*>(visit), 4 * nleaves);
-        launch_node_min_ids(a.pts, a.clouds, a.ncl, nleaves, a.lt, nodes, visit, s);
-    }
     hipLaunchKernelGGL(k_nlab_tree, dim3(nblocks(nleaves)), dim3(kBlock), 0, s, a.label, a.clouds, a.ncl, nleaves,
                        a.lt, nodes, visit, (const Counters*)a.C);
     comp_dispatches(3, n, a.pts, nodes, a.clouds, a.ncl, a.bucket, a.lt, sc, (const int32_t*)a.list, &a.C->late,
