@@ -371,7 +371,7 @@ hipError_t copy_share(emst_ctx* c, const std::vector<OutSeg>& pieces, size_t chu
 // buffer runs on the calling thread, which also takes the page faults of
 // memory that the caller has just allocated: the links of 10^7 points (120 MB)
 // took 13.0 ms, now 4.8, of which 1.2 are the device's sort.
-int copy_out(emst_ctx* c, std::initializer_list<OutSeg> segs)
+int copy_out(emst_ctx* c, const std::vector<OutSeg>& segs)
 {
     size_t total = 0;
     for (const OutSeg& s : segs) total += s.dst ? s.bytes : 0;
@@ -423,6 +423,25 @@ int copy_out(emst_ctx* c, std::initializer_list<OutSeg> segs)
     for (hipError_t e : err)
         if (e != hipSuccess) return fail(c, EMST_E_HIP, std::string("copy of results: ") + hipGetErrorString(e));
     return EMST_OK;
+}
+
+// Results to a caller's buffers.  Memory that the runtime knows (pinned, or the
+// device's) takes its copy straight: a pinned slot and a memcpy between would
+// only delay it, and device memory takes no memcpy.
+int copy_results(emst_ctx* c, std::initializer_list<OutSeg> segs)
+{
+    std::vector<OutSeg> rest;
+    for (const OutSeg& s : segs) {
+        if (!s.dst || !s.bytes) continue;
+        hipPointerAttribute_t at{};
+        const bool known = hipPointerGetAttributes(&at, s.dst) == hipSuccess;
+        if (!known) (void)hipGetLastError();
+        if (known && at.type != hipMemoryTypeUnregistered)
+            HIPCHK(c, hipMemcpyAsync(s.dst, s.src, s.bytes, hipMemcpyDeviceToHost, c->stream));
+        else
+            rest.push_back(s);
+    }
+    return copy_out(c, rest);       // returns after all work queued before it
 }
 
 int read_counters(emst_ctx* c, Counters* h) { return copy_out(c, {{h, c->C, sizeof(Counters)}}); }
@@ -1422,7 +1441,7 @@ int morton_samples(emst_ctx* c, float* feat, float* target)
     launch_radius_features(c->dim, pts.p, nodes.p, cl.L, lt, n, c->feat.p, c->ls.p, s);
     launch_radius_targets(c->K, n, c->cand_key.p, ids.p, c->inv.p, c->ls.p, c->pred.p, s);
     LAUNCHCHK(c);
-    return copy_out(c, {{feat, c->feat.p, sizeof(float) * n * 8}, {target, c->pred.p, sizeof(float) * n}});
+    return copy_results(c, {{feat, c->feat.p, sizeof(float) * n * 8}, {target, c->pred.p, sizeof(float) * n}});
 }
 
 int need_points(emst_ctx* c)
@@ -1726,7 +1745,7 @@ int emst_get_cloud_results(emst_ctx* c, double* weight, int32_t* edges, int32_t*
     launch_cloud_results(c->xyz, c->dim, c->dcl.p, ncl, c->eu.p, c->ev_.p, c->eround.p, c->cloud_w.p,
                          c->cloud_e.p, c->cloud_r.p, s);
     LAUNCHCHK(c);
-    return copy_out(c, {{weight, c->cloud_w.p, sizeof(double) * ncl},
+    return copy_results(c, {{weight, c->cloud_w.p, sizeof(double) * ncl},
                         {edges, c->cloud_e.p, sizeof(int32_t) * ncl},
                         {last_round, c->cloud_r.p, sizeof(int32_t) * ncl}});
 }
@@ -1778,7 +1797,7 @@ int emst_get_edges(emst_ctx* c, int32_t* u, int32_t* v, float* d2, int64_t* m)
     launch_edges_out(second ? c->keys1.p : c->keys0.p, second ? c->vals1.p : c->vals0.p, c->ed2.p, cnt, bits, du, dv,
                      dd, s);
     LAUNCHCHK(c);
-    return copy_out(c, {{u, du, sizeof(int32_t) * cnt}, {v, dv, sizeof(int32_t) * cnt}, {d2, dd, sizeof(float) * cnt}});
+    return copy_results(c, {{u, du, sizeof(int32_t) * cnt}, {v, dv, sizeof(int32_t) * cnt}, {d2, dd, sizeof(float) * cnt}});
 }
 
 int emst_get_weight(emst_ctx* c, double* w, int64_t* size)
@@ -1843,15 +1862,15 @@ int emst_get_labels(emst_ctx* c, int32_t* labels)
     if (c->n == 0) return EMST_OK;
     launch_labels_out(c->n, c->label.p, c->pts.p, c->inv.p, c->list.p, c->stream);
     LAUNCHCHK(c);
-    return copy_out(c, {{labels, c->list.p, sizeof(int32_t) * c->n}});
+    return copy_results(c, {{labels, c->list.p, sizeof(int32_t) * c->n}});
 }
 
 int emst_get_rescaled(emst_ctx* c, float* xyz, double* unit_x)
 {
     int rc = ensure_built(c);
     if (rc) return rc;
-    return copy_out(c, {{unit_x, &c->P->unit_x, sizeof(double)},
-                        {c->n > 0 ? xyz : nullptr, c->resc.p, sizeof(float) * c->n * c->dim}});
+    return copy_results(c, {{unit_x, &c->P->unit_x, sizeof(double)},
+                            {c->n > 0 ? xyz : nullptr, c->resc.p, sizeof(float) * c->n * c->dim}});
 }
 
 int emst_get_trace(emst_ctx* c, emst_round_trace* rows, int32_t* nrows)
@@ -1882,7 +1901,7 @@ int emst_get_candidates(emst_ctx* c, int32_t* cand, float* cd2, int32_t* k)
     launch_cands_out(c->K, c->n, c->cand_key.p, c->inv.p, tc.p, td.p, c->stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(c, EMST_E_HIP, std::string("candidates: ") + hipGetErrorString(e));
-    return copy_out(c, {{cand, tc.p, sizeof(int32_t) * c->n * c->K}, {cd2, td.p, sizeof(float) * c->n * c->K}});
+    return copy_results(c, {{cand, tc.p, sizeof(int32_t) * c->n * c->K}, {cd2, td.p, sizeof(float) * c->n * c->K}});
 }
 
 int emst_get_cell_grid(emst_ctx* c, int32_t R, int32_t* ext_dual, int32_t* cell_of, int64_t* cell_start,
