@@ -3721,6 +3721,15 @@ constexpr int kSmallPacket = 8;
 // largest K-th distance after its own leaves, so they reach further
 constexpr int kKnnGatherWork = 1024;
 constexpr int kKnnGatherLeaves = 256;
+// Packets of the neighbour lists, at least: few points take fewer queries to a
+// packet, 8 at least.  2048 packets of 64 (131071 points of eight Gaussians)
+// are two waves a SIMD, and the launch takes as long as its longest packet; of
+// 32 queries each reads fewer leaves.  Runs, ms, 64 to a packet / at least
+// 2000, 4000, 8000, 16000 packets: those points 1.751 / 1.751, 1.676, 1.655,
+// 1.690; 131071 uniform ones 1.288 / 1.295, 1.273, 1.295, 1.322; 30000 of eight
+// Gaussians 1.491 / 1.420, 1.412, 1.417, 1.417; 400000 of 64 1.948 / 1.963,
+// 1.950, 1.992, 2.026; 131071 in the plane 1.203 / 1.206, 1.200, 1.213, 1.238.
+constexpr int64_t kKnnPackets = 4000;
 
 // nearest point in another component, for the points of qlist (count in
 // nq_dev): packet traversal as in the cone search, one best per query, by
@@ -4487,7 +4496,7 @@ __global__ __launch_bounds__(64) void k_knn_first(int64_t n, const float4* __res
                                                  const Node* __restrict__ nodes, const Cloud* __restrict__ clouds,
                                                  int ncl, int bucket, LeafTable lt, const int32_t* __restrict__ inv,
                                                  int32_t* __restrict__ corr, uint64_t* __restrict__ corr_key,
-                                                 NbrList nb, Counters* C, int collect)
+                                                 NbrList nb, Counters* C, int collect, int qpp)
 {
     __shared__ int32_t stk_id[64];
     __shared__ int32_t stk_ver[64];
@@ -4498,8 +4507,8 @@ __global__ __launch_bounds__(64) void k_knn_first(int64_t n, const float4* __res
     if (C->done) return;                    // a build whose input was refused on the device
     const int lane = __lane_id();
     if (blockIdx.x == 0 && lane == 0) C->knn_round1 = 1u;
-    const int64_t p = (int64_t)blockIdx.x * 64 + lane;
-    const bool active = p < n;
+    const int64_t p0 = (int64_t)blockIdx.x * qpp, p = p0 + lane;
+    const bool active = lane < qpp && p < n;
     const float4 me = pts[active ? p : 0];
     const float px = me.x, py = me.y, pz = me.z;
     const int my_cl = active ? find_cloud(clouds, ncl, p) : -1;
@@ -4612,7 +4621,7 @@ __global__ __launch_bounds__(64) void k_knn_first(int64_t n, const float4* __res
         };
         // the leaves holding the packet's points of this cloud
         const int first = (int)__builtin_ctzll(minem), last = 63 - (int)__builtin_clzll(minem);
-        const int64_t pf = (int64_t)blockIdx.x * 64 + first, pl = (int64_t)blockIdx.x * 64 + last;
+        const int64_t pf = p0 + first, pl = p0 + last;
         const int leaf_lo = (int)(L + (lt.of[pf] - lfirst)), leaf_hi = (int)(L + (lt.of[pl] - lfirst));
         for (int lf = leaf_lo; lf <= leaf_hi; ++lf) scan_own(lf);
         // gather the other leaves within the largest K-th d2 of the packet's box
@@ -4752,7 +4761,7 @@ __global__ __launch_bounds__(64) void k_knn_first(int64_t n, const float4* __res
         const int slot = blockIdx.x % kWorkSlots;
         atomicAdd(&C->work[kWorkKnnNodes][slot], (unsigned long long)st_nodes);
         atomicAdd(&C->work[kWorkKnnLeaves][slot], (unsigned long long)st_leaves);
-        atomicAdd(&C->work[kWorkKnnPairs][slot], 64ull * st_steps);
+        atomicAdd(&C->work[kWorkKnnPairs][slot], (unsigned long long)qpp * st_steps);
         atomicAdd(&C->work[kWorkKnnWalks][slot], (unsigned long long)st_walks);
     }
     if (!active) return;
@@ -5497,14 +5506,16 @@ void launch_knn_first(int dim, int64_t n, const float4* pts, const Node* nodes, 
                       const NbrList& nb, Counters* C, bool collect, hipStream_t s)
 {
     if (n <= 0) return;
-    const unsigned P = (unsigned)((n + 63) / 64);
+    int qpp = 64;
+    while (qpp > 8 && n < kKnnPackets * qpp) qpp >>= 1;
+    const unsigned P = nblocks(n, qpp);
     const int cs = collect ? 1 : 0;
     if (dim == 3)
         hipLaunchKernelGGL(k_knn_first<3>, dim3(P), dim3(64), 0, s, n, pts, nodes, cl, ncl, bucket, lt, inv, corr,
-                           corr_key, nb, C, cs);
+                           corr_key, nb, C, cs, qpp);
     else
         hipLaunchKernelGGL(k_knn_first<2>, dim3(P), dim3(64), 0, s, n, pts, nodes, cl, ncl, bucket, lt, inv, corr,
-                           corr_key, nb, C, cs);
+                           corr_key, nb, C, cs, qpp);
 }
 
 void launch_dup_fill(int dim, int64_t n, const int32_t* label, const float4* pts, const int32_t* inv,
