@@ -80,7 +80,7 @@ typedef struct {
                                (NodeSpiralSearchMD, NodeEMST.h:67-509, selected in the reference by
                                EMST_SPIRAL_SEARCH_KD_SLAB_2 0, SolutionEMST.h:55-56).  Both build
                                the same forests.  1 has no cone candidates and no 2.5D mode; it
-                               keeps each point's nearest neighbours from the build (10 in 3D, 121
+                               keeps each point's nearest neighbours from the build (8 in 3D, 97
                                bytes per point; 6 in 2D, 73 bytes), which answer the early rounds
                                without a search; its
                                learned seed predicts each component's edge length per round */
