@@ -246,14 +246,23 @@ void release(DevBuf<T>& b)
 
 // leaf cells hold a power of two of points in [8, 64] (the cone search maps
 // one leaf point per lane, 64 / bucket queries per pass of the wave).  The
-// default is the fastest measured at 10^7 points: for the cone search 16 in
-// 2D (8 cones, cheap pairs: smaller leaves cut pairs more than they add node
-// tests) and 64 in 3D; for the component search 64 in both (2D power-law:
-// 21.3 ms per EMST against 22.1 with 16).
-int choose_bucket(const emst_options& o, int dim)
+// default: 64 in 3D and for the component search (2D power-law: 21.3 ms per
+// EMST against 22.1 with 16).  The 2D cone search takes 32, with a first
+// radius of 4 spacings: its first pass drops far points 64 at a time, so
+// larger leaves cost it few pairs and save node tests, and a larger radius
+// leaves fewer queries open.  Leaves of 16 / 32 / 64, ms per run (16 with 3
+// spacings, the others with 4): 10^6 uniform points 1.82 / 1.61 / 1.57, 10^6
+// clustered 2.32 / 2.19 / 2.43, 3*10^6 power-law 5.10 / 4.37 / 4.33, 6*10^5 of
+// eight Gaussians 2.26 / 1.89 / 1.74, 2*10^5 clustered 1.37 / 1.19 / 1.17, 10^4
+// 0.74 / 0.69 / 0.67; 32 with 3 spacings 1.68, 2.14, 4.57, 2.39, 1.21, 0.70.
+// The 2D seed models and their samples describe leaves of 16.
+constexpr int kModelBucket2D = 16;
+constexpr float kConeSeedScale2D = 4.0f;
+
+int choose_bucket(const emst_options& o, int dim, bool learned)
 {
     int b = o.bucket_size;
-    if (b <= 0) b = dim == 2 && o.round_search != 1 ? 16 : 64;
+    if (b <= 0) b = dim == 2 && o.round_search != 1 ? (learned ? kModelBucket2D : 32) : 64;
     int r = 8;
     while (r < b && r < 64) r <<= 1;
     return r;
@@ -505,6 +514,14 @@ int layout_clouds(emst_ctx* c, int bucket)
     c->P = c->params.p;
     HIPCHK(c, hipMemcpyAsync(c->dcl.p, c->hcl.data(), sizeof(Cloud) * c->ncl, hipMemcpyHostToDevice, c->stream));
     return EMST_OK;
+}
+
+// a seed model came or went: the leaves that it describes, for points already set
+int relayout(emst_ctx* c)
+{
+    if (!c->have_points) return EMST_OK;
+    const int b = choose_bucket(c->opt, c->dim, c->learned);
+    return b == c->bucket ? EMST_OK : layout_clouds(c, b);
 }
 
 LeafTable leaf_table(const emst_ctx* c) { return LeafTable{c->lstart.p, c->leaf_of.p}; }
@@ -1410,13 +1427,14 @@ int morton_samples(emst_ctx* c, float* feat, float* target)
         (rc = ensure(c, c->feat, (size_t)n * 8)) || (rc = ensure(c, c->pred, (size_t)n)) ||
         (rc = ensure(c, c->ls, (size_t)n)))
         return rc;
+    const int bucket = choose_bucket(c->opt, c->dim, true);
     Cloud cl = c->hcl[0];
     HIPCHK(c, hipMemcpyAsync(dcl.p, &cl, sizeof(Cloud), hipMemcpyHostToDevice, s));
     launch_zero_u32(reinterpret_cast<uint32_t*>(cnt.p), sizeof(Counters) / sizeof(uint32_t), s);
     launch_rescale_keys(c->xyz, dcl.p, 1, n, c->dim, c->mbits, c->P, c->resc.p, keys0.p, false, s);
     radix_sort(keys0.p, vals0.p, keys1.p, vals1.p, n, sort_key_bits(c), true, c->hist.p, s);
     launch_gather_sorted(c->resc.p, vals0.p, n, c->dim, pts.p, inv.p, ids.p, s);
-    launch_leaves(keys0.p, n, dcl.p, 1, c->bucket, vals1.p, reinterpret_cast<uint32_t*>(keys1.p), c->scan_tmp.p,
+    launch_leaves(keys0.p, n, dcl.p, 1, bucket, vals1.p, reinterpret_cast<uint32_t*>(keys1.p), c->scan_tmp.p,
                   lstart.p, leaf_of.p, cloud_lf.p, c->P, cnt.p, false, s);
     LAUNCHCHK(c);
     int32_t lf[2] = {0, 0};
@@ -1547,6 +1565,8 @@ emst_ctx* emst_create(const emst_options* opt)
         c->seed_scale = o.seed_scale;
     else if (o.round_search == 1 && o.dim == 3)
         c->seed_scale = kCompSeedScale3D;
+    else if (o.round_search == 0 && o.dim == 2)
+        c->seed_scale = kConeSeedScale2D;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         g_create_error = "hipStreamCreate failed";
         delete c;
@@ -1605,7 +1625,7 @@ int emst_set_clouds(emst_ctx* c, int32_t ncl, const int64_t* npts, const float* 
     c->ncl = ncl;
     c->hcl.assign(ncl, Cloud{});
     for (int32_t k = 0; k < ncl; ++k) c->hcl[k].n = npts[k];
-    int rc = layout_clouds(c, choose_bucket(c->opt, dim));
+    int rc = layout_clouds(c, choose_bucket(c->opt, dim, c->learned));
     if (rc) return rc;
     if (on_device) {
         c->xyz = xyz;
@@ -2022,7 +2042,7 @@ int emst_set_radius_model(emst_ctx* c, const float* model)
     if (!model) {
         c->learned = false;
         c->built = false;
-        return EMST_OK;
+        return relayout(c);
     }
     if (c->opt.cone_dim == 2 && c->opt.dim == 3)
         return fail(c, EMST_E_ARG, "the learned seed radius is not defined for the 2.5D mode");
@@ -2032,7 +2052,7 @@ int emst_set_radius_model(emst_ctx* c, const float* model)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->learned = true;
     c->built = false;       // the next run searches with the new seeds
-    return EMST_OK;
+    return relayout(c);
 }
 
 int emst_get_radius_samples(emst_ctx* c, float* feat, float* target, int64_t* m)

@@ -49,12 +49,14 @@ typedef struct {
     int32_t level_radius;   /* R of the reference cell grid (levelRadius); cells are 2R wide */
     int32_t max_rounds;     /* Boruvka round cap; the reference stops at 100 */
     int32_t bucket_size;    /* points per leaf cell of the search hierarchy: a power of two in
-                               [8, 64], rounded up (0 = 16 for the 2D cone search, else 64) */
+                               [8, 64], rounded up (0 = 32 for the 2D cone search, 16 with a
+                               seed model and for its samples, else 64) */
     int32_t trace;          /* 1: record per-round forest size, length and phase times */
     int32_t device;         /* HIP device ordinal */
     int32_t radius_mode;    /* 0 plain; 1 learned seed radius (needs emst_set_radius_model) */
     float seed_scale;       /* plain-form first search radius, in mean spacings of the point's
-                               leaf cell (0 = default: 3.0, 1.0 for the 3D component search);
+                               leaf cell (0 = default: 3.0, 4.0 for the 2D cone search, 1.0 for
+                               the 3D component search);
                                changes work, never results */
     int32_t cone_dim;       /* dimension of the cones (DimCM): 0 = the point dimension; 2 with
                                3D points is the 2.5D mode, SolutionEMST<3,2>
