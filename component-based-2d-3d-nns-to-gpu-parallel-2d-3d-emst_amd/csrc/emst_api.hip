@@ -734,8 +734,9 @@ int search_cones(emst_ctx* c, bool first)
     // launch: the search then takes as long as its longest packet, and two
     // launches have two of those.  One launch against two, ms (seed 3.5): 3D
     // uniform 1.37 / 0.98 at 2*10^5 points and 2.22 / 1.55 at 4*10^5,
-    // clustered 2.95 / 3.57 and 3.84 / 3.58; 2D uniform 0.33 / 0.37 and
-    // 0.48 / 0.42, clustered 0.67 / 0.80 and 0.85 / 0.89.
+    // clustered 2.95 / 3.57 and 3.84 / 3.58; whole 2D runs, uniform 0.88 / 0.92
+    // and 1.16 / 1.12 at 4.5*10^5, 1.45 / 1.35 at 7*10^5, clustered 1.19 / 1.39,
+    // 1.46 / 1.63 and 1.80 / 1.94, of eight Gaussians 1.74 / 1.59 at 4.5*10^5.
     SplitScratch split{};
     split.open_mask = c->open_mask.p;
     split.cnt = c->open_cnt.p;
@@ -895,8 +896,8 @@ int build(emst_ctx* c, bool all_cones)
     // Late cones (k_late_mark) in 3D, where most of the search's time goes to
     // cones that no round asks for: not where points coincide (their groups
     // share cones), and 2D cones cost less than the rounds that ask for them
-    // (10^6 uniform points 1.85 ms a run without, 1.80 with, 3*10^5 clustered
-    // ones 1.37 and 2.8).  3D, without / with, ms a run: uniform 10^4 0.69 /
+    // (leaves of 16: 10^6 uniform points 1.85 ms a run without, 1.80 with, 3*10^5
+    // clustered ones 1.37 and 2.8).  3D, without / with, ms a run: uniform 10^4 0.69 /
     // 0.58, 2*10^5 2.10 / 1.03, 10^6 4.3 / 2.1; clustered 10^4 1.22 / 1.06,
     // 5*10^4 2.03 / 1.96, 2*10^5 3.6 / 2.2, 10^6 6.7 / 4.8, 4*10^6 16.7 /
     // 10.1, with a seed model 17.6 / 11.3.
