@@ -274,6 +274,18 @@ struct ConeRest {
     Counters* C;
 };
 enum { kRestRound, kRestCheck };        // k_cone_rest: a point's cones, or the check of its target
+constexpr int32_t kReachAll = 0x7fffffff;       // every cone of the point is exact
+// The smallest d2 (bits) that a candidate unknown so far can have for a late
+// point whose exact candidates have all joined its component: its cones are
+// exact up to and with `reach` (bits; -1: none of them), and an earlier search
+// found no candidate beyond the reach nearer than `lo` (bits; all ones: none
+// made).  One at just that d2 may exist, and at the component's edge its ids
+// may be the smaller ones, so the point is asked while this is <= the edge.
+__host__ __device__ inline uint32_t late_least(int32_t reach, uint32_t lo)
+{
+    const uint32_t past = (uint32_t)(reach + 1);
+    return lo == 0xffffffffu || lo < past ? past : lo;
+}
 void launch_late_cones(const ConeRest& a, hipStream_t s);
 void launch_late_search(const ConeRest& a, Node* nodes, unsigned long long* visit, int64_t nleaves, bool first,
                         float seed_scale, const SplitScratch& sc, hipStream_t s);

@@ -1382,7 +1382,6 @@ __device__ __forceinline__ int32_t key_bound(unsigned long long k)
 }
 
 constexpr int kMaxCappedPasses = 6;
-constexpr int32_t kReachAll = 0x7fffffff;       // every cone of the point is exact
 // packets of a cone search, at least (launch_cone_search), and the resumed
 // queries up to which their packets take kConeFewPacket each
 constexpr int64_t kConePackets = 2500;
@@ -2828,9 +2827,10 @@ __device__ __forceinline__ uint64_t edge_key1(uint64_t ck, uint32_t pid)
 // of R_0^2; -1: none is known; kReachAll: all are exact), and only the exact
 // ones are ranked.  The rounds go on without the rest: a late point matters
 // only in a round in which every exact candidate of its has joined its
-// component while the component's smallest edge is beyond what the point has
-// seen (its reach, or the nearest outside point that an earlier round found,
-// corr_key).  Those points are listed here, after the round's minima.  Few of
+// component while an unknown one could be as near as the component's smallest
+// edge (late_least, from its reach and the nearest outside point beyond it
+// that an earlier round found, corr_key): equal d2 counts, since the ids
+// decide.  Those points are listed here, after the round's minima.  Few of
 // them get their cones searched to the end (k_cone_rest).  More of them pause
 // the round, and their nearest points outside the component are searched
 // instead (launch_late_search).
@@ -2857,12 +2857,10 @@ __global__ __launch_bounds__(kBlock) void k_late_mark(int64_t n, const int32_t* 
         if (p < n && corr[p] == -2) {
             const int32_t r = reach[p];
             if (r != kReachAll) {
-                // no outside point's d2 is below `seen`
-                const uint32_t lo = (uint32_t)(corr_key[p] >> 32);
-                const int32_t seen = max(r, lo == 0xffffffffu ? -1 : (int32_t)lo);
-                const uint32_t edge = (uint32_t)(comp1[label[p]] >> 32);
-                need = seen < 0 || edge > (uint32_t)seen;
-                if (need && seen >= 0) corr_key[p] = ((uint64_t)(uint32_t)seen << 32) | 0xffffffffull;
+                const uint32_t least = late_least(r, (uint32_t)(corr_key[p] >> 32));
+                need = least <= (uint32_t)(comp1[label[p]] >> 32);
+                // (the paused search starts there)
+                if (need && least > 0u) corr_key[p] = ((uint64_t)least << 32) | 0xffffffffull;
             }
         }
         const uint64_t m = __ballot(need);
