@@ -3738,7 +3738,11 @@ constexpr int64_t kKnnPackets = 4000;
 // each pass) also bounds the search: a point whose nearest outside point lies
 // beyond it cannot hold the component's edge, and it stops with that d2 as
 // its lower bound (corr = -1).  Exact results enter comp1 as they close.
-template <int D, int BK, bool SAMPLE>
+//
+// LATE: the queries are late points of the cone form (launch_late_search).
+// Their first lower bound is that of their unknown candidates (late_least):
+// points outside their component do lie within it, hidden from their cones.
+template <int D, int BK, bool SAMPLE, bool LATE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_comp_search(
     const float4* __restrict__ pts, const Node* __restrict__ nodes,
     const Cloud* __restrict__ clouds, int ncl, int bucket_rt, LeafTable lt, const int32_t* __restrict__ qlist,
@@ -3840,6 +3844,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                 }
                 if (!positive_finite(r)) r = 1e-6f;
             }
+            const int32_t from = inner;
             float r2 = r * r;
             // a launch that resumes at pass_lo: the state the earlier passes left
             for (int k = 0; k < pass_lo; ++k) {
@@ -3968,6 +3973,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                     float qlo[3] = {open ? px : INFINITY, open ? py : INFINITY, open ? pz : INFINITY};
                     float qhi[3] = {open ? px : -INFINITY, open ? py : -INFINITY, open ? pz : -INFINITY};
                     int32_t imin = open ? inner : 0x7fffffff;
+                    int32_t fmost = open ? from : -1;
                     for (int off = 32; off > 0; off >>= 1) {
     #pragma unroll
                         for (int k = 0; k < 3; ++k) {
@@ -3975,6 +3981,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                             qhi[k] = fmaxf(qhi[k], __shfl_xor(qhi[k], off));
                         }
                         imin = min(imin, __shfl_xor(imin, off));
+                        if (LATE) fmost = max(fmost, __shfl_xor(fmost, off));
                     }
                     const int fo = (int)__builtin_ctzll(__ballot(open));
                     const int32_t lab0 = __builtin_amdgcn_readfirstlane(__shfl(mylab, fo));
@@ -4011,8 +4018,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
                             // Without it a pass whose radius first reaches a far
                             // cluster gathered most of that cluster, outgrew its
                             // lists and walked (512 clouds of eight Gaussians:
-                            // 153000 -> 34000 walks per run)
-                            if (pass_ && (xl == kNlabMixed || one_lab)) ub = __float_as_uint(far);
+                            // 153000 -> 34000 walks per run).  (Late points:
+                            // a node beyond all of their first bounds, so that
+                            // its points are not hidden ones)
+                            if (pass_ && (xl == kNlabMixed || one_lab) && (!LATE || (int32_t)bd > fmost))
+                                ub = __float_as_uint(far);
                         }
                         B = min(B, wave_min_u32(ub));
                         pass_ = pass_ && bd <= B;
@@ -4211,7 +4221,7 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v)
     return v;
 }
 
-template <int D>
+template <int D, bool LATE>
 __global__ __launch_bounds__(64 * kDeferWaves) void k_comp_search_deferred(
     const float4* __restrict__ pts, const Node* __restrict__ nodes, const Cloud* __restrict__ clouds, int ncl,
     LeafTable lt, const uint64_t* __restrict__ defer, const int32_t* __restrict__ label,
@@ -4271,6 +4281,7 @@ __global__ __launch_bounds__(64 * kDeferWaves) void k_comp_search_deferred(
             }
             if (!positive_finite(r)) r = 1e-6f;
         }
+        const int32_t from = inner;
         float r2 = r * r;
         for (int k = 0; k < pass0; ++k) {
             inner = max(inner, (int32_t)__float_as_uint(r2));
@@ -4357,7 +4368,8 @@ __global__ __launch_bounds__(64 * kDeferWaves) void k_comp_search_deferred(
                         bd = __float_as_uint(box_d2(x, far));
                         leaf = nd >= L;
                         pass_ = xl != kNlabEmpty && xl != mylab && bd <= B && (int32_t)__float_as_uint(far) > inner;
-                        if (pass_) ub = __float_as_uint(far);       // it holds a point outside
+                        // it holds a point outside (late points: none of the hidden ones)
+                        if (pass_ && (!LATE || (int32_t)bd > from)) ub = __float_as_uint(far);
                     }
                     B = min(B, wave_min_u32(ub));
                     pass_ = pass_ && bd <= B;
@@ -5380,7 +5392,9 @@ void launch_comp_seed_init(int64_t n, const float4* pts, int32_t* csize, uint32_
     hipLaunchKernelGGL(k_comp_seed_init, dim3(nblocks(n)), dim3(kBlock), 0, s, n, pts, csize, cbox);
 }
 
-// the component search's dispatches over a list of points (nq of them)
+// the component search's dispatches over a list of points (nq of them); LATE:
+// late points of the cone form (3D)
+template <bool LATE>
 static void comp_dispatches(int dim, int64_t n, const float4* pts, const Node* nodes, const Cloud* cl, int ncl,
                             int bucket, LeafTable lt, const SplitScratch& sc, const int32_t* list,
                             const uint32_t* nq, const int32_t* label, int32_t* corr, uint64_t* corr_key,
@@ -5388,15 +5402,15 @@ static void comp_dispatches(int dim, int64_t n, const float4* pts, const Node* n
                             hipStream_t s, hipEvent_t* ev)
 {
     const int64_t P = (n + 63) / 64;
-    auto kern = dim == 3 ? (bucket == 64 ? k_comp_search<3, 64, false> : k_comp_search<3, 0, false>)
-                         : (bucket == 16 ? k_comp_search<2, 16, false> : k_comp_search<2, 0, false>);
+    auto kern = dim == 3 ? (bucket == 64 ? k_comp_search<3, 64, false, LATE> : k_comp_search<3, 0, false, LATE>)
+                         : (bucket == 16 ? k_comp_search<2, 16, false, false> : k_comp_search<2, 0, false, false>);
     // (2D at its default 64-point leaves runs the runtime-size instance: a
     // <2, 64> instance measured 7% slower on the 2D power-law cloud)
     // pass 0 over the searching points; their open packets' lanes into open_mask
     if (ev) (void)hipEventRecord(ev[0], s);
     if (dim == 3 && n >= kSampleMin) {
         const int64_t gs = std::min<int64_t>((P + kSampleStep - 1) / kSampleStep, kSampleBlocks);
-        hipLaunchKernelGGL((k_comp_search<3, 0, true>), dim3((unsigned)gs), dim3(64), 0, s, pts, nodes, cl, ncl, bucket,
+        hipLaunchKernelGGL((k_comp_search<3, 0, true, LATE>), dim3((unsigned)gs), dim3(64), 0, s, pts, nodes, cl, ncl, bucket,
                            lt, list, nq, label, inv, seed_scale, corr, corr_key, comp1, 0, kMaxCappedPasses,
                            (uint64_t*)nullptr, seed_r, (uint64_t*)nullptr, C, 0);
     }
@@ -5414,7 +5428,7 @@ static void comp_dispatches(int dim, int64_t n, const float4* pts, const Node* n
                        ev != nullptr ? 1 : 0);
     // the queries the packets handed over, one wave each
     if (sc.defer != nullptr) {
-        auto dk = dim == 3 ? k_comp_search_deferred<3> : k_comp_search_deferred<2>;
+        auto dk = dim == 3 ? k_comp_search_deferred<3, LATE> : k_comp_search_deferred<2, false>;
         hipLaunchKernelGGL(dk, dim3(kDeferBlocks), dim3(64 * kDeferWaves), 0, s, pts, nodes, cl, ncl, lt,
                            (const uint64_t*)sc.defer, label, inv, seed_scale, corr, corr_key, comp1, seed_r, C,
                            ev != nullptr ? 1 : 0);
@@ -5442,7 +5456,7 @@ void launch_late_search(const ConeRest& a, Node* nodes, unsigned long long* visi
                            reinterpret_cast<uint32_t*>(visit), 4 * nleaves);
     hipLaunchKernelGGL(k_nlab_tree, dim3(nblocks(nleaves)), dim3(kBlock), 0, s, a.label, a.clouds, a.ncl, nleaves,
                        a.lt, nodes, visit, (const Counters*)a.C);
-    comp_dispatches(3, n, a.pts, nodes, a.clouds, a.ncl, a.bucket, a.lt, sc, (const int32_t*)a.list, &a.C->late,
+    comp_dispatches<true>(3, n, a.pts, nodes, a.clouds, a.ncl, a.bucket, a.lt, sc, (const int32_t*)a.list, &a.C->late,
                     a.label, a.corr, a.corr_key, a.comp1, a.inv, seed_scale, nullptr, a.C, s, nullptr);
     hipLaunchKernelGGL(k_late_settle, dim3(nblocks(n)), dim3(kBlock), 0, s, (const int32_t*)a.list, a.ids, a.label,
                        a.corr, (const uint64_t*)a.corr_key, (const uint64_t*)a.comp1, sc.list2, a.C);
@@ -5489,7 +5503,7 @@ void launch_comp_round(int dim, int64_t n, const float4* pts, const uint32_t* id
             seed_r = cs.R;
         }
     }
-    comp_dispatches(dim, n, pts, nodes, cl, ncl, bucket, lt, sc, (const int32_t*)sc.list, nq, label, corr, corr_key,
+    comp_dispatches<false>(dim, n, pts, nodes, cl, ncl, bucket, lt, sc, (const int32_t*)sc.list, nq, label, corr, corr_key,
                     comp1, inv, seed_scale, seed_r, C, s, ev);
     // comp1 now holds every component's edge: the sample log of this round
     if (cs.features_on && cs.samples != nullptr)
