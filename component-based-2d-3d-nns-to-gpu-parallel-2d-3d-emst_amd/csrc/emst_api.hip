@@ -695,6 +695,13 @@ NbrList nbr_list(emst_ctx* c)
 // 0.59, 2048 0.52 / 0.51, clustered 4000 0.86 / 0.81, 2048 0.60 / 0.68.)
 constexpr float kLateSeed = 0.5f, kLateLearned = 0.35f;
 constexpr int64_t kLateMin = 1 << 12;
+// Where more than this share of the points is late and has no candidate at all
+// (1 / kLateBlind; 1 / kLateBlindLearned of them with a model), the first radius
+// is not one of this cloud's spacings, and the rounds would search for nearly
+// all of its points: every cone first, then.  Late / given up, ms a run: a
+// lidar sweep's rings of 30000 points (71% of them) 2.83 / 1.75, a line of 5820 (8%)
+// 1.00 / 0.88; 5*10^5 clustered points (5%) 3.71 / 5.87.
+constexpr int64_t kLateBlind = 16, kLateBlindLearned = 4;
 
 ConeRest cone_rest(emst_ctx* c)
 {
@@ -906,24 +913,31 @@ int build(emst_ctx* c, bool all_cones)
     c->late_tree = false;
     int rc4;
     if (c->late && (rc4 = ensure(c, c->reach, (size_t)n))) return rc4;
-    if ((rc4 = search_cones(c, true))) return rc4;
-    launch_dup_fill(c->cdim, n, c->label.p, c->pts.p, c->inv.p, c->cand_key.p, c->cand_pos.p, nullptr, c->corr.p,
-                    c->corr_key.p, c->C, dup, s);
-    launch_rank_cones(c->cdim, n, c->cand_key.p, c->cand_pos.p, nullptr, n, c->rkey.p, c->rpos.p, c->cursor.p,
-                      c->late ? c->reach.p : nullptr, nullptr, s);
-    LAUNCHCHK(c);
-    // while grouping is on only group points can hold a zero-distance or no
-    // candidate, and k_dup_fill refreshes those; the queue serves the
-    // per-point form
-    // (a point's smallest cone key, which the search leaves as round 1's, is at
-    // distance zero or empty exactly when some cone is: one key a point is
-    // read instead of K, 0.16 -> 0.01 ms at 4*10^6 3D points)
-    if (!c->grouped) launch_flag_research(1, n, c->corr_key.p, c->list.p, c->late ? c->reach.p : nullptr, c->C, s);
-    LAUNCHCHK(c);
-    HIPCHK(c, hipEventRecord(c->ev[3], s));
     Counters h{};
-    int rc = read_counters(c, &h);
-    if (rc) return rc;
+    for (;;) {
+        if ((rc4 = search_cones(c, true))) return rc4;
+        launch_dup_fill(c->cdim, n, c->label.p, c->pts.p, c->inv.p, c->cand_key.p, c->cand_pos.p, nullptr, c->corr.p,
+                        c->corr_key.p, c->C, dup, s);
+        launch_rank_cones(c->cdim, n, c->cand_key.p, c->cand_pos.p, nullptr, n, c->rkey.p, c->rpos.p, c->cursor.p,
+                          c->late ? c->reach.p : nullptr, nullptr, s);
+        LAUNCHCHK(c);
+        // while grouping is on only group points can hold a zero-distance or no
+        // candidate, and k_dup_fill refreshes those; the queue serves the
+        // per-point form
+        // (a point's smallest cone key, which the search leaves as round 1's, is at
+        // distance zero or empty exactly when some cone is: one key a point is
+        // read instead of K, 0.16 -> 0.01 ms at 4*10^6 3D points)
+        if (!c->grouped) launch_flag_research(1, n, c->corr_key.p, c->list.p, c->late ? c->reach.p : nullptr, c->C, s);
+        LAUNCHCHK(c);
+        HIPCHK(c, hipEventRecord(c->ev[3], s));
+        if ((rc4 = read_counters(c, &h))) return rc4;
+        if (!c->late || work_total(h, kWorkBlind) * (c->seed_r ? kLateBlindLearned : kLateBlind) <= n) break;
+        // too many points have seen no other: every cone first
+        c->late = false;
+        launch_zero_u32(&c->C->research, 2, s);
+        launch_zero_u32(reinterpret_cast<uint32_t*>(c->C->work[kWorkConePackets]),
+                        2 * (int64_t)(kWorkKinds - kWorkConePackets) * kWorkSlots, s);
+    }
     if (c->grouped && h.underflow) {
         // distinct points at float distance 0: the groups would merge
         // candidates that the per-point rule keeps apart; search ungrouped

@@ -27,7 +27,9 @@ enum {
     kWorkCompWalks, kWorkKnnWalks,
     // the last full cone search: packets, node-test steps, leaves entered,
     // leaf points read per packet, point pairs
-    kWorkConePackets, kWorkConeNodes, kWorkConeLeaves, kWorkConePoints, kWorkConePairs, kWorkKinds
+    kWorkConePackets, kWorkConeNodes, kWorkConeLeaves, kWorkConePoints, kWorkConePairs,
+    kWorkBlind,             // late points without any candidate after the first pass
+    kWorkKinds
 };
 constexpr int kWorkCompKinds = kWorkConePackets;    // the component search's kinds come first
 
