@@ -153,7 +153,8 @@ struct emst_ctx {
     DevBuf<int32_t> reach;              // late cones (k_late_mark)
     bool late = false;                  // points may hold late cones
     bool no_late = false;               // a choice of theirs failed its check: exact cones
-    bool late_tree = false;             // this build's nodes hold their smallest ids
+    bool late_visit = false;            // visit has been cleared for this build's hierarchy
+    bool cones_full = false;            // late, but this build's cone candidates are all exact (full_cones)
     const float* seed_r = nullptr;      // the build's learned seeds
     DevBuf<Params> params;
     DevBuf<double> cloud_w;
@@ -730,8 +731,9 @@ ConeRest cone_rest(emst_ctx* c)
     return a;
 }
 
-// The cone search over every point.  first: writes round 1's targets.
-int search_cones(emst_ctx* c, bool first)
+// The cone search over every point.  first: writes round 1's targets; late:
+// leaves late cones.
+int search_cones(emst_ctx* c, bool first, bool late)
 {
     const int64_t n = c->n;
     hipStream_t s = c->stream;
@@ -753,43 +755,53 @@ int search_cones(emst_ctx* c, bool first)
     const int mode = c->opt.search_split;
     split.compact_frac = mode == 2 ? -1.0 : 1.0;
     const bool many = c->cdim == c->dim && n >= ((int64_t)1 << (c->dim == 3 ? 18 : 19));
-    const bool use_split = c->late || mode == 2 || mode == 3 || (mode == 0 && many);
+    const bool use_split = late || mode == 2 || mode == 3 || (mode == 0 && many);
     launch_cone_search(c->dim, c->cdim, c->pts.p, c->nodes.p, c->dcl.p, c->ncl, c->bucket, leaf_table(c), n, nullptr,
                        n, c->label.p, false, c->inv.p, c->seed_r, c->seed_scale,
-                       !c->late ? 1.f : c->seed_r ? kLateLearned : kLateSeed, c->cand_key.p, c->cand_pos.p, nullptr,
+                       !late ? 1.f : c->seed_r ? kLateLearned : kLateSeed, c->cand_key.p, c->cand_pos.p, nullptr,
                        first ? c->corr.p : nullptr, first ? c->corr_key.p : nullptr, c->C, true, dup_state(c),
-                       use_split ? &split : nullptr, c->late ? c->reach.p : nullptr, s);
+                       use_split ? &split : nullptr, late ? c->reach.p : nullptr, s);
     LAUNCHCHK(c);
     HIPCHK(c, hipEventRecord(c->ev[2], s));
     // read with the counters (into the context, which outlives any early
     // return while the copy is queued)
     c->resumed_h = 0;
-    if (use_split && !c->late && n > 0)
+    if (use_split && !late && n > 0)
         HIPCHK(c, hipMemcpyAsync(&c->resumed_h, split.off + (n + 63) / 64, sizeof(uint32_t), hipMemcpyDeviceToHost,
                                  s));
     return EMST_OK;
 }
 
-// Every cone exact, for callers that read them, count their search or repeat
-// it: the search again from full seeds (going on from the late points' small
-// radius instead tests twice as many nodes).
-int complete_cones(emst_ctx* c)
+// Every cone exact, for callers that read the cones or count their search: the
+// search again from full seeds (going on from the late points' small radius
+// instead tests twice as many nodes).  The rounds' state (ranked cones,
+// targets, reach) stays as it is: a run goes on as it would have.
+int full_cones(emst_ctx* c)
 {
-    if (!c->late) return EMST_OK;
+    if (!c->late || c->cones_full) return EMST_OK;
     hipStream_t s = c->stream;
-    c->late = false;
     launch_zero_u32(reinterpret_cast<uint32_t*>(c->C->work[kWorkConePackets]),
                     2 * (int64_t)(kWorkKinds - kWorkConePackets) * kWorkSlots, s);
-    int rc = search_cones(c, false);
+    int rc = search_cones(c, false, false);
     if (rc) return rc;
-    launch_rank_cones(c->cdim, c->n, c->cand_key.p, c->cand_pos.p, nullptr, c->n, c->rkey.p, c->rpos.p, c->cursor.p,
-                      nullptr, nullptr, s);
-    launch_revive(c->n, c->corr.p, s);
-    LAUNCHCHK(c);
     Counters h{};
     if ((rc = read_counters(c, &h))) return rc;
     for (int k = 0; k < 5; ++k) c->stats[k] = work_total(h, kWorkConePackets + k);
     c->stats[8] = c->resumed_h;
+    c->cones_full = true;
+    return EMST_OK;
+}
+
+// Every cone exact for the rounds too, before the first one.
+int complete_cones(emst_ctx* c)
+{
+    const int rc = full_cones(c);
+    if (rc || !c->late) return rc;
+    c->late = false;
+    launch_rank_cones(c->cdim, c->n, c->cand_key.p, c->cand_pos.p, nullptr, c->n, c->rkey.p, c->rpos.p, c->cursor.p,
+                      nullptr, nullptr, c->stream);
+    launch_revive(c->n, c->corr.p, c->stream);
+    LAUNCHCHK(c);
     return EMST_OK;
 }
 
@@ -910,12 +922,12 @@ int build(emst_ctx* c, bool all_cones)
     // 10.1, with a seed model 17.6 / 11.3.
     c->late = !all_cones && !c->no_late && c->opt.search_split == 0 && c->ncl == 1 && c->cdim == 3 && n >= kLateMin &&
               !any_dup;
-    c->late_tree = false;
+    c->late_visit = c->cones_full = false;
     int rc4;
     if (c->late && (rc4 = ensure(c, c->reach, (size_t)n))) return rc4;
     Counters h{};
     for (;;) {
-        if ((rc4 = search_cones(c, true))) return rc4;
+        if ((rc4 = search_cones(c, true, c->late))) return rc4;
         launch_dup_fill(c->cdim, n, c->label.p, c->pts.p, c->inv.p, c->cand_key.p, c->cand_pos.p, nullptr, c->corr.p,
                         c->corr_key.p, c->C, dup, s);
         launch_rank_cones(c->cdim, n, c->cand_key.p, c->cand_pos.p, nullptr, n, c->rkey.p, c->rpos.p, c->cursor.p,
@@ -987,11 +999,11 @@ constexpr int kOneLaunchRounds = 16;
 // The kernels of one Boruvka round (SolutionEMST::activate).  Round control
 // lives on the device (k_round_begin / k_round_end), so a round issued after
 // the run has finished does nothing.  trace: events after each phase.
-void issue_round(emst_ctx* c, bool tr, unsigned long long* stamps = nullptr, bool begin = true)
+void issue_round(emst_ctx* c, bool tr, unsigned long long* stamps = nullptr)
 {
     hipStream_t s = c->stream;
-    if (begin) launch_round_begin(c->C, s);
-    if (begin && tr) (void)hipEventRecord(c->ev[3], s);
+    launch_round_begin(c->C, s);
+    if (tr) (void)hipEventRecord(c->ev[3], s);
     // group points: zero-distance '+' cones while the group spans several
     // components, the representative's own cones once it is one (the
     // repeated search of NodeEMST.h:1051-1077, without searching again); the
@@ -1054,9 +1066,9 @@ int resume_late(emst_ctx* c, Counters* h)
     if ((rc = ensure(c, c->list2, (size_t)c->n)) || (rc = ensure(c, c->defer, (size_t)c->n)) ||
         (rc = ensure(c, c->visit, 2 * (size_t)c->nleaves)))
         return rc;
-    launch_late_search(cone_rest(c), c->nodes.p, c->visit.p, c->nleaves, !c->late_tree,
+    launch_late_search(cone_rest(c), c->nodes.p, c->visit.p, c->nleaves, !c->late_visit,
                        kCompSeedScale3D, split_scratch(c), s);
-    c->late_tree = true;
+    c->late_visit = true;
     const bool tr = c->opt.trace != 0;
     if (tr) HIPCHK(c, hipEventRecord(c->ev[4], s));
     const CycleState cy = cycle_state(c);
@@ -1490,7 +1502,7 @@ int ensure_built(emst_ctx* c, bool cones = false)
     int rc = need_points(c);
     if (rc) return rc;
     if (!c->built) return build(c, cones);
-    return cones ? complete_cones(c) : EMST_OK;
+    return cones ? full_cones(c) : EMST_OK;
 }
 
 // The rounds of a built context, to the end; times[2] = their device time.
@@ -2110,7 +2122,7 @@ int emst_get_search_stats(emst_ctx* c, int64_t* stats, int32_t* n_stats)
     if (!c || !stats || !n_stats) return EMST_E_ARG;
     if (c->built && c->late) {
         HIPCHK(c, hipSetDevice(c->opt.device));
-        const int rc = complete_cones(c);
+        const int rc = full_cones(c);
         if (rc) return rc;
     }
     const int32_t k = std::min<int32_t>(*n_stats, 18);

@@ -262,9 +262,9 @@ int emst_get_times(emst_ctx* ctx, float* times, int32_t* n_times);
  * counterpart in the reference. */
 int emst_get_round_ends(emst_ctx* ctx, float* ms, int32_t* n);
 
-/* Counters of the last full cone search (the work behind its bytes; a run that
- * left cones to its rounds, see emst_options.search_split, makes that search
- * here):
+/* Counters of the last full cone search (the work behind its bytes; for a run
+ * that left cones to its rounds, see emst_options.search_split, that search is
+ * made here, once, beside the run, which goes on as it would have):
  * [0] packets (waves of at most 64 queries), [1] node-test steps (a hierarchy
  * node against a packet's queries, or up to 64 nodes against the packet's
  * box), [2] leaf cells entered, [3] leaf points read (summed over packets), [4] point pairs
