@@ -246,7 +246,8 @@ int emst_get_cell_grid(emst_ctx* ctx, int32_t level_radius, int32_t* ext_dual,
 /* Kernel times of the last emst_run (ms, device events on the context's
  * stream): [0] build (bbox, rescale, sort, hierarchy, coincident groups, the
  * learned seed's features and inference when set, and the candidates ranked
- * for the rounds), [1] round-1 cone search, [2] Boruvka rounds, [3] total,
+ * for the rounds), [1] round-1 cone search, [2] Boruvka rounds, [3] total
+ * (where a run starts over with every cone, the times of both attempts),
  * [4] the per-round component search's search dispatches (k_comp_search)
  * summed over the rounds, [5] the component search's neighbour lists at
  * build (k_knn_first); [4] and [5] in traced runs (options.trace; 0
