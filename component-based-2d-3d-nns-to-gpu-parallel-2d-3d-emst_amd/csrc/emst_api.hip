@@ -335,19 +335,20 @@ int alloc_all(emst_ctx* c)
     return EMST_OK;
 }
 
-int ensure_pinned(emst_ctx* c, PinBuf& b, size_t bytes)
+// false: pinned memory is refused (a limit on it, say)
+bool ensure_pinned(PinBuf& b, size_t bytes)
 {
-    if (b.cap >= bytes) return EMST_OK;
+    if (b.cap >= bytes) return true;
     if (b.p) (void)hipHostFree(b.p);
     b.p = nullptr;
     b.cap = 0;
     if (hipHostMalloc((void**)&b.p, bytes, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         b.p = nullptr;
-        return fail(c, EMST_E_OOM, "hipHostMalloc of " + std::to_string(bytes) + " bytes failed");
+        return false;
     }
     b.cap = bytes;
-    return EMST_OK;
+    return true;
 }
 
 struct OutSeg {
@@ -378,6 +379,15 @@ hipError_t copy_share(emst_ctx* c, const std::vector<OutSeg>& pieces, size_t chu
     return e;
 }
 
+// Without pinned memory: the runtime's own copies of pageable buffers.
+int copy_plain(emst_ctx* c, const std::vector<OutSeg>& segs)
+{
+    for (const OutSeg& s : segs)
+        if (s.dst && s.bytes) HIPCHK(c, hipMemcpyAsync(s.dst, s.src, s.bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return EMST_OK;
+}
+
 // Device results to pageable host memory, after the work queued on the
 // stream; returns once they are there.  The runtime's own copy of a pageable
 // buffer runs on the calling thread, which also takes the page faults of
@@ -391,9 +401,8 @@ int copy_out(emst_ctx* c, const std::vector<OutSeg>& segs)
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return EMST_OK;
     }
-    int rc;
     if (total <= kSmallOut) {
-        if ((rc = ensure_pinned(c, c->pin_small, kSmallOut + 64 * 8))) return rc;
+        if (!ensure_pinned(c->pin_small, kSmallOut + 64 * 8)) return copy_plain(c, segs);
         size_t at = 0;
         for (const OutSeg& s : segs)
             if (s.dst && s.bytes) {
@@ -416,7 +425,7 @@ int copy_out(emst_ctx* c, const std::vector<OutSeg>& segs)
             pieces.push_back({(char*)s.dst + at, (const char*)s.src + at, std::min(chunk, s.bytes - at)});
     const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
     const size_t nth = std::min<size_t>({pieces.size(), (size_t)kCopyThreads, (size_t)cores});
-    if ((rc = ensure_pinned(c, c->pin_ring, 2 * nth * chunk))) return rc;
+    if (!ensure_pinned(c->pin_ring, 2 * nth * chunk)) return copy_plain(c, segs);
     for (size_t k = 0; k < 2 * nth; ++k)
         if (!c->slot_ev[k]) HIPCHK(c, hipEventCreateWithFlags(&c->slot_ev[k], hipEventDisableTiming));
     std::vector<hipError_t> err(nth, hipSuccess);
