@@ -1723,23 +1723,26 @@ int emst_autotune(emst_ctx* c, int32_t* best_bucket, float* best_scale, float* b
     // the cone search's leaf size, seed and form are tuned on the cone form
     const int rs0 = c->opt.round_search;
     c->opt.round_search = 0;
-    // each choice by its whole run: with late cones the build's search is a
-    // part of the search
-    auto whole = [&](float* build_ms) {
+    // each choice by its build and search; by its whole run in 3D, where the
+    // rounds search too (late cones)
+    const bool rounds_too = c->cdim == 3 && c->ncl == 1;
+    auto time_choice = [&](float* build_ms, float* ms) {
         c->no_grouping = c->no_late = false;
         int r = build(c, false);
-        *build_ms = c->times[0] + c->times[1];
-        return r ? r : run_rounds(c);
+        *build_ms = *ms = c->times[0] + c->times[1];
+        if (r || !rounds_too) return r;
+        r = run_rounds(c);
+        *ms = c->times[3];
+        return r;
     };
-    float best = 0.f, bms = 0.f, ms = 0.f;
+    float best = 0.f, bms = 0.f, ms = 0.f, t = 0.f;
     int bb = 64;
     float bs = c->seed_scale;
     for (int b : {16, 32, 64})
         for (float sc : {2.f, 3.f, 4.f}) {
             if ((rc = layout_clouds(c, b))) break;
             c->seed_scale = sc;
-            if ((rc = whole(&ms))) break;
-            const float t = c->times[0] + c->times[1] + c->times[2];
+            if ((rc = time_choice(&ms, &t))) break;
             if (best == 0.f || t < best) {
                 best = t;
                 bms = ms;
@@ -1756,8 +1759,7 @@ int emst_autotune(emst_ctx* c, int32_t* best_bucket, float* best_scale, float* b
         c->seed_scale = bs;
         for (int sp : {1, 2, 3}) {
             c->opt.search_split = sp;
-            if ((rc = whole(&ms))) break;
-            const float t = c->times[0] + c->times[1] + c->times[2];
+            if ((rc = time_choice(&ms, &t))) break;
             if (t < best) {
                 best = t;
                 bms = ms;

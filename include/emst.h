@@ -162,10 +162,11 @@ int emst_set_clouds(emst_ctx* ctx, int32_t ncl, const int64_t* npts, const float
 int emst_get_cloud_results(emst_ctx* ctx, double* weight, int32_t* edges, int32_t* last_round);
 
 /* Autotuner (no counterpart in the reference, whose cell size is the fixed
- * level radius): times runs of the context's current points on the device
+ * level radius): times the build and cone search of the context's current
+ * points on the device (whole runs of one 3D cloud, whose rounds search too)
  * for every leaf size (points per leaf cell: 16, 32,
  * 64) and plain seed scale (2, 3, 4 leaf spacings), then every search_split
- * form (1, 2, 3) for the fastest pair, each by whole runs, then round_search 0
+ * form (1, 2, 3) for the fastest pair, then whole runs with round_search 0
  * and 1 at 64-point leaves (not with a learned model set, nor in the 2.5D
  * mode, where the caller's choice stays); keeps the fastest choice in the context (used by
  * every later set_points / set_clouds / run) and returns the pair; best_ms =
