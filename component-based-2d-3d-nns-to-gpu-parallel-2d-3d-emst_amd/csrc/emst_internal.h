@@ -288,6 +288,22 @@ __host__ __device__ inline uint32_t late_least(int32_t reach, uint32_t lo)
     const uint32_t past = (uint32_t)(reach + 1);
     return lo == 0xffffffffu || lo < past ? past : lo;
 }
+// The smallest edge key (d2, min id) that such a candidate can give the point
+// (id pid).  ck: what the earlier search left, the key (d2, id) of the nearest
+// one, none at that d2 having a smaller id; or with all ones for an id a d2 up
+// to and with which there is none.
+__host__ __device__ inline uint64_t late_first(int32_t reach, uint64_t ck, uint32_t pid)
+{
+    const uint32_t id = (uint32_t)ck;
+    uint32_t lo = (uint32_t)(ck >> 32);
+    if (lo != 0xffffffffu && id == 0xffffffffu) ++lo;
+    const uint32_t least = late_least(reach, lo);
+    const bool known = least == lo && id != 0xffffffffu;
+    return ((uint64_t)least << 32) | (known ? (id < pid ? id : pid) : 0u);
+}
+// corr of a late point whose nearest point outside its component, beyond its
+// reach, is known (its position q) and not checked against its cones
+__host__ __device__ inline int32_t late_held(int32_t q) { return -3 - q; }      // (and back)
 void launch_late_cones(const ConeRest& a, hipStream_t s);
 void launch_late_search(const ConeRest& a, Node* nodes, unsigned long long* visit, int64_t nleaves, bool first,
                         float seed_scale, const SplitScratch& sc, hipStream_t s);

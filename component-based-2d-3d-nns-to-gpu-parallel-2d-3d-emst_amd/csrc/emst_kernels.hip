@@ -2751,7 +2751,7 @@ __device__ __forceinline__ void round_min_point(bool inb, int64_t p, int K, cons
 {
     int32_t lp = 0;
     uint64_t key1 = kEmptyKey;
-    bool valid = false;
+    bool valid = false, held = false;
     if (inb) {
         lp = label[p];
         int32_t c = corr[p];
@@ -2760,7 +2760,12 @@ __device__ __forceinline__ void round_min_point(bool inb, int64_t p, int K, cons
         // since components only merge, the point never has an outgoing
         // candidate again (until a repeated cone search or a group
         // refresh gives it new candidates)
-        if (c != -2 && !(c >= 0 && label[c] != lp)) {
+        if (c <= late_held(0)) {
+            // (late cones) it bounds the component's edge while it is outside;
+            // its key stays as the point's lower bound
+            held = label[late_held(c)] != lp;
+            if (!held) corr[p] = -2;
+        } else if (c != -2 && !(c >= 0 && label[c] != lp)) {
             c = -1;
             ck = kEmptyKey;
             // kStep ranks per step, their loads independent of each other,
@@ -2803,9 +2808,9 @@ __device__ __forceinline__ void round_min_point(bool inb, int64_t p, int K, cons
             }
             cursor[p] = (uint8_t)r;
             corr[p] = c == -1 ? -2 : c;
-            corr_key[p] = ck;
+            if (c != -1) corr_key[p] = ck;
         }
-        if (c >= 0) {
+        if (c >= 0 || held) {
             const uint32_t pid = ids[p];
             const uint32_t qid = (uint32_t)ck;
             key1 = (ck & 0xffffffff00000000ull) | (uint64_t)min(pid, qid);
@@ -2840,17 +2845,25 @@ __device__ __forceinline__ uint64_t edge_key1(uint64_t ck, uint32_t pid)
 // of R_0^2; -1: none is known; kReachAll: all are exact), and only the exact
 // ones are ranked.  The rounds go on without the rest: a late point matters
 // only in a round in which every exact candidate of its has joined its
-// component while an unknown one could be as near as the component's smallest
-// edge (late_least, from its reach and the nearest outside point beyond it
-// that an earlier round found, corr_key): equal d2 counts, since the ids
-// decide.  Those points are listed here, after the round's minima.  Few of
-// them get their cones searched to the end (k_cone_rest).  More of them pause
-// the round, and their nearest points outside the component are searched
-// instead (launch_late_search).
+// component while an unknown one could be its component's smallest edge
+// (late_first, from its reach and the nearest outside point beyond it that an
+// earlier round found, corr_key).  Those points are listed here, after the
+// round's minima.  Few of them get their cones searched to the end
+// (k_cone_rest).  More of them pause the round, and their nearest points
+// outside the component are searched instead (launch_late_search).
+//
+// A nearest outside point so found that was not its component's edge is held
+// (late_held).  While it stays outside, it takes part in the minima, so that
+// few points of isolated clusters are asked again, and its owner is asked only
+// when its edge is the smallest.  Without it every point of a component with
+// no other edge was: solid blocks of 64 voxels apart from each other
+// (110592 points, whose every gap ties) 587000 points searched in 8 rounds and
+// 3.25 ms a run, now 206000 and 2.42.
 constexpr int kLateChunk = 2048;        // points per block: one list reservation each
 constexpr int kLatePer = kLateChunk / kBlock;
 
-__global__ __launch_bounds__(kBlock) void k_late_mark(int64_t n, const int32_t* __restrict__ label,
+__global__ __launch_bounds__(kBlock) void k_late_mark(int64_t n, const uint32_t* __restrict__ ids,
+                                                     const int32_t* __restrict__ label,
                                                      const int32_t* __restrict__ corr,
                                                      uint64_t* __restrict__ corr_key,
                                                      const uint64_t* __restrict__ comp1,
@@ -2867,14 +2880,20 @@ __global__ __launch_bounds__(kBlock) void k_late_mark(int64_t n, const int32_t* 
     for (int i = 0; i < kLatePer; ++i) {
         const int64_t p = c0 + i * 64;
         bool need = false;
-        if (p < n && corr[p] == -2) {
+        const int32_t c = p < n ? corr[p] : 0;
+        if (c == -2) {
             const int32_t r = reach[p];
             if (r != kReachAll) {
-                const uint32_t least = late_least(r, (uint32_t)(corr_key[p] >> 32));
-                need = least <= (uint32_t)(comp1[label[p]] >> 32);
+                const uint64_t ck = corr_key[p], edge = comp1[label[p]];
+                uint64_t first = late_first(r, ck, 0u);
+                // (its id matters where the d2 ties)
+                if (first >> 32 == edge >> 32) first = late_first(r, ck, ids[p]);
+                need = first <= edge;
                 // (the paused search starts there)
-                if (need && least > 0u) corr_key[p] = ((uint64_t)least << 32) | 0xffffffffull;
+                if (need && first >> 32 != 0u) corr_key[p] = first | 0xffffffffull;
             }
+        } else if (c <= late_held(0)) {
+            need = edge_key1(corr_key[p], ids[p]) == comp1[label[p]];
         }
         const uint64_t m = __ballot(need);
         at[i] = tot + (uint32_t)__popcll(m & lanemask_lt());
@@ -2903,16 +2922,16 @@ __global__ __launch_bounds__(kBlock) void k_late_mark(int64_t n, const int32_t* 
 __global__ __launch_bounds__(kBlock) void k_revive(int64_t n, int32_t* __restrict__ corr)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n && corr[p] == -2) corr[p] = -1;
+    if (p < n && corr[p] <= -2) corr[p] = -1;
 }
 
 // After the search of the listed points' nearest points outside their
 // components: a point whose edge is its component's smallest keeps it as its
 // target and is listed for k_cone_rest's check (not in round 1, where every
 // point is a component and its nearest point is the smallest cone candidate);
-// the others wait, their nearest outside point's d2 a lower bound.  A pair at
-// distance zero is left to the exact cones (done = 4), with its rule of
-// repeated searches.
+// the others wait (late_held, or the d2 where their search stopped as a lower
+// bound).  A pair at distance zero is left to the exact cones (done = 4), with
+// its rule of repeated searches.
 __global__ __launch_bounds__(kBlock) void k_late_settle(const int32_t* __restrict__ list,
                                                        const uint32_t* __restrict__ ids,
                                                        const int32_t* __restrict__ label,
@@ -2933,7 +2952,7 @@ __global__ __launch_bounds__(kBlock) void k_late_settle(const int32_t* __restric
             keep = edge_key1(ck, ids[p]) == comp1[label[p]];
             if ((ck >> 32) == 0u) C->done = 4u;
         }
-        if (!keep) corr[p] = -2;
+        if (!keep) corr[p] = corr[p] >= 0 ? late_held(corr[p]) : -2;
     }
     const bool add = keep && C->round > 1u;
     const uint64_t m = __ballot(add);
@@ -3115,6 +3134,8 @@ __global__ __launch_bounds__(64) void k_cone_rest(ConeRest a, const uint32_t* __
             continue;
         }
         // results
+        const bool held = a.corr[p] <= late_held(0);
+        const uint64_t was = edge_key1(a.corr_key[p], a.ids[p]);
         uint64_t key = kEmptyKey;
         int32_t pos = -1;
         if (lane < CC::K) {
@@ -3136,12 +3157,14 @@ __global__ __launch_bounds__(64) void k_cone_rest(ConeRest a, const uint32_t* __
         const int first = outm ? (int)__builtin_ctzll(outm) : CC::K;
         if (lane == (outm ? first : 0)) {
             a.cursor[p] = (uint8_t)first;
-            // (a target that is still outside was the smallest candidate, and stays it)
-            a.corr[p] = outm ? pos : -2;
-            a.corr_key[p] = outm ? key : kEmptyKey;
-            if (outm) {
-                const uint64_t k1 = (key & 0xffffffff00000000ull) | (uint64_t)min(a.ids[p], (uint32_t)key);
-                atomic_min_if_lower(&a.comp1[lp], k1);
+            const uint64_t k1 = outm ? edge_key1(key, a.ids[p]) : kEmptyKey;
+            // (a held edge that no cone has stays held, for k_late_seen; a
+            // target that is still outside was the smallest candidate, and
+            // stays it)
+            if (!held || k1 == was) {
+                a.corr[p] = outm ? pos : -2;
+                a.corr_key[p] = outm ? key : kEmptyKey;
+                if (outm) atomic_min_if_lower(&a.comp1[lp], k1);
             }
         }
     }
@@ -3157,18 +3180,28 @@ __global__ __launch_bounds__(64) void k_cone_rest(ConeRest a, const uint32_t* __
 // candidate there: a cone's nearest point is one of its component, which lies
 // nearer to that outside point and so has the smaller edge.  The component's
 // edge is then within what the point has seen; if not (in floats), the run
-// needs exact cones.
+// needs exact cones.  So it does where the edge is one held until now that is
+// no cone's; another such point takes its ranked candidates from here on.
 __global__ __launch_bounds__(kBlock) void k_late_seen(const int32_t* __restrict__ list,
+                                                     const uint32_t* __restrict__ ids,
                                                      const int32_t* __restrict__ label,
-                                                     const int32_t* __restrict__ corr,
+                                                     int32_t* __restrict__ corr,
+                                                     const uint64_t* __restrict__ corr_key,
                                                      const uint64_t* __restrict__ comp1,
                                                      const int32_t* __restrict__ reach, Counters* C)
 {
     if (C->done) return;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= C->late) return;
-    const int32_t p = list[t], r = reach[p];
-    if (corr[p] == -2 && r != kReachAll && (r < 0 || (uint32_t)(comp1[label[p]] >> 32) > (uint32_t)r)) C->done = 4u;
+    const int32_t p = list[t], c = corr[p], r = reach[p];
+    if (c >= 0) return;
+    const uint64_t edge = comp1[label[p]];
+    if (c <= late_held(0)) {
+        if (edge_key1(corr_key[p], ids[p]) == edge) C->done = 4u;
+        corr[p] = -1;
+    } else if (r != kReachAll && (r < 0 || (uint32_t)(edge >> 32) > (uint32_t)r)) {
+        C->done = 4u;
+    }
 }
 
 // second phase: among members matching (d2, min id), the smallest max id.
@@ -3742,6 +3775,20 @@ constexpr int kKnnGatherLeaves = 256;
 // 1.950, 1.992, 2.026; 131071 in the plane 1.203 / 1.206, 1.200, 1.213, 1.238.
 constexpr int64_t kKnnPackets = 4000;
 
+// d2 (bits) to which a component's edge lets its points search.  Late points go
+// some 0.01% further: where distances tie but for rounding (voxels), those just
+// beyond the edge are then found, and held for the next rounds, instead of
+// searched in each (the blocks at k_late_mark: 332000 points searched and 2.62
+// ms a run without).
+constexpr int32_t kLateSlack = 1 << 10;
+
+template <bool LATE>
+__device__ __forceinline__ int32_t edge_limit(uint64_t k)
+{
+    const int32_t b = key_bound(k);
+    return LATE && b < 0x7f000000 ? b + kLateSlack : b;
+}
+
 // nearest point in another component, for the points of qlist (count in
 // nq_dev): packet traversal as in the cone search, one best per query, by
 // iterative deepening from the seed radius R_0 (capped passes R_k = 8^(k/2) R_0,
@@ -3902,7 +3949,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
             };
             for (int pass = pass_lo; pass <= pass_hi; ++pass) {
                 const bool last = pass == kMaxCappedPasses;
-                const int32_t cbb = open ? key_bound(comp1[mylab]) : 0x7fffffff;
+                const int32_t cbb = open ? edge_limit<LATE>(comp1[mylab]) : 0x7fffffff;
                 // a point whose component already has an edge (a kept target, or
                 // a member's result) searches straight out to it in one pass
                 // instead of deepening by 4x per pass
@@ -4319,7 +4366,7 @@ __global__ __launch_bounds__(64 * kDeferWaves) void k_comp_search_deferred(
             const bool last = pass == kMaxCappedPasses;
             // (other waves lower comp1[mylab] meanwhile, and the lanes of one
             // load can see different values: one lane's steers the wave)
-            const int32_t cbb = key_bound(wave_first_u64(comp1[mylab]));
+            const int32_t cbb = edge_limit<LATE>(wave_first_u64(comp1[mylab]));
             const int32_t cap = last || cbb != 0x7fffffff ? 0x7fffffff : (int32_t)__float_as_uint(r2);
             if (cbb <= inner) {
                 open = false;
@@ -5367,11 +5414,12 @@ void launch_late_cones(const ConeRest& a, hipStream_t s)
 {
     if (a.n <= 0) return;
     hipLaunchKernelGGL(k_late_mark, dim3((unsigned)((a.n + kLateChunk - 1) / kLateChunk)), dim3(kBlock), 0, s, a.n,
-                       a.label, (const int32_t*)a.corr, a.corr_key, (const uint64_t*)a.comp1,
+                       a.ids, a.label, (const int32_t*)a.corr, a.corr_key, (const uint64_t*)a.comp1,
                        (const int32_t*)a.reach, a.list, a.C);
     cone_rest(a, &a.C->late, kRestFew, kRestRound, s);
     hipLaunchKernelGGL(k_late_seen, dim3((unsigned)(kRestFew / kBlock)), dim3(kBlock), 0, s, (const int32_t*)a.list,
-                       a.label, (const int32_t*)a.corr, (const uint64_t*)a.comp1, (const int32_t*)a.reach, a.C);
+                       a.ids, a.label, a.corr, (const uint64_t*)a.corr_key, (const uint64_t*)a.comp1,
+                       (const int32_t*)a.reach, a.C);
 }
 
 void launch_revive(int64_t n, int32_t* corr, hipStream_t s)
