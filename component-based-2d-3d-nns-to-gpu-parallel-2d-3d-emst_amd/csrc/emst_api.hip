@@ -672,7 +672,7 @@ SplitScratch split_scratch(emst_ctx* c)
     sc.list = c->list.p;
     sc.list2 = c->list2.p;
     sc.defer = c->defer.p;
-    sc.compact_frac = 1.0;
+    sc.in_place = false;
     return sc;
 }
 
@@ -764,7 +764,7 @@ int search_cones(emst_ctx* c, bool first, bool late)
     split.tmp = c->open_tmp.p;
     split.list = c->list.p;     // free until the rounds' research queue
     const int mode = c->opt.search_split;
-    split.compact_frac = mode == 2 ? -1.0 : 1.0;
+    split.in_place = mode == 2;
     const bool many = c->cdim == c->dim && n >= ((int64_t)1 << (c->dim == 3 ? 18 : 19));
     const bool use_split = late || mode == 2 || mode == 3 || (mode == 0 && many);
     launch_cone_search(c->dim, c->cdim, c->pts.p, c->nodes.p, c->dcl.p, c->ncl, c->bucket, leaf_table(c), n, nullptr,

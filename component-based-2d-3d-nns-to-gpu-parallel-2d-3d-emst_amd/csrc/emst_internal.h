@@ -240,7 +240,7 @@ struct SplitScratch {
     int32_t* list;          // n
     int32_t* list2;         // n (component search: the queries left open after pass 0)
     uint64_t* defer;        // n (component search: queries handed to the per-query pass)
-    double compact_frac;    // resume from a compacted list when at most this share of the queries is open
+    bool in_place;          // resume every packet in place, not from a compacted list (cone search)
 };
 // dim: point dimension (distances); cdim: cone dimension (cdim = 2 with dim =
 // 3 is the 2.5D mode: wedges over the xy plane).  split (nullptr: one launch

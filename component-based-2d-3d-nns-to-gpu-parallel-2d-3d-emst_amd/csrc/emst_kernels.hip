@@ -5393,7 +5393,7 @@ void launch_cone_search(int dim, int cdim, const float4* pts, const Node* nodes,
                        (const int32_t*)split->list, nq, label, check_labels ? 1 : 0, inv, seed_r, seed_scale,
                        cand_key, cand_pos, revive, first_corr, first_key, C, cs, dup, 1, kMaxCappedPasses,
                        (uint64_t*)nullptr, (const uint32_t*)(split->off + P), (const uint64_t*)split->open_mask,
-                       (int64_t)(split->compact_frac * (double)nq), 64);
+                       split->in_place ? (int64_t)-1 : nq, 64);
 }
 
 // Points that k_cone_rest takes at most in a round; a round with more pauses.
