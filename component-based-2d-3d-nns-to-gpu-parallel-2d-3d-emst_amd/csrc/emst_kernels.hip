@@ -2858,7 +2858,7 @@ __device__ __forceinline__ uint64_t edge_key1(uint64_t ck, uint32_t pid)
 // when its edge is the smallest.  Without it every point of a component with
 // no other edge was: solid blocks of 64 voxels apart from each other
 // (110592 points, whose every gap ties) 587000 points searched in 8 rounds and
-// 3.25 ms a run, now 206000 and 2.42.
+// 3.25 ms a run, now 207000 and 2.39.
 constexpr int kLateChunk = 2048;        // points per block: one list reservation each
 constexpr int kLatePer = kLateChunk / kBlock;
 

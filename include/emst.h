@@ -70,7 +70,8 @@ typedef struct {
     int32_t search_split;   /* round-1 cone search launches (changes work, never results):
                                0 auto: 3D from 2^12 points (one cloud, no two at one place)
                                the first pass with a smaller radius, the cones beyond it
-                               when a round asks for them; otherwise, and where the cones
+                               when a round asks for them (every cone first where that radius
+                               shows many points no other); otherwise, and where the cones
                                themselves are asked for, 3 from 2^18 points in 3D and 2^19
                                in 2D (not in the 2.5D mode), else 1; 1 one launch for
                                every pass; 2 first pass, then the open queries resumed in place;
